@@ -96,7 +96,7 @@ typedef enum rk_status {
 
 /* Decode launch policy (ROTATEK_KERNEL). */
 typedef enum rk_policy {
-  RK_POLICY_PAPER = 0,  /* one work unit per query head: K/V re-read per head */
+  RK_POLICY_PAPER = 0,  /* one work unit per query head (short calls; else as GQA) */
   RK_POLICY_GQA = 1     /* the query heads of a KV group share each K/V tile  */
 } rk_policy;
 
@@ -128,7 +128,7 @@ int rk_device_cu_count(int device, int* status);
  * (dtype of q_full).  1 <= D <= 128, 0 <= Dk <= 128 (Dk = 0: every channel
  * pruned, visual logits are the bias alone; R_partial and k_sparse may then
  * have no storage).  q, K, V and out share one dtype (F16, BF16 or F32;
- * fp32 runs a VALU kernel, one unit per query head); R_partial and
+ * fp32 runs a VALU kernel); R_partial and
  * delta_mu may be F16, BF16 or F32.
  * The workspace (size from rk_rotatek_decode_check, 256-byte aligned) holds
  * the split partials and, in its first RK_DECODE_TICKET_BYTES, the
@@ -143,7 +143,8 @@ int rk_device_cu_count(int device, int* status);
  * rk_set_decode_merge), and is hipGraph-capturable.  Calls that overlap
  * on one workspace race.  policy RK_POLICY_PAPER with num_kv_groups > 1 runs the
  * grouped decomposition (each K/V tile read once per KV head; the result
- * differs from one unit per query head only in fp32 summation order).
+ * differs from one unit per query head only in fp32 summation order), except
+ * for fp32 calls short enough for one workgroup per CU.
  */
 int rk_rotatek_decode_check(const rk_tensor* q_full, const rk_tensor* R_partial,
                             const rk_tensor* delta_mu, const rk_tensor* k_full,
@@ -236,7 +237,9 @@ int rk_append_kv(const rk_tensor* k_new, const rk_tensor* v_new, const rk_tensor
 
 /* Dense (full-channel) decode, the baseline the RotateK speed-up is measured
  * against (full_channel_flash_decoding.py:162-229, gqa_decode.py:254-277):
- * q [B,H_q,D], k/v [B,H_kv,S,D], out [B,H_q,D]. */
+ * q [B,H_q,D], k/v [B,H_kv,S,D], out [B,H_q,D].  policy as above; with
+ * num_kv_groups > 1 RK_POLICY_PAPER keeps one unit per query head for calls
+ * short enough for one workgroup per CU, in every dtype. */
 int rk_full_channel_decode_check(const rk_tensor* q, const rk_tensor* k,
                                  const rk_tensor* v, int64_t num_kv_groups,
                                  const rk_tensor* out, int32_t policy,

@@ -60,10 +60,7 @@ struct DecodeArgs {
   // others chunk_vis; see rk_plan_decode)
   int32_t cmajor, nfast;
   int64_t chunk_fast;
-  // xgroup > 1 (one unit per query head, G query heads per KV head): the
-  // units of a KV head that read the same chunk run in consecutive slots of
-  // one XCD (see decode_kernel); units = B * H_q
-  int32_t xgroup, units;
+  int32_t units;
   int32_t r_dtype, dm_dtype, has_bias, has_mask;
   // prologue layouts: q rows contiguous and 16-byte aligned (one 16-byte load
   // per thread); R a contiguous, 16-byte aligned [128][Dk] 16-bit block

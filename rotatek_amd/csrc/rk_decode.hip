@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <atomic>
+#include <algorithm>
 #include <mutex>
 #include <unordered_set>
 
@@ -489,24 +490,39 @@ int check_rotatek(const rk_tensor* q, const rk_tensor* R, const rk_tensor* dm,
   return RK_OK;
 }
 
-// The RotateK entry points run the paper family (ROTATEK_KERNEL=paper, one
-// unit per query head, fused_decode.py:370) with the grouped decomposition
-// when query heads share a KV head: the G heads of a group then read each
-// K/V tile once instead of G times (measured on MI355X, B=32 with 8 KV heads
-// of 4 query heads: 429 -> 208 us).  Every head's scores, softmax and P V
-// are computed as in the per-head decomposition, in fp32 with the same
-// hi + lo operand splits, so the two differ only in fp32 summation order.
-// The dense baseline keeps the per-head decomposition (the reference's
-// structure, full_channel_flash_decoding.py:197-203).
-int32_t rotatek_policy(int32_t policy, int64_t G) {
-  return policy == RK_POLICY_PAPER && G > 1 ? RK_POLICY_GQA : policy;
-}
-
 // The plan of a checked call (fp32 over 4-byte elements).
 int plan_for(const Checked& c, bool has_vis, int32_t policy, int cus, rk_decode_plan* p) {
   const bool f32 = c.dtype == RK_F32;
   return rk_plan_decode(c.B, c.H_q, c.H_kv, has_vis ? c.Dk : 0, has_vis ? c.S_v : 0, c.S_f, f32 ? 4 : 2, policy,
                         cus, p);
+}
+
+// The decomposition of a checked call.  The paper family (ROTATEK_KERNEL=paper,
+// one unit per query head, fused_decode.py:370 and
+// full_channel_flash_decoding.py:197-203) runs grouped where query heads
+// share a KV head: the G heads of a group then read each K/V tile once
+// instead of G times.  Every head's scores, softmax and P V are computed as
+// in the per-head decomposition, in fp32 with the same hi + lo operand
+// splits, so the two differ only in fp32 summation order.  Measured on MI355X,
+// B=32 with 8 KV heads of 4 query heads at 16k tokens: RotateK 429 -> 208 us,
+// dense 795 -> 321 us.  Short calls keep one unit per query head while that
+// grid is one round of one workgroup per CU, of at most the byte cap each:
+// nothing waits for the repeated reads there (K/V are a few MB, in the
+// caches after the first head), and a one-head workgroup has the shorter
+// prologue, softmax and merge.  Graph-replayed us per step, per head /
+// grouped.  Dense, 8 KV heads of 4, B=1: bf16 300 tokens 11.2 / 12.7, 2000
+// 12.4 / 13.0, and past the round 8000 19.6 / 14.5; fp32 2000 tokens 12.3 /
+// 19.7, 8000 (1 MB workgroups) 37.6 / 25.4.  RotateK, keep 32, 4 KV heads of
+// 7, B=1: fp32 1000 + 100 tokens 11.7 / 25.1, 4097 + 60 16.9 / 26.7; in 16
+// bits the lines cross inside the round (1000 + 100 tokens 10.1 / 10.8,
+// 2304 + 128 12.7 / 11.2), so those calls stay grouped.
+int32_t decode_policy(const Checked& c, bool has_vis, int32_t policy, int cus) {
+  if (policy != RK_POLICY_PAPER || c.G == 1) return policy;
+  rk_decode_plan p;
+  if ((!has_vis || c.dtype == RK_F32) && plan_for(c, has_vis, policy, cus, &p) == RK_OK && p.grid <= cus &&
+      std::max(p.chunk_full * 256, p.chunk_vis * (c.Dk + 128)) * rk::dtype_size(c.dtype) <= knobs().max_wg)
+    return policy;
+  return RK_POLICY_GQA;
 }
 
 int resolve_cus(int32_t num_cus, int* st) {
@@ -555,6 +571,7 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
   int st = RK_OK;
   const int cus = resolve_cus(0, &st);
   if (st) return st;
+  policy = decode_policy(c, has_vis, policy, cus);
   rk_decode_plan p;
   st = plan_for(c, has_vis, policy, cus, &p);
   if (st) return st;
@@ -674,10 +691,9 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
     a.rot_x = gx > 1 && p.wg_vis % gx != 0 ? 1 : 0;
   }
   a.units = (int32_t)p.units;
-  a.xgroup = policy == RK_POLICY_PAPER && c.G > 1 && c.dtype != RK_F32 ? (int32_t)c.G : 0;
-  if (a.xgroup || c.dtype == RK_F32) a.rot_x = 0;
+  if (c.dtype == RK_F32) a.rot_x = 0;
   a.scale_log2 = (float)(rk::kLog2e / sqrt((double)c.D));  // 1 / sqrt(D) (fused_decode.py:340)
-  a.cmajor = has_vis && c.dtype != RK_F32 && !a.xgroup ? p.chunk_major : 0;
+  a.cmajor = has_vis && c.dtype != RK_F32 ? p.chunk_major : 0;
   // the 16-bit kernels carry the single-launch merge at head_dim 128 with
   // 16-byte loads only; elsewhere the merge kernel runs
   if (c.dtype != RK_F32 && !(vec && c.D == 128)) a.fused = 0;
@@ -734,7 +750,7 @@ extern "C" int rk_rotatek_decode_check(const rk_tensor* q_full, const rk_tensor*
   if (st) return st;
   if (policy != RK_POLICY_PAPER && policy != RK_POLICY_GQA) return RK_ERR_ARG;
   rk_decode_plan p;
-  st = plan_for(c, true, rotatek_policy(policy, c.G), cus, &p);
+  st = plan_for(c, true, decode_policy(c, true, policy, cus), cus, &p);
   if (st) return st;
   if (workspace_bytes) *workspace_bytes = p.workspace_bytes;
   return RK_OK;
@@ -754,7 +770,7 @@ extern "C" int rk_rotatek_decode(const rk_tensor* q_full, const rk_tensor* R_par
   if ((st = check_out(out, c))) return st;
   if (policy != RK_POLICY_PAPER && policy != RK_POLICY_GQA) return RK_ERR_ARG;
   return run_decode(c, q_full, R_partial, delta_mu, k_full, v_full, mask_full, k_sparse, v_sparse,
-                    out, rotatek_policy(policy, c.G), workspace, workspace_bytes, stream, true);
+                    out, policy, workspace, workspace_bytes, stream, true);
 }
 
 extern "C" int rk_rotatek_decode_varlen(const rk_tensor* q_full, const rk_tensor* R_partial,
@@ -794,7 +810,7 @@ extern "C" int rk_rotatek_decode_varlen(const rk_tensor* q_full, const rk_tensor
     }
   }
   return run_decode(c, q_full, R_partial, delta_mu, k_full, v_buf, mask_full, k_sparse, v_sparse,
-                    out, rotatek_policy(policy, c.G), workspace, workspace_bytes, stream, true, len_full,
+                    out, policy, workspace, workspace_bytes, stream, true, len_full,
                     v_gap > 0 ? v_gap_at : -1, v_gap, k_new, v_new);
 }
 
@@ -903,7 +919,7 @@ extern "C" int rk_full_channel_decode_check(const rk_tensor* q, const rk_tensor*
   const int cus = resolve_cus(num_cus, &st);
   if (st) return st;
   rk_decode_plan p;
-  st = plan_for(c, false, policy, cus, &p);
+  st = plan_for(c, false, decode_policy(c, false, policy, cus), cus, &p);
   if (st) return st;
   if (workspace_bytes) *workspace_bytes = p.workspace_bytes;
   return RK_OK;
@@ -968,9 +984,9 @@ extern "C" int rk_rotatek_decode_noalloc(const rk_tensor* q_full, const rk_tenso
   if (!out) return RK_ERR_NULL;
   if ((st = check_out(out, c))) return st;
   if (policy != RK_POLICY_PAPER && policy != RK_POLICY_GQA) return RK_ERR_ARG;
-  const int32_t pol = rotatek_policy(policy, c.G);
   const int cus = resolve_cus(0, &st);
   if (st) return st;
+  const int32_t pol = decode_policy(c, true, policy, cus);
   rk_decode_plan p;
   if ((st = plan_for(c, true, pol, cus, &p))) return st;
   if (p.workspace_bytes > RK_NOALLOC_SCRATCH_BYTES) return RK_ERR_SCRATCH;

@@ -505,9 +505,6 @@ __device__ __forceinline__ void merge_fused(const DecodeArgs& a, int u, int b, i
 
 // APPEND: fused append of k_new / v_new (span cache decode step); a
 // separate instantiation so the plain decode carries none of its registers.
-// NTL: V rows and compact visual Key rows use non-temporal loads (false for
-// the grouped one-unit-per-query-head mode, whose G units of a KV head read
-// each line through one XCD's L2).
 // DPART (16-byte loads only): head_dim a.D < 128, a multiple of 8.  The
 // lanes of channels past D load an in-bounds duplicate of channels D-8..D-1
 // (V: only output channels past D see it, and those are not written; full
@@ -519,8 +516,7 @@ __device__ __forceinline__ void merge_fused(const DecodeArgs& a, int u, int b, i
 // (a.fused set).  A separate instantiation: inlined into every
 // kernel, the merge's code raised the split pass's register pressure
 // enough to spill scalar registers in its loops.
-template <class TT, int DKB, bool VEC, int HMAX, bool HAS_VIS, bool APPEND, bool NTL = true, bool DPART = false,
-          bool FUSED = false>
+template <class TT, int DKB, bool VEC, int HMAX, bool HAS_VIS, bool APPEND, bool DPART = false, bool FUSED = false>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 decode_kernel(const DecodeArgs a) {
   static_assert(!DPART || VEC, "the element-wise kernels mask head_dim at run time");
@@ -561,21 +557,6 @@ decode_kernel(const DecodeArgs a) {
   int u = a.cmajor ? (int)blockIdx.x : (int)blockIdx.y;
   int x = a.cmajor ? (int)blockIdx.y : (int)blockIdx.x + (a.rot_x ? u % a.np : 0);
   x = x >= a.np ? x - a.np : x;
-  if (!NTL && a.xgroup > 1) {  // compiled into the grouped mode's instantiation only
-    // Workgroup id i = y * np + x runs on XCD i mod 8 as the (i / 8)-th of
-    // that XCD.  Each XCD takes a contiguous range of the work items
-    // ((b, kv) major, then chunk, then the query head j of the group), so
-    // the G units that read one K/V chunk are neighbours on one XCD and
-    // share its L2 instead of each fetching the chunk from HBM.
-    const int64_t N = (int64_t)a.units * a.np, bid = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-    const int64_t c = bid & 7, q8 = N >> 3, r8 = N & 7;
-    const int64_t item = c * q8 + min(c, r8) + (bid >> 3);
-    const int64_t grp = item / a.xgroup;  // (b, kv, chunk)
-    const int j = (int)(item - grp * a.xgroup);
-    const int64_t ukv = grp / a.np;
-    x = (int)(grp - ukv * a.np);
-    u = (int)(ukv * a.xgroup + j);
-  }
   const int b = u / a.units_per_b;
   const int r_in_b = u - b * a.units_per_b;
   const int kv = r_in_b / a.spk;
@@ -623,9 +604,7 @@ decode_kernel(const DecodeArgs a) {
   for (int j = 0; j < 8; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // A-operand token row of this lane inside a block, per score sub-block
   const uint32_t krow0 = 8 * (n >> 2) + (n & 3), krow1 = krow0 + 4;
-  // the units of one KV head visit a chunk's blocks in the same order
-  const uint32_t useed = !NTL && a.xgroup > 1 ? (uint32_t)(u / a.xgroup) : (uint32_t)u;
-  const uint32_t rot_seed = (useed * 0x9E3779B1u) ^ ((uint32_t)x * 0x85EBCA77u);
+  const uint32_t rot_seed = ((uint32_t)u * 0x9E3779B1u) ^ ((uint32_t)x * 0x85EBCA77u);
 
   // Prologue order: the first NBUF K/V blocks are requested, then the
   // prologue's own loads (q rows; R / delta_mu or the mask bytes), and only
@@ -723,12 +702,12 @@ decode_kernel(const DecodeArgs a) {
 #pragma unroll
       for (int kb = 0; kb < DKB; ++kb) {
         const uint32_t ch = kFoldK ? 0u : kch[kb];
-        B.k[0][kb] = load_row8b<VEC, NTL && DKB == 1>(ksb, r0, ch, a.ks_sd, knv[kb]);
-        B.k[1][kb] = load_row8b<VEC, NTL && DKB == 1>(ksb, r1, ch, a.ks_sd, knv[kb]);
+        B.k[0][kb] = load_row8b<VEC, DKB == 1>(ksb, r0, ch, a.ks_sd, knv[kb]);
+        B.k[1][kb] = load_row8b<VEC, DKB == 1>(ksb, r1, ch, a.ks_sd, knv[kb]);
       }
 #pragma unroll
       for (int r = 0; r < 8; ++r)
-        B.v[r] = load_row8b<VEC, NTL>(vsb, min(vro + vb0 + (uint32_t)r * vss2, vlast), VEC ? 0u : vch, a.vs_sd, vnv);
+        B.v[r] = load_row8b<VEC, true>(vsb, min(vro + vb0 + (uint32_t)r * vss2, vlast), VEC ? 0u : vch, a.vs_sd, vnv);
     };
 
     // q R: thread (c, part) loads R[part*L .. part*L+L-1][c], forms partial
@@ -975,7 +954,7 @@ decode_kernel(const DecodeArgs a) {
       for (int r = 0; r < 8; ++r) {
         uint32_t row = min(t0 + 8u * g + r, t_last);
         row += row >= a.vf_gap_at ? a.vf_gap : 0u;
-        B.v[r] = load_row8<VEC, NTL>(vfb, row * a.vf_ss, vch, a.vf_sd, vnv);
+        B.v[r] = load_row8<VEC, true>(vfb, row * a.vf_ss, vch, a.vf_sd, vnv);
       }
     };
 
@@ -1101,7 +1080,7 @@ decode_kernel(const DecodeArgs a) {
 // P V over the block's rows, with the block's probabilities broadcast
 // from LDS.
 //   decode32_kernel   one query head per unit (G = 1, or the paper
-//                     family's dense baseline);
+//                     family's short dense calls);
 //   decode32g_kernel  up to HG = 8 query heads of one KV head per unit (the
 //                     grouped decomposition, gqa_decode.py:121-210): each
 //                     K and V row is loaded once and serves every head (one
@@ -1624,37 +1603,23 @@ hipError_t launch_one(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   constexpr bool kCanFuse = VEC && !DPART;
   if (a.fused && !kCanFuse) return hipErrorInvalidValue;
   bool launched = false;
-  // grouped one-unit-per-query-head mode (temporal loads): the dense
-  // baseline's paper family at G > 1 only (the RotateK entries run that
-  // family grouped, see rotatek_policy)
-  if constexpr (VEC && HMAX == 1 && !HAS_VIS) {
-    if (a.xgroup > 1) {
-      if (a.fused)
-        hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, HAS_VIS, false, false, DPART, kCanFuse>), grid,
-                           dim3(kThreads), 0, s, a);
-      else
-        hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, HAS_VIS, false, false, DPART>), grid,
-                           dim3(kThreads), 0, s, a);
-      launched = true;
-    }
-  }
   if constexpr (HAS_VIS) {  // the span cache's step always carries the visual span
     if (!launched && a.k_new) {
       if (a.fused)
-        hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, true, true, true, DPART, kCanFuse>), grid,
+        hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, true, true, DPART, kCanFuse>), grid,
                            dim3(kThreads), 0, s, a);
       else
-        hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, true, true, true, DPART>), grid, dim3(kThreads),
+        hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, true, true, DPART>), grid, dim3(kThreads),
                            0, s, a);
       launched = true;
     }
   }
   if (!launched) {
     if (a.fused)
-      hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, HAS_VIS, false, true, DPART, kCanFuse>), grid,
+      hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, HAS_VIS, false, DPART, kCanFuse>), grid,
                          dim3(kThreads), 0, s, a);
     else
-      hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, HAS_VIS, false, true, DPART>), grid, dim3(kThreads),
+      hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, HAS_VIS, false, DPART>), grid, dim3(kThreads),
                          0, s, a);
   }
   hipError_t e = hipGetLastError();
