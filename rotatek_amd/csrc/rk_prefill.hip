@@ -35,6 +35,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "rk_common.h"
@@ -77,9 +78,12 @@ __device__ __forceinline__ int slot_nv(int c0, int D) { return max(min(D - c0, 8
 
 // Eight 16-bit channels c0..c0+7 of row `t` (clamped by the caller); the
 // element-wise form reads the first nv and zeroes the rest.
-template <bool VEC>
+template <bool VEC, bool NT = false>
 __device__ __forceinline__ uint4 ldrow(const uint16_t* base, const KeyView& k, uint32_t t, uint32_t c0, int nv = 8) {
-  if constexpr (VEC) {
+  if constexpr (VEC && NT) {
+    const u32x4 v = __builtin_nontemporal_load((const u32x4*)((const char*)base + (t * k.ss + c0) * 2u));
+    return make_uint4(v.x, v.y, v.z, v.w);
+  } else if constexpr (VEC) {
     return *(const uint4*)((const char*)base + (t * k.ss + c0) * 2u);
   } else {
     uint32_t w[4] = {0, 0, 0, 0};
@@ -151,7 +155,13 @@ __device__ __forceinline__ void head_query_norms(const KeyView& k, const QNormAr
 // (x == splits) that forms the head's floored query norms.  Only these
 // instantiations carry that code: its registers would otherwise set the
 // occupancy of the summing loop.
-template <class TT, bool VEC, bool QN, bool QV>
+//
+// NT: non-temporal row loads, for Keys larger than the 256 MB memory-side
+// cache, which no later pass finds there (B=32, 32 heads, 14000 tokens, 3.7 GB:
+// 6.3 -> 6.6 TB/s).  Smaller Keys keep ordinary loads: the covariance and
+// the rotation read them again (12001 tokens x 32 heads, 98 MB: covariance
+// with non-temporal mean loads 50 -> 53 us).
+template <class TT, bool VEC, bool NT, bool QN, bool QV>
 __global__ void __launch_bounds__(kThreads) mean_kernel(KeyView k, int64_t chunk, int splits, float* part,
                                                         QNormArgs qa) {
   __shared__ float s_sum[16][128];
@@ -173,7 +183,7 @@ __global__ void __launch_bounds__(kThreads) mean_kernel(KeyView k, int64_t chunk
     for (int64_t t = t0 + rg; t < t1; t += 64) {
       uint4 v[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = ldrow<VEC>(base, k, min((uint32_t)(t + 16 * i), last), cl, nv);
+      for (int i = 0; i < 4; ++i) v[i] = ldrow<VEC, NT>(base, k, min((uint32_t)(t + 16 * i), last), cl, nv);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         if (t + 16 * i < t1) {
@@ -248,23 +258,102 @@ __host__ __device__ constexpr int tile_row(int t) {
 }
 __host__ __device__ constexpr int tile_col(int t) { return tile_row(t) + t - tile_index(tile_row(t), tile_row(t)); }
 
+// Where a covariance and its mean go, and the query-aware weighting (qn:
+// floored norms [B*H][128], null without it; rfac = fp32(1 / D)).
+struct CovOut {
+  float* cov;
+  int64_t c_b, c_h, c_r, c_c;
+  float* mu;  // optional
+  int64_t m_b, m_h, m_c;
+  const float* qn;
+  float rfac;
+};
+
+// 1e-4 max(mean|diag(C o qn qn^T)|, 1e-6) from the diagonal dg_in[c] =
+// C[c][c] (threads 0..D-1; the sum is a fixed xor tree in each of waves 0
+// and 1, then the two halves, times torch's mean factor rfac = fp32(1/D)),
+// as the weighted covariance's ridge.
+__device__ __forceinline__ float weighted_ridge(float diag, const float* s_qn, int tid, int D, float rfac,
+                                                float* s_wsum) {
+  if (tid < 128) {
+    const float qd = s_qn[tid];
+    float dg = tid < D ? fabsf(diag * (qd * qd)) : 0.f;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) dg += shfl_xor(dg, off);
+    if ((tid & 63) == 0) s_wsum[tid >> 6] = dg;
+  }
+  __syncthreads();
+  return 1e-4f * fmaxf((s_wsum[0] + s_wsum[1]) * rfac, 1e-6f);
+}
+
+// The covariance of one head from its fp32 sums in LDS (s_red: the upper
+// tiles, kTS floats apart), as covfin_kernel / covfin_qw_kernel form it from
+// partials, with the same operations: round to the key dtype, symmetrise,
+// and with o.qn weight and add the ridge.  The workgroup writes whole rows.
+template <class TT, int kTS>
+__device__ __forceinline__ void finish_head(const CovOut& o, float* s_red, int bh, int H, int D, int tid) {
+  __shared__ __align__(16) float s_fq[128];
+  __shared__ float s_fw[2];
+  const int b = bh / H, h = bh - b * H;
+#pragma unroll 4
+  for (int t = 0; t < kTiles; ++t) {
+    const float v = s_red[t * kTS + tid];
+    s_red[t * kTS + tid] = TT::to_f32(TT::from_f32(v));
+  }
+  if (o.qn && tid < 128) s_fq[tid] = o.qn[(int64_t)bh * 128 + tid];
+  __syncthreads();
+  float ridge = 0.f;
+  if (o.qn) {  // launch-uniform
+    const float dx = s_red[tile_index(tid & 7, tid & 7) * kTS + 17 * ((tid & 127) >> 3)];
+    ridge = weighted_ridge(0.5f * (dx + dx), s_fq, tid, D, o.rfac, s_fw);
+  }
+  // entry (r, c), r = 8m + i, c = 8n + j: of tile (i, j) at (m, n), or of
+  // the mirror (j, i) at (n, m); a diagonal tile holds both
+  float* cb = o.cov + b * o.c_b + (int64_t)h * o.c_h;
+  const int c = tid & 127, j = c & 7, n = c >> 3;
+#pragma unroll 4
+  for (int r = tid >> 7; r < D; r += 2) {
+    const int i = r & 7, m = r >> 3;
+    const int lo = min(i, j), hi = max(i, j);
+    const float* tl = s_red + tile_index(lo, hi) * kTS;
+    const float rc = tl[i <= j ? m * 16 + n : n * 16 + m];
+    const float cr = i == j ? tl[n * 16 + m] : rc;
+    float v = 0.5f * (rc + cr);
+    if (o.qn) {
+      const float a = v * (s_fq[r] * s_fq[c]);
+      v = 0.5f * (a + a) + (r == c ? ridge : 0.f);
+    }
+    if (c < D) cb[r * o.c_r + c * o.c_c] = v;
+  }
+}
+
 // grid (splits, B*H): each wave accumulates Kc^T Kc over its interleaved
 // 32-token blocks for all 36 upper tiles; the four waves are summed in LDS
 // and the workgroup writes one [36][256] partial, and, with dpart, its 128
 // diagonal entries once more as one contiguous row dpart[bh][x][128] (what
 // the weighted finalisation sums for the ridge).
-template <class TT, bool VEC>
+//
+// NT: as mean_kernel.  FIN (one workgroup per head, the plan for many
+// heads): the workgroup holds the head's whole sums and finishes them itself
+// (finish_head), without the partials' round trip through memory and the
+// finalisation launch: B=32, 32 heads, 14000 tokens, 108 us of 685.
+template <class TT, bool VEC, bool NT = false, bool FIN = false>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 cov_kernel(KeyView k, int64_t chunk, int splits, const float* mean_part, int mean_splits, float mfac,
-           float* part, float* dpart) {
+           float* part, float* dpart, CovOut o) {
+  // FIN reads whole covariance rows, consecutive lanes in consecutive tiles:
+  // eight more words per tile put them on different banks
+  constexpr int kTS = FIN ? 264 : 256;
   __shared__ float s_c[128];
-  __shared__ float s_red[kTiles * 256];
+  __shared__ float s_red[kTiles * kTS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
   const int x = blockIdx.x, bh = blockIdx.y;
   if (tid < 128) {
     // centre = mean rounded to the key dtype (kv_pruning_utils.py:113);
     // channels past D have none
-    s_c[tid] = tid < k.D ? TT::to_f32(TT::from_f32(head_mean(mean_part, bh, mean_splits, tid, mfac))) : 0.f;
+    const float mu = tid < k.D ? head_mean(mean_part, bh, mean_splits, tid, mfac) : 0.f;
+    s_c[tid] = TT::to_f32(TT::from_f32(mu));
+    if (FIN && o.mu && tid < k.D) o.mu[(bh / k.H) * o.m_b + (int64_t)(bh % k.H) * o.m_h + tid * o.m_c] = mu;
   }
   __syncthreads();
   float cen[8];
@@ -297,7 +386,7 @@ cov_kernel(KeyView k, int64_t chunk, int splits, const float* mean_part, int mea
       uint4 rows[8];
 #pragma unroll
       for (int r = 0; r < 8; ++r)
-        rows[r] = ldrow<VEC>(base, k, MASK ? min((uint32_t)(tb + r), last) : (uint32_t)(tb + r), cl, nv);
+        rows[r] = ldrow<VEC, NT>(base, k, MASK ? min((uint32_t)(tb + r), last) : (uint32_t)(tb + r), cl, nv);
       const int64_t left = t1 - tb;
       const int nvalid = !ch_ok ? 0 : left >= 8 ? 8 : (left > 0 ? (int)left : 0);
       uint32_t w[8][4];
@@ -357,11 +446,15 @@ cov_kernel(KeyView k, int64_t chunk, int splits, const float* mean_part, int mea
       for (int t = 0; t < kTiles; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          float& dst = s_red[t * 256 + (4 * g + r) * 16 + n];
+          float& dst = s_red[t * kTS + (4 * g + r) * 16 + n];
           dst = (w == 0) ? acc[t][r] : dst + acc[t][r];
         }
     }
     __syncthreads();
+  }
+  if constexpr (FIN) {
+    finish_head<TT, kTS>(o, s_red, bh, k.H, k.D, tid);
+    return;
   }
   float* out = part + ((int64_t)bh * splits + x) * (kTiles * 256);
   for (int i = tid; i < kTiles * 256; i += kThreads) out[i] = s_red[i];
@@ -382,9 +475,7 @@ cov_kernel(KeyView k, int64_t chunk, int splits, const float* mean_part, int mea
 template <class TT>
 __global__ void __launch_bounds__(kThreads) covfin_kernel(const float* part, int splits,
                                                           const float* mean_part, int mean_splits,
-                                                          float mfac, float* cov, int64_t cs_b, int64_t cs_h,
-                                                          int64_t cs_r, int64_t cs_c, float* mu, int64_t ms_b,
-                                                          int64_t ms_h, int64_t ms_c, int H, int D) {
+                                                          float mfac, CovOut o, int H, int D) {
   __shared__ float s_t[256];
   const int tid = threadIdx.x, t = blockIdx.x, bh = blockIdx.y;
   const int b = bh / H, h = bh - b * H;
@@ -394,16 +485,16 @@ __global__ void __launch_bounds__(kThreads) covfin_kernel(const float* part, int
   s_t[tid] = TT::to_f32(TT::from_f32(sum));
   __syncthreads();
   const int i = tile_row(t), j = tile_col(t), m = tid >> 4, n = tid & 15;
-  float* cb = cov + b * cs_b + (int64_t)h * cs_h;
+  float* cb = o.cov + b * o.c_b + (int64_t)h * o.c_h;
   const int r = 8 * m + i, c = 8 * n + j;
   const float rc = s_t[tid];
   const float cr = i == j ? s_t[n * 16 + m] : rc;
   if (r < D && c < D) {
-    cb[r * cs_r + c * cs_c] = 0.5f * (rc + cr);
-    if (i != j) cb[c * cs_r + r * cs_c] = 0.5f * (cr + rc);
+    cb[r * o.c_r + c * o.c_c] = 0.5f * (rc + cr);
+    if (i != j) cb[c * o.c_r + r * o.c_c] = 0.5f * (cr + rc);
   }
-  if (t == 0 && tid < D && mu)
-    mu[b * ms_b + (int64_t)h * ms_h + tid * ms_c] = head_mean(mean_part, bh, mean_splits, tid, mfac);
+  if (t == 0 && tid < D && o.mu)
+    o.mu[b * o.m_b + (int64_t)h * o.m_h + tid * o.m_c] = head_mean(mean_part, bh, mean_splits, tid, mfac);
 }
 
 // ------------------------------------------------------------------ rotate / score
@@ -423,17 +514,30 @@ struct RotArgs {
   int32_t Dk;
   uint16_t* out;
   int64_t o_sb, o_sh, o_ss, o_sd;
+  int32_t r_vec;  // R in the Keys' type, rows of whole, aligned 16-byte slots
+  int32_t o_vec;  // 16-bit STORE: rows of whole, aligned 16-byte slots
+  int32_t o_stream;  // more output than the memory-side cache holds: non-temporal stores
   float* spart;
   int64_t chunk;
   int32_t splits;
 };
 
-template <class TT, int NT, bool VEC, bool SCORE>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+// The kept channel of accumulator row m of tile t.  With whole pairs of tiles
+// a lane (rows 4g..4g+3 of both) holds eight consecutive channels 32 p + 8g..,
+// so STORE writes 16 bytes per token and pair, a pair's four lanes one
+// 64-byte segment; a single tile keeps its natural order.
+template <int NT>
+__host__ __device__ constexpr int kept_of(int t, int m) {
+  return NT == 1 ? m : 32 * (t >> 1) + 8 * (m >> 2) + 4 * (t & 1) + (m & 3);
+}
+
+template <class TT, int NT, bool VEC, bool SCORE, bool FAST = false>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FAST ? 4 : 2)))
 rot_kernel(const RotArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t s_rt[NT * 16][128 + 8];  // R^T, padded rows
   __shared__ float s_sc[kWaves][NT * 16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, n = lane & 15;
   const int x = blockIdx.x, bh = blockIdx.y;
   const int b = bh / a.k.H, h = bh - b * a.k.H;
   const uint16_t* base = head_base(a.k, bh);
@@ -441,35 +545,53 @@ rot_kernel(const RotArgs a) {
   // this thread's batch is (c, kk) = (e % 128, e / 128): consecutive threads
   // take consecutive c; all loads are issued before any is converted.
   const int64_t rb = b * a.R_sb + (int64_t)h * a.R_sh;
-  const int D = a.k.D;
+  const int D = FAST ? 128 : a.k.D;
   constexpr int kPer = NT * 16 * 128 / kThreads;
-  uint32_t raw[kPer];
+  constexpr int kBatch = kPer < 16 ? kPer : 16;
+  if (FAST && a.r_vec) {
+    // 16-byte loads of R's rows (8 kept channels of one channel c each)
+    uint4 v[NT];
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int e = tid + i * kThreads, kk = e >> 7, c = e & 127;
-    raw[i] = load_raw(a.R, rb + min(c, D - 1) * a.R_sd + min(kk, a.Dk - 1) * a.R_sk, a.r_dtype);
-  }
+    for (int i = 0; i < NT; ++i) {
+      const int e = tid + i * kThreads, kk = 8 * (e & (2 * NT - 1)), c = e / (2 * NT);
+      v[i] = *(const uint4*)((const uint16_t*)a.R + rb + c * a.R_sd + min(kk, a.Dk - 8));
+    }
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int e = tid + i * kThreads, kk = e >> 7, c = e & 127;
-    s_rt[kk][c] = TT::from_f32(kk < a.Dk && c < D ? raw_to_f32(raw[i], a.r_dtype) : 0.f);
+    for (int i = 0; i < NT; ++i) {
+      const int e = tid + i * kThreads, kk = 8 * (e & (2 * NT - 1)), c = e / (2 * NT);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        s_rt[kk + j][c] = kk < a.Dk ? (uint16_t)(word(v[i], j >> 1) >> ((j & 1) * 16)) : (uint16_t)0;
+    }
+  } else
+#pragma unroll 1
+  for (int i0 = 0; i0 < kPer; i0 += kBatch) {
+    uint32_t raw[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int e = tid + (i0 + i) * kThreads, kk = e >> 7, c = e & 127;
+      raw[i] = load_raw(a.R, rb + min(c, D - 1) * a.R_sd + min(kk, a.Dk - 1) * a.R_sk, a.r_dtype);
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int e = tid + (i0 + i) * kThreads, kk = e >> 7, c = e & 127;
+      s_rt[kk][c] = TT::from_f32(kk < a.Dk && c < D ? raw_to_f32(raw[i], a.r_dtype) : 0.f);
+    }
   }
   __syncthreads();
   // channel slots 32 ks + 8 g of this lane (past D: see the file comment)
   uint32_t cl[4];
   int nv[4];
-  bool cok[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
     cl[ks] = slot_c0<VEC>(32 * ks + 8 * g, D);
     nv[ks] = slot_nv(32 * ks + 8 * g, D);
-    cok[ks] = 32 * ks + 8 * g < D;
   }
-  const bool dpart = VEC && D < 128;  // launch-uniform
+  const bool dpart = !FAST && VEC && D < 128;  // launch-uniform
 
-  float sc[NT][4];
+  float sc[SCORE ? NT : 1][4];
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+  for (int t = 0; t < (SCORE ? NT : 1); ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) sc[t][r] = 0.f;
   const int64_t t0 = (int64_t)x * a.chunk, t1 = min(a.k.S, t0 + a.chunk);
@@ -480,24 +602,24 @@ rot_kernel(const RotArgs a) {
   // store variant 32-token steps, so its output path fits in registers.
   constexpr int TB = SCORE ? 4 : 2;
   constexpr int kStep = 16 * TB;
-  const int64_t nstep = (t1 - t0 + kStep - 1) / kStep;
+  const int nstep = (int)((t1 - t0 + kStep - 1) / kStep);
   const uint32_t last = (uint32_t)max(t1 - 1, (int64_t)0);
-  auto load = [&](uint4 (&bk)[TB][4], int64_t st) {
-    const int64_t ts = t0 + st * kStep;
+  auto load = [&](uint4 (&bk)[TB][4], int st) {
+    const uint32_t ts = (uint32_t)min(t0 + (int64_t)st * kStep, (int64_t)last);  // wave-uniform
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) {
-      const int64_t tok = ts + 16 * tb + n;
-      const uint32_t tr = min((uint32_t)min(tok, (int64_t)last), last);
+      const uint32_t tr = min(ts + 16 * tb + n, last);
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) bk[tb][ks] = ldrow<VEC>(base, a.k, tr, cl[ks], nv[ks]);
     }
   };
-  auto compute = [&](uint4 (&bk)[TB][4], int64_t st) {
-    const int64_t ts = t0 + st * kStep;
+  uint16_t* ob = a.out + b * a.o_sb + (int64_t)h * a.o_sh;  // this head's rows
+  auto compute = [&](uint4 (&bk)[TB][4], int st) {
+    const int left = (int)min(t1 - (t0 + (int64_t)st * kStep), (int64_t)kStep);  // tokens of this step
     if constexpr (SCORE) {
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb)
-        if (ts + 16 * tb + n >= t1)
+        if (16 * tb + n >= left)
 #pragma unroll
           for (int ks = 0; ks < 4; ++ks) bk[tb][ks] = make_uint4(0, 0, 0, 0);
     }
@@ -506,40 +628,63 @@ rot_kernel(const RotArgs a) {
       for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
-          if (!cok[ks]) bk[tb][ks] = make_uint4(0, 0, 0, 0);
+          if (32 * ks + 8 * g >= D) bk[tb][ks] = make_uint4(0, 0, 0, 0);
     }
-#pragma unroll(NT <= 2 ? NT : 1)
-    for (int t = 0; t < NT; ++t) {
-      f32x4 c[TB];
+    constexpr int NP = NT == 1 ? 1 : 2;  // tiles per pass
+    // opaque: keeps the R^T fragments in LDS (hoisted out of the step loop
+    // they take 16 registers a tile, and the occupancy with them)
+    int aoff = n * 0;
+    asm volatile("" : "+v"(aoff));
+    const uint16_t* rt = &s_rt[0][0] + aoff;
+#pragma unroll 1
+    for (int t = 0; t < NT; t += NP) {
+      f32x4 c[NP][TB];
 #pragma unroll
-      for (int tb = 0; tb < TB; ++tb) c[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) c[p][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        const uint4 av = *(const uint4*)&s_rt[16 * t + n][32 * ks + 8 * g];
 #pragma unroll
-        for (int tb = 0; tb < TB; ++tb) c[tb] = TT::mfma(av, bk[tb][ks], c[tb]);
+        for (int p = 0; p < NP; ++p) {
+          const uint4 av = *(const uint4*)(rt + kept_of<NT>(t + p, n) * (128 + 8) + 32 * ks + 8 * g);
+#pragma unroll
+          for (int tb = 0; tb < TB; ++tb) c[p][tb] = TT::mfma(av, bk[tb][ks], c[p][tb]);
+        }
       }
       if constexpr (SCORE) {
 #pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
+        for (int p = 0; p < NP; ++p)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) sc[t][r] += fabsf(c[tb][r]);
+          for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[t + p][r] += fabsf(c[p][tb][r]);
       } else {
+        const int k0 = kept_of<NT>(t, 4 * g);
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) {
-          const int64_t tok = ts + 16 * tb + n;
-          if (tok < t1) {
-            uint16_t* o = a.out + b * a.o_sb + (int64_t)h * a.o_sh + tok * a.o_ss;
-            const int k0 = 16 * t + 4 * g;
-            if (k0 + 3 < a.Dk && a.o_sd == 1 && (((uintptr_t)(o + k0)) & 7) == 0) {
-              uint2 w;
-              w.x = TT::from_f32(c[tb][0]) | ((uint32_t)TT::from_f32(c[tb][1]) << 16);
-              w.y = TT::from_f32(c[tb][2]) | ((uint32_t)TT::from_f32(c[tb][3]) << 16);
-              *(uint2*)(o + k0) = w;
+          if (16 * tb + n < left) {
+            uint16_t* o = ob + (t0 + (int64_t)st * kStep + 16 * tb + n) * a.o_ss;
+            if constexpr (FAST) {  // whole slots of 8 kept channels, aligned
+              if (k0 < a.Dk) {
+                if constexpr (NP == 2) {
+                  const u32x4 w = {TT::pack2(c[0][tb][0], c[0][tb][1]), TT::pack2(c[0][tb][2], c[0][tb][3]),
+                                   TT::pack2(c[1][tb][0], c[1][tb][1]), TT::pack2(c[1][tb][2], c[1][tb][3])};
+                  if (a.o_stream)
+                    __builtin_nontemporal_store(w, (u32x4*)(o + k0));
+                  else
+                    *(u32x4*)(o + k0) = w;
+                } else {
+                  *(uint2*)(o + k0) = make_uint2(TT::pack2(c[0][tb][0], c[0][tb][1]),
+                                                 TT::pack2(c[0][tb][2], c[0][tb][3]));
+                }
+              }
             } else {
 #pragma unroll
-              for (int r = 0; r < 4; ++r)
-                if (k0 + r < a.Dk) o[(k0 + r) * a.o_sd] = TT::from_f32(c[tb][r]);
+              for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                  if (k0 + 4 * p + r < a.Dk) o[(k0 + 4 * p + r) * a.o_sd] = TT::from_f32(c[p][tb][r]);
             }
           }
         }
@@ -548,7 +693,7 @@ rot_kernel(const RotArgs a) {
   };
   uint4 bA[TB][4], bB[TB][4];
   if (wave < nstep) load(bA, wave);
-  for (int64_t st = wave; st < nstep; st += 2 * kWaves) {
+  for (int st = wave; st < nstep; st += 2 * kWaves) {
     load(bB, st + kWaves);
     compute(bA, st);
     if (st + kWaves >= nstep) break;
@@ -566,7 +711,7 @@ rot_kernel(const RotArgs a) {
         v += shfl_xor(v, 2);
         v += shfl_xor(v, 4);
         v += shfl_xor(v, 8);
-        if (n == 0) s_sc[wave][16 * t + 4 * g + r] = v;
+        if (n == 0) s_sc[wave][kept_of<NT>(t, 4 * g + r)] = v;
       }
     __syncthreads();
     for (int kk = tid; kk < NT * 16; kk += kThreads) {
@@ -826,7 +971,8 @@ __global__ void __launch_bounds__(128) gather_kernel(const void* R, int r_dtype,
 // G heads.  The covariance goes through LDS (rows padded to 129), so the
 // transposed read is conflict-free; out may alias cov.  CV / QV: 16-byte
 // row loads of the covariance / the queries (unit inner stride, aligned).
-constexpr int kQHeads = 8;  // query heads whose window rows are loaded together (G <= 8: one batch)
+constexpr int kQHeads = 4;  // query heads whose window rows are loaded together (eight at a time took 134
+                            // registers and left the mean launch, which carries this code, at three waves per SIMD)
 
 // Thread (rs = t/16, c8 = t%16) of 256: the fp32 sums over the G query
 // heads of window rows rs and rs + 16 (of the last W rows), channels
@@ -951,7 +1097,7 @@ __device__ void floored_query_norms(const float (&acc)[2][8], int W, int D, floa
   if (tid < D) {
     v = s_qn[tid];
     int rank = 0;
-#pragma unroll
+#pragma unroll 8
     for (int j4 = 0; j4 < 32; ++j4) {
       const float4 u = *(const float4*)&s_qn[4 * j4];
       const float uu[4] = {u.x, u.y, u.z, u.w};
@@ -971,23 +1117,6 @@ __device__ void floored_query_norms(const float (&acc)[2][8], int W, int D, floa
     s_qn[tid] = tid >= D ? 0.f : isnan(fl) ? fl : fmaxf(v, fl);
   }
   __syncthreads();
-}
-
-// 1e-4 max(mean|diag(C o qn qn^T)|, 1e-6) from the diagonal dg_in[c] =
-// C[c][c] (threads 0..D-1; the sum is a fixed xor tree in each of waves 0
-// and 1, then the two halves, times torch's mean factor rfac = fp32(1/D)),
-// as the weighted covariance's ridge.
-__device__ __forceinline__ float weighted_ridge(float diag, const float* s_qn, int tid, int D, float rfac,
-                                                float* s_wsum) {
-  if (tid < 128) {
-    const float qd = s_qn[tid];
-    float dg = tid < D ? fabsf(diag * (qd * qd)) : 0.f;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) dg += shfl_xor(dg, off);
-    if ((tid & 63) == 0) s_wsum[tid >> 6] = dg;
-  }
-  __syncthreads();
-  return 1e-4f * fmaxf((s_wsum[0] + s_wsum[1]) * rfac, 1e-6f);
 }
 
 // grid (B*H_kv), 256 threads: query-aware weighting of one covariance
@@ -1082,10 +1211,7 @@ __global__ void __launch_bounds__(256) qweight_kernel(const float* cov, int64_t 
 template <class TT>
 __global__ void __launch_bounds__(kThreads) covfin_qw_kernel(const float* part, const float* dpart, int splits,
                                                              const float* mean_part, int mean_splits, float mfac,
-                                                             const float* qn, float* cov, int64_t cs_b,
-                                                             int64_t cs_h, int64_t cs_r, int64_t cs_c, float* mu,
-                                                             int64_t ms_b, int64_t ms_h, int64_t ms_c, int H, int D,
-                                                             float rfac) {
+                                                             CovOut o, int H, int D) {
   __shared__ float s_t[256];
   __shared__ __align__(16) float s_qn[128];
   __shared__ float s_wsum[2];
@@ -1095,7 +1221,7 @@ __global__ void __launch_bounds__(kThreads) covfin_qw_kernel(const float* part, 
   // tile entry tid and (threads < 128) diagonal entry C[tid][tid]
   float sum = strided_sum(pb + t * 256 + tid, splits, kTiles * 256);
   float dsum = strided_sum(dpart + (int64_t)bh * splits * 128 + (tid & 127), splits, 128);
-  const float qv = qn[(int64_t)bh * 128 + (tid & 127)];
+  const float qv = o.qn[(int64_t)bh * 128 + (tid & 127)];
   asm volatile("" : "+v"(sum));  // fp32, then the key dtype (two roundings)
   asm volatile("" : "+v"(dsum));
   s_t[tid] = TT::to_f32(TT::from_f32(sum));
@@ -1103,9 +1229,9 @@ __global__ void __launch_bounds__(kThreads) covfin_qw_kernel(const float* part, 
   const float dx = TT::to_f32(TT::from_f32(dsum));
   const float diag = 0.5f * (dx + dx);  // the symmetrised diagonal, as covfin writes it
   __syncthreads();
-  const float ridge = weighted_ridge(diag, s_qn, tid, D, rfac, s_wsum);
+  const float ridge = weighted_ridge(diag, s_qn, tid, D, o.rfac, s_wsum);
   const int i = tile_row(t), j = tile_col(t), m = tid >> 4, n = tid & 15;
-  float* cb = cov + b * cs_b + (int64_t)h * cs_h;
+  float* cb = o.cov + b * o.c_b + (int64_t)h * o.c_h;
   const int r = 8 * m + i, c = 8 * n + j;
   const float rc = s_t[tid];
   const float cr = i == j ? s_t[n * 16 + m] : rc;
@@ -1113,11 +1239,11 @@ __global__ void __launch_bounds__(kThreads) covfin_qw_kernel(const float* part, 
   const float w = s_qn[r] * s_qn[c];
   const float a = sym * w, bt = symt * w;
   if (r < D && c < D) {
-    cb[r * cs_r + c * cs_c] = 0.5f * (a + bt) + (r == c ? ridge : 0.f);
-    if (i != j) cb[c * cs_r + r * cs_c] = 0.5f * (bt + a);
+    cb[r * o.c_r + c * o.c_c] = 0.5f * (a + bt) + (r == c ? ridge : 0.f);
+    if (i != j) cb[c * o.c_r + r * o.c_c] = 0.5f * (bt + a);
   }
-  if (t == 0 && tid < D && mu)
-    mu[b * ms_b + (int64_t)h * ms_h + tid * ms_c] = head_mean(mean_part, bh, mean_splits, tid, mfac);
+  if (t == 0 && tid < D && o.mu)
+    o.mu[b * o.m_b + (int64_t)h * o.m_h + tid * o.m_c] = head_mean(mean_part, bh, mean_splits, tid, mfac);
 }
 
 }  // namespace prefill
@@ -1179,18 +1305,42 @@ int splits_for(int64_t bh, int64_t S, int cus, int64_t min_tokens) {
   return (int)want;
 }
 
+// Bytes of the memory-side cache (MALL): larger tensors are streamed.
+constexpr int64_t kMallBytes = INT64_C(256) << 20;
+
 struct CovPlan {
   int mean_splits, cov_splits;
   int64_t mean_chunk, cov_chunk;
   size_t off_mean, off_cov, off_diag, off_qn, total;
 };
 
+// Workgroups per head of the covariance pass: the split of least cost, in
+// token times of a full round (two workgroups per CU, the kernel's register
+// budget): rounds x (tokens per workgroup + 360 for the centre, the sum of
+// the waves and the partial, 8 us) + 0.66 per partial for the finalisation's
+// reads (a single workgroup per head has none).  B=10, 32 heads, 4000 tokens:
+// 2 -> 3 splits, 177 -> 161 us; B=32, 14000 tokens: one.
+int cov_splits_for(int64_t bh, int64_t S, int cus) {
+  if (S <= 0 || bh <= 0) return 1;
+  const int64_t cap = std::min<int64_t>(cdiv(S, 256), 64);
+  double best = 0;
+  int splits = 1;
+  for (int64_t s = 1; s <= cap; ++s) {
+    const double cost = (double)cdiv(bh * s, 2 * (int64_t)cus) * (double)(cdiv(S, s) + 360) + (s > 1 ? 0.66 * bh * s : 0);
+    if (s == 1 || cost < best) best = cost, splits = (int)s;
+  }
+  return splits;
+}
+
 CovPlan cov_plan(int64_t B, int64_t H, int64_t S, int cus) {
   CovPlan p;
   const int64_t bh = B * H;
-  p.mean_splits = splits_for(bh, S, cus, 256);
+  // the mean pass has no epilogue to speak of: at most 512 tokens a
+  // workgroup, so that grids of many heads end evenly (B=32, 32 heads, 14000
+  // tokens, one workgroup per head: 938 us, 3.9 TB/s; 28 per head: 560)
+  p.mean_splits = (int)std::min<int64_t>(std::max<int64_t>(splits_for(bh, S, cus, 256), cdiv(S, 512)), 4096);
   p.mean_chunk = cdiv(S > 0 ? S : 1, p.mean_splits);
-  p.cov_splits = splits_for(bh, S, cus, 512);
+  p.cov_splits = cov_splits_for(bh, S, cus);
   p.cov_chunk = cdiv(S > 0 ? S : 1, p.cov_splits);
   p.off_mean = 0;
   p.off_cov = align256((size_t)bh * p.mean_splits * 128 * sizeof(float));
@@ -1255,36 +1405,52 @@ hipError_t launch_cov(const KeyView& k, bool vec, const CovPlan& p, int64_t B, f
     dpart = (float*)((char*)ws + p.off_diag);
     gmq.x += 1;
   }
+  const CovOut o{cov, cov_t->stride[0], cov_t->stride[1], cov_t->stride[2], cov_t->stride[3], mu,
+                 mu_t ? mu_t->stride[0] : 0, mu_t ? mu_t->stride[1] : 0, mu_t ? mu_t->stride[2] : 0,
+                 qw ? qn : nullptr, rfac};
   const int64_t mc = p.mean_chunk, cc = p.cov_chunk;
   const int ms = p.mean_splits, cs = p.cov_splits;
-  if (vec) {
+  auto mean = [&](auto v, auto nt) {
+    constexpr bool V = decltype(v)::value, N = decltype(nt)::value;
     if (!qw)
-      hipLaunchKernelGGL((mean_kernel<TT, true, false, false>), gm, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
+      hipLaunchKernelGGL((mean_kernel<TT, V, N, false, false>), gm, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
     else if (qw->vec)
-      hipLaunchKernelGGL((mean_kernel<TT, true, true, true>), gmq, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
+      hipLaunchKernelGGL((mean_kernel<TT, V, N, true, true>), gmq, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
     else
-      hipLaunchKernelGGL((mean_kernel<TT, true, true, false>), gmq, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
-    hipLaunchKernelGGL((cov_kernel<TT, true>), gc, dim3(kThreads), 0, s, k, cc, cs, mpart, ms, mfac, cpart, dpart);
+      hipLaunchKernelGGL((mean_kernel<TT, V, N, true, false>), gmq, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
+  };
+  auto covk = [&](auto kern) {
+    hipLaunchKernelGGL(kern, gc, dim3(kThreads), 0, s, k, cc, cs, mpart, ms, mfac, cpart, dpart, o);
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  bool finished = false;
+  if constexpr (TT::kBytes == 2) {
+    if (vec) {
+      // Keys past the memory-side cache are streamed; one workgroup per head
+      // finishes its head
+      const bool nt = bh * k.S * k.D * 2 > kMallBytes;
+      finished = cs == 1;
+      nt ? mean(yes, yes) : mean(yes, no);
+      if (finished)
+        nt ? covk(cov_kernel<TT, true, true, true>) : covk(cov_kernel<TT, true, false, true>);
+      else
+        nt ? covk(cov_kernel<TT, true, true, false>) : covk(cov_kernel<TT, true, false, false>);
+    } else {
+      mean(no, no);
+      covk(cov_kernel<TT, false>);
+    }
   } else {
-    if (!qw)
-      hipLaunchKernelGGL((mean_kernel<TT, false, false, false>), gm, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
-    else if (qw->vec)
-      hipLaunchKernelGGL((mean_kernel<TT, false, true, true>), gmq, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
-    else
-      hipLaunchKernelGGL((mean_kernel<TT, false, true, false>), gmq, dim3(kThreads), 0, s, k, mc, ms, mpart, qa);
-    hipLaunchKernelGGL((cov_kernel<TT, false>), gc, dim3(kThreads), 0, s, k, cc, cs, mpart, ms, mfac, cpart, dpart);
+    vec ? mean(yes, no) : mean(no, no);
+    vec ? covk(cov_kernel<TT, true>) : covk(cov_kernel<TT, false>);
   }
-  if (qw) {
-    hipLaunchKernelGGL((covfin_qw_kernel<TT>), dim3(kTiles, (unsigned)bh), dim3(kThreads), 0, s, cpart, dpart,
-                       p.cov_splits, mpart, p.mean_splits, mfac, qn, cov, cov_t->stride[0], cov_t->stride[1],
-                       cov_t->stride[2], cov_t->stride[3], mu, mu_t ? mu_t->stride[0] : 0,
-                       mu_t ? mu_t->stride[1] : 0, mu_t ? mu_t->stride[2] : 0, k.H, k.D, rfac);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL((covfin_kernel<TT>), dim3(kTiles, (unsigned)bh), dim3(kThreads), 0, s, cpart, p.cov_splits,
-                     mpart, p.mean_splits, mfac, cov, cov_t->stride[0], cov_t->stride[1], cov_t->stride[2],
-                     cov_t->stride[3], mu, mu_t ? mu_t->stride[0] : 0, mu_t ? mu_t->stride[1] : 0,
-                     mu_t ? mu_t->stride[2] : 0, k.H, k.D);
+  if (finished) return hipGetLastError();
+  const dim3 gf(kTiles, (unsigned)bh);
+  if (qw)
+    hipLaunchKernelGGL((covfin_qw_kernel<TT>), gf, dim3(kThreads), 0, s, cpart, dpart, cs, mpart, ms, mfac, o, k.H,
+                       k.D);
+  else
+    hipLaunchKernelGGL((covfin_kernel<TT>), gf, dim3(kThreads), 0, s, cpart, cs, mpart, ms, mfac, o, k.H, k.D);
   return hipGetLastError();
 }
 
@@ -1418,7 +1584,9 @@ hipError_t launch_rot(const RotArgs& a, bool vec, dim3 grid, hipStream_t s) {
     else
       hipLaunchKernelGGL((rot32_kernel<NT, false, SCORE>), grid, dim3(kThreads), 0, s, a);
   } else {
-    if (vec)
+    if (!SCORE && vec && a.o_vec && a.k.D == 128)
+      hipLaunchKernelGGL((rot_kernel<TT, NT, true, false, true>), grid, dim3(kThreads), 0, s, a);
+    else if (vec)
       hipLaunchKernelGGL((rot_kernel<TT, NT, true, SCORE>), grid, dim3(kThreads), 0, s, a);
     else
       hipLaunchKernelGGL((rot_kernel<TT, NT, false, SCORE>), grid, dim3(kThreads), 0, s, a);
@@ -1457,7 +1625,17 @@ void fill_rot(RotArgs& a, const KeyView& k, const rk_tensor* R, int64_t Dk) {
   a.Dk = (int32_t)Dk;
 }
 
-int rot_splits(int64_t bh, int64_t S, int cus) { return splits_for(bh, S, cus, 512); }
+// One round of four workgroups per CU (the STORE kernels' occupancy), of at
+// least 128 tokens (one 32-token step per wave) and at most 512: shorter
+// workgroups even out the end of grids of many rounds (B=32, 32 heads, 14000
+// tokens, keep 32: 911 us with one workgroup per head, 866 at 1536 tokens,
+// 823 at 512, 830 at 256; one image, 2304 tokens, keep 64: 9.7 -> 8.8 us
+// with 128-token workgroups allowed).
+int rot_splits(int64_t bh, int64_t S, int cus) {
+  if (S <= 0 || bh <= 0) return 1;
+  const int64_t want = std::max(std::min(cdiv(4 * (int64_t)cus, bh), cdiv(S, 128)), cdiv(S, 512));
+  return (int)std::min<int64_t>(want, 4096);
+}
 
 }  // namespace
 
@@ -1486,6 +1664,9 @@ extern "C" int rk_rotate_keys(const rk_tensor* keys, const rk_tensor* R_partial,
   a.o_sh = out->stride[1];
   a.o_ss = out->stride[2];
   a.o_sd = out->stride[3];
+  a.o_vec = rows_vec(out, Dk) ? 1 : 0;
+  a.o_stream = rk::numel(out) * rk::dtype_size(out->dtype) > kMallBytes ? 1 : 0;
+  a.r_vec = R_partial->dtype == keys->dtype && rows_vec(R_partial, Dk) ? 1 : 0;
   a.splits = rot_splits(B * H, k.S, cus);
   a.chunk = cdiv(k.S, a.splits);
   const dim3 grid((unsigned)a.splits, (unsigned)(B * H));
