@@ -5,26 +5,31 @@
 //
 // Per iteration, as the reference:
 //   W = C V;  G = W^T W;  G += eps * mean(diag G) * I;  G = L L^T;  V = W L^-T
-// One 256-thread workgroup owns one matrix and keeps everything in LDS
-// (C 128 x 132, V/W 128 x (KP+4), G KP x (KP+1), L KP x KP, (L^-1)^T
-// KP x (KP+4), 4 KB scratch: 153 KB at KP = 64).  The three products run on v_mfma_f32_16x16x4_f32:
-//   W = C V            8 x KP/16 tiles of 16 x 16 over the four waves
-//   G = W^T W          (KP/16)^2 tiles
-//   Cholesky + L^-1    KP <= 32: one pass in wave 0 (lane i holds row i of
-//                      G; column j of L goes through LDS and serves both
-//                      the row updates and step j of the substitution
-//                      L x = e_c that lane c runs for column c of L^-1).
-//                      KP = 64: 16-column panels, each factored in wave 0
-//                      with its diagonal block of L^-1; the trailing update
-//                      of G and the blocks of L^-1 below the diagonal run
-//                      on the MFMA over all waves (141.7 -> 100.5 us for 32
-//                      matrices at k = 64; no gain at k <= 32)
-//   V = W (L^-1)^T     8 x KP/16 tiles
+// One 256-thread workgroup owns one matrix.  C stays in registers, V^T, W^T,
+// G, X = L^-1 and L in LDS (19 / 48 / 120 KB at KP = 16 / 32 / 64, so
+// several matrices share a CU at KP <= 32).  The products run on
+// v_mfma_f32_16x16x4_f32, 32 cycles each on the wave's SIMD, which bounds C V
+// and the solve; each is formed transposed, so that the accumulators of one
+// are the operands of the next:
+//   W^T = V^T C^T      KP/16 x 8 tiles of 16 x 16, two columns of them a wave
+//   G = W^T W          the lower tiles; those off the diagonal beside the
+//                      first panel's elimination
+//   Cholesky, L^-1     16-column panels: the diagonal block is inverted in
+//                      wave 0 by DPP elimination (invert_block), the rest is
+//                      MFMA products on waves 1-3 while wave 0 inverts the
+//                      next one
+//   V^T = X W^T        from W^T's registers
+// Cycles of one iteration (wave 0, KP = 16 / 32 / 64): W 2400 / 4500 /
+// 8800, diagonal of G 1400, ridge 350, panels 2100 / 5300 / 11900, V 360 /
+// 950 / 2800.  32 matrices, 5 iterations: 26.4 -> 20.0 us at k = 16, 47.6 ->
+// 34.5 at 32, 115 -> 65 at 64; 1024 matrices 109 -> 50, 194 -> 109, 455 -> 279.
 // Padding columns of V are zero, so their rows and columns of G are too: a
 // unit diagonal there makes that block the identity, and V keeps them zero.
 // The start block V0 comes from the caller (the reference draws it with
 // torch.randn from a seeded device generator, rotation.py:88-90).
 #include <math.h>
+
+#include <utility>
 
 #include "rk_common.h"
 #include "rk_host.h"
@@ -38,8 +43,6 @@ typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 
 constexpr int kD = 128;
 constexpr int kThreads = 256;
-constexpr int kCPad = kD + 4;  // C row stride: 16-byte reads of rows n = 0..15 cover all 64 banks
-constexpr int kLook = 3;       // single-pass Cholesky: column entries passed by readlane ahead of the LDS broadcast
 
 // D = A B + D on v_mfma_f32_16x16x4_f32 (A 16x4, B 4x16): lane (g, n) supplies
 // A[n][g] and B[g][n] and holds D[4g + i][n], i = 0..3.
@@ -54,435 +57,386 @@ __device__ __forceinline__ lds_f32* opaque_lds(float* p) {
   return (lds_f32*)(uintptr_t)a;
 }
 
+// LDS written and read within one wave: no barrier, but the compiler may
+// not move the accesses across this point.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Lane J of each 16-lane row, in every lane of the row (DPP row_newbcast).
+template <int J>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + J, 0xf, 0xf, true));
+}
+
+// The sum over each 16-lane row, in every lane of the row (DPP rotations).
+__device__ __forceinline__ float row_sum(float v) {
+  auto rot = [](float x, auto ctrl) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  v += rot(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+  v += rot(v, std::integral_constant<int, 0x124>{});
+  v += rot(v, std::integral_constant<int, 0x122>{});
+  v += rot(v, std::integral_constant<int, 0x121>{});
+  return v;
+}
+__device__ __forceinline__ float lane_value(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+
+// v += m * (v of lane J of the 16-lane row), for a group of registers.  As
+// v_fmac_f32 with the DPP row broadcast on its first source: written out,
+// since from the builtin the compiler keeps a v_mov_dpp per value, all
+// through one register, with the two wait states a DPP read needs before
+// each (3.1 against 2.8 us an iteration at k = 16).  The wait states stand
+// around the group instead: in front for values that the instructions before
+// may have written, behind for DPP reads of these results.  The instructions
+// of a group do not depend on each other.
+#define RK_F(d) "v_fmac_f32_dpp " d ", " d ", %[m] row_newbcast:%c[j] row_mask:0xf bank_mask:0xf\n\t"
+#define RK_F4(d0, d1, d2, d3) RK_F(d0) RK_F(d1) RK_F(d2) RK_F(d3)
+#define RK_V4(v) "+v"((v)[0]), "+v"((v)[1]), "+v"((v)[2]), "+v"((v)[3])
+#define RK_F8 RK_F4("%0", "%1", "%2", "%3") RK_F4("%4", "%5", "%6", "%7")
+#define RK_F12 RK_F8 RK_F4("%8", "%9", "%10", "%11")
+#define RK_F16 RK_F12 RK_F4("%12", "%13", "%14", "%15")
+#define RK_F20 RK_F16 RK_F4("%16", "%17", "%18", "%19")
+// G0: the first group of four columns of a that still changes
+template <int J, int G0>
+__device__ __forceinline__ void fmac_bcast(float (&a)[16], float (&y)[4], float m) {
+  if constexpr (G0 == 0)
+    asm volatile("s_nop 1\n\t" RK_F20 "s_nop 1"
+                 : RK_V4(a), RK_V4(a + 4), RK_V4(a + 8), RK_V4(a + 12), RK_V4(y)
+                 : [m] "v"(m), [j] "n"(J));
+  else if constexpr (G0 == 1)
+    asm volatile("s_nop 1\n\t" RK_F16 "s_nop 1"
+                 : RK_V4(a + 4), RK_V4(a + 8), RK_V4(a + 12), RK_V4(y)
+                 : [m] "v"(m), [j] "n"(J));
+  else if constexpr (G0 == 2)
+    asm volatile("s_nop 1\n\t" RK_F12 "s_nop 1" : RK_V4(a + 8), RK_V4(a + 12), RK_V4(y) : [m] "v"(m), [j] "n"(J));
+  else
+    asm volatile("s_nop 1\n\t" RK_F8 "s_nop 1" : RK_V4(a + 12), RK_V4(y) : [m] "v"(m), [j] "n"(J));
+}
+#undef RK_F20
+#undef RK_F16
+#undef RK_F12
+#undef RK_F8
+#undef RK_V4
+#undef RK_F4
+#undef RK_F
+
+// Step J of invert_block: subtract a_nJ / a_JJ times row J from the rows
+// n > J, in the block (whole groups of four columns from J + 1 on: the
+// columns up to J are not read again) and in the identity being turned
+// into its inverse.
+template <int J>
+__device__ __forceinline__ void eliminate(float (&a)[16], float (&y)[4], float& own, int n, bool& bad) {
+  const float piv = row_bcast<J>(a[J]);
+  bad |= !__builtin_amdgcn_classf(piv, 0x180);  // positive, finite, not zero
+  own = n == J ? piv : own;
+  if constexpr (J < 15)  // no row follows the last
+    fmac_bcast<J, (J + 1) / 4>(a, y, n > J ? -(a[J] * __builtin_amdgcn_rcpf(piv)) : 0.f);
+}
+
+template <int... J>
+__device__ __forceinline__ void eliminate_all(float (&a)[16], float (&y)[4], float& own, int n, bool& bad,
+                                              std::integer_sequence<int, J...>) {
+  (eliminate<J>(a, y, own, n, bad), ...);
+}
+
+// X = L^-1 of a symmetric positive definite 16 x 16 block A = L L^T, in one
+// wave: lane (g, n) brings row n (every g the same) and leaves with
+// X[n][4 g + c], c = 0..3, which is the A operand of an MFMA over X's
+// columns.  Gaussian elimination on [A | I]: A's rows in every 16-lane
+// row, four columns of I each; the eliminated identity is D^1/2 X with D
+// the pivots.  Rows are passed by DPP, so a step is a short chain (the
+// pivot's broadcast, its reciprocal, the multiplier, the next pivot's
+// update) with no LDS round trip; about 130 cycles a step, most of it the
+// issue of its fused multiply-adds.
+__device__ __forceinline__ f32x4 invert_block(float (&a)[16], int g, int n, bool& bad) {
+  float y[4], own = 1.f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) y[c] = n == 4 * g + c ? 1.f : 0.f;
+  eliminate_all(a, y, own, n, bad, std::make_integer_sequence<int, 16>{});
+  const float r = __builtin_amdgcn_rsqf(own);
+  return f32x4{y[0] * r, y[1] * r, y[2] * r, y[3] * r};
+}
+
 template <int KP>
-__global__ void __launch_bounds__(kThreads) power_iter_kernel(
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(KP > 32 ? 1 : 2))) power_iter_kernel(
     const float* cov, int64_t c_sb, int64_t c_sh, int64_t c_sr, int64_t c_sc, const float* v0, int64_t v_sb,
     int64_t v_sh, int64_t v_sr, int64_t v_sc, float* out, int64_t o_sb, int64_t o_sh, int64_t o_sr,
-    int64_t o_sc, int H, int k, int iters, float eps, int32_t* info, int D) {
-  // V / W and (L^-1)^T row stride, 4 mod 16: reads of rows 4g + r (r fixed)
-  // at columns n = 0..15 hit banks 16g + n, and 16-byte reads of rows n at
-  // column 4g cover all 64 banks
-  constexpr int SP = KP + 4;
-  constexpr int LP = KP + 4;
-  constexpr int GP = KP + 1;        // G row (row per lane in the Cholesky)
-  constexpr int NTJ = KP / 16;      // 16-column tiles of W / V
-  constexpr int TPW = 8 * NTJ / 4;  // 16 x 16 tiles of W per wave
-  constexpr int NG = NTJ * NTJ;     // 16 x 16 tiles of G
-  constexpr int TPG = NG >= 4 ? NG / 4 : 1;
-  constexpr int NP16 = KP / 16;     // Cholesky panels
-  __shared__ __align__(16) float sC[kD * kCPad];
-  __shared__ __align__(16) float sV[kD * SP];
-  // G, then L by columns; the tail takes the idle lanes' last column writes
-  // G (the single-pass path rewrites it as L by columns; its tail takes the
-  // idle lanes' last column writes)
-  __shared__ __align__(16) float sG[KP * GP > KP * KP + 64 ? KP * GP : KP * KP + 64];
-  // blocked path: L by columns, sLc[j * KP + m] = L_mj (1 / L_jj on the diagonal)
-  __shared__ __align__(16) float sLc[KP > 32 ? KP * KP : 1];
-  // X = L^-1 transposed, sLt[c * LP + i] = X[i][c]; rows >= KP: scratch for
-  // the single-pass path's idle lanes
-  __shared__ float sLt[64 * LP];
-  __shared__ float sT[KP > 32 ? 4 * 256 : 1];  // blocked path: per-wave 16 x 16 product scratch
+    int64_t o_sc, int H, int k, int iters, float eps, int32_t* info, int cvec, int D) {
+  constexpr int NT = KP / 16;  // 16-column tiles of V / W, 16-column panels of G
+  // Row strides of 4 mod 16 floats: 16-byte reads of rows n = 0..15 at column
+  // 4g, and accumulator writes of rows 4g + i at column n, cover all 64 banks
+  constexpr int VS = kD + 4;
+  constexpr int GS = KP + 4;
+  __shared__ __align__(16) float sVt[KP * VS];  // V^T
+  __shared__ __align__(16) float sWt[KP * VS];  // W^T
+  __shared__ __align__(16) float sG[KP * GS];   // G, lower tiles
+  __shared__ __align__(16) float sX[KP * GS];   // X = L^-1, lower tiles
+  __shared__ __align__(16) float sL[NT > 1 ? KP * GS : 4];  // L, tiles below the diagonal
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, n = lane & 15;
   const int bh = blockIdx.x, b = bh / H, h = bh - b * H;
   const float* C = cov + b * c_sb + (int64_t)h * c_sh;
   const float* V0 = v0 + b * v_sb + (int64_t)h * v_sh;
 
-  // Stage C and V0 in LDS.  The loads of a batch are all issued before any
-  // of them is stored, so the copy costs a few memory round trips rather
-  // than one per element.  With a head_dim D < 128 the rows and columns
-  // past D are zeros (their loads re-read an in-bounds entry): W = C V, G,
-  // L and V = W L^-T then equal the D x D iteration's, with exact zeros in
-  // the padded rows.
-  constexpr int kCB = 16;  // elements per thread per batch
-  if (D == kD) {  // (the addresses step by two rows per element, no clamps)
-    for (int e0 = 0; e0 < kD * kD; e0 += kThreads * kCB) {
-      float v[kCB];
+  // C stays in registers over the iterations: wave w owns its row tiles 2w
+  // and 2w + 1, lane (g, n) of k-group q the entries C[16 ti + n][16 q + 4 g + r].
+  // With a head_dim D < 128 the rows and columns past D are zeros (their
+  // loads re-read an in-bounds entry): W = C V, G, L and V = W L^-T then
+  // equal the D x D iteration's, with exact zeros in the padded rows.
+  f32x4 cf[2][8];
+  if (cvec) {  // (D == 128, 16-byte rows)
 #pragma unroll
-      for (int i = 0; i < kCB; ++i) {
-        const int e = e0 + i * kThreads + tid, r = e >> 7, c = e & 127;
-        v[i] = C[r * c_sr + c * c_sc];
-      }
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int i = 0; i < kCB; ++i) {
-        const int e = e0 + i * kThreads + tid;
-        sC[(e >> 7) * kCPad + (e & 127)] = v[i];
-      }
-    }
+      for (int q = 0; q < 8; ++q)
+        cf[t][q] = *(const f32x4*)(C + (int64_t)(16 * (2 * wave + t) + n) * c_sr + 16 * q + 4 * g);
   } else {
-    for (int e0 = 0; e0 < kD * kD; e0 += kThreads * kCB) {
-      float v[kCB];
 #pragma unroll
-      for (int i = 0; i < kCB; ++i) {
-        const int e = e0 + i * kThreads + tid, r = e >> 7, c = e & 127;
-        const float x = C[min(r, D - 1) * c_sr + min(c, D - 1) * c_sc];
-        v[i] = r < D && c < D ? x : 0.f;
-      }
+    for (int t = 0; t < 2; ++t) {
+      const int row = 16 * (2 * wave + t) + n;
+      const float* cr = C + (int64_t)min(row, D - 1) * c_sr;
 #pragma unroll
-      for (int i = 0; i < kCB; ++i) {
-        const int e = e0 + i * kThreads + tid;
-        sC[(e >> 7) * kCPad + (e & 127)] = v[i];
-      }
+      for (int q = 0; q < 8; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int col = 16 * q + 4 * g + r;
+          const float x = cr[(int64_t)min(col, D - 1) * c_sc];
+          cf[t][q][r] = row < D && col < D ? x : 0.f;
+        }
     }
   }
-  constexpr int kVB = kD * KP / kThreads < kCB ? kD * KP / kThreads : kCB;  // divides kD * KP / kThreads
-  static_assert((kD * kD) % (kThreads * kCB) == 0 && (kD * KP) % (kThreads * kVB) == 0, "whole batches");
+  // V0 transposed into LDS, a batch of loads at a time
+  constexpr int kVB = kD * KP / kThreads < 16 ? kD * KP / kThreads : 16;
+  static_assert((kD * KP) % (kThreads * kVB) == 0, "whole batches");
   for (int e0 = 0; e0 < kD * KP; e0 += kThreads * kVB) {
     float v[kVB];
 #pragma unroll
     for (int i = 0; i < kVB; ++i) {
       const int e = e0 + i * kThreads + tid, r = e / KP, c = e - r * KP;
-      v[i] = c < k && r < D ? V0[r * v_sr + c * v_sc] : 0.f;
+      const float x = V0[min(r, D - 1) * v_sr + min(c, k - 1) * v_sc];
+      v[i] = c < k && r < D ? x : 0.f;
     }
 #pragma unroll
     for (int i = 0; i < kVB; ++i) {
-      const int e = e0 + i * kThreads + tid, r = e / KP;
-      sV[r * SP + (e - r * KP)] = v[i];
+      const int e = e0 + i * kThreads + tid, r = e / KP, c = e - r * KP;
+      sVt[c * VS + r] = v[i];
     }
   }
-  for (int e = tid; e < 64 * LP; e += kThreads) sLt[e] = 0.f;  // X's upper blocks are never written
   __syncthreads();
 
-  // Wave w owns the 16 x 16 output tiles w, w + 4, w + 8, ... of each
-  // product.  With NTJ column tiles (NTJ divides 4) tile w + 4t sits at row
-  // tile ti0 + t * RS and column tile tj0.
-  constexpr int RS = 4 / NTJ;
-  const int ti0 = wave / NTJ, tj0 = wave - (wave / NTJ) * NTJ;
-  // a pivot that is not positive and finite (wave 0, uniform)
-  bool bad = false;
+  bool bad = false;  // a pivot that is not positive and finite (wave 0)
+  f32x4 vt[NT][2];   // V^T tiles (tj, 2w + t): lane (g, n) holds V^T[16 tj + 4 g + i][16 ti + n]
+  if (iters == 0) {
+#pragma unroll
+    for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vt[tj][t][i] = sVt[(16 * tj + 4 * g + i) * VS + 16 * (2 * wave + t) + n];
+  }
 
   for (int it = 0; it < iters; ++it) {
     // LDS bases, opaque to the compiler once per iteration: every access
     // below is one of these plus a lane part plus an immediate offset
     // (< 64 KB), so no per-access address is kept in a register across
     // iterations
-    lds_f32* const lC = opaque_lds(sC);
-    lds_f32* const lV = opaque_lds(sV);
+    lds_f32* const lV = opaque_lds(sVt);
+    lds_f32* const lW = opaque_lds(sWt);
     lds_f32* const lG = opaque_lds(sG);
-    lds_f32* const lLt = opaque_lds(sLt);
-    lds_f32* const lLc = opaque_lds(sLc);
-    lds_f32* const lT = opaque_lds(sT);
+    lds_f32* const lX = opaque_lds(sX);
+    lds_f32* const lL = opaque_lds(sL);
 
-    // ---- W = C V on the MFMA.  In the four MFMA steps of k-group q, lane
-    // (g, n) supplies k = 16q + 4g + r, r = 0..3 (any assignment of k to
-    // (step, g) sums the same products), so one 16-byte read of C's row
-    // feeds all four; group q + 1 is read while group q computes
-    {
-      const lds_f32* pa = lC + (16 * ti0 + n) * kCPad + 4 * g;  // C[16 ti + n][16 q + 4 g + r]
-      const lds_f32* pb = lV + 4 * g * SP + 16 * tj0 + n;       // V[16 q + 4 g + r][16 tj + n]
-      f32x4 acc[TPW], a[2][TPW];
-      float bv[2][4];
+    // ---- W^T = V^T C^T: the accumulators leave each lane with
+    // W^T[16 tj + 4 g + i][16 ti + n], the B operand of the solve below
+    f32x4 wt[NT][2];
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tj = 0; tj < NT; ++tj) wt[tj][0] = wt[tj][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) a[0][t] = *(const lds_f32x4*)&pa[16 * RS * t * kCPad];
+    for (int q = 0; q < kD / 16; ++q) {
+      f32x4 a[NT];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bv[0][r] = pb[r * SP];
+      for (int tj = 0; tj < NT; ++tj) a[tj] = *(const lds_f32x4*)&lV[(16 * tj + n) * VS + 16 * q + 4 * g];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) wt[tj][t] = mfma4(a[tj][r], cf[t][q][r], wt[tj][t]);
+    }
+#pragma unroll
+    for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lW[(16 * tj + 4 * g + i) * VS + 16 * (2 * wave + t) + n] = wt[tj][t][i];
+    __syncthreads();
+
+    // ---- G = W^T W: the diagonal tiles now, one to a wave; the others
+    // below the diagonal by waves 1-3 while wave 0 eliminates the first
+    // panel, which needs only the diagonal.  Two accumulators per tile so
+    // consecutive MFMAs do not wait on each other.
+    auto g_tile = [&](int ti, int tj) {
+      f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int q = 0; q < kD / 16; ++q) {
-        const int cur = q & 1, nxt = cur ^ 1;
-        if (q + 1 < kD / 16) {
+        const f32x4 av = *(const lds_f32x4*)&lW[(16 * tj + n) * VS + 16 * q + 4 * g];
+        const f32x4 bv = ti == tj ? av : *(const lds_f32x4*)&lW[(16 * ti + n) * VS + 16 * q + 4 * g];
 #pragma unroll
-          for (int t = 0; t < TPW; ++t) a[nxt][t] = *(const lds_f32x4*)&pa[16 * RS * t * kCPad + 16 * (q + 1)];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) bv[nxt][r] = pb[(16 * (q + 1) + r) * SP];
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int t = 0; t < TPW; ++t) acc[t] = mfma4(a[cur][t][r], bv[cur][r], acc[t]);
+        for (int r = 0; r < 4; ++r) acc[r & 1] = mfma4(av[r], bv[r], acc[r & 1]);
       }
-      __syncthreads();
-      lds_f32* pw = lV + (16 * ti0 + 4 * g) * SP + 16 * tj0 + n;
+      *(lds_f32x4*)&lG[(16 * ti + n) * GS + 16 * tj + 4 * g] = acc[0] + acc[1];
+    };
 #pragma unroll
-      for (int t = 0; t < TPW; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pw[(16 * RS * t + i) * SP] = acc[t][i];
-    }
+    for (int ti = 0; ti < NT; ++ti)
+      if (wave == ti) g_tile(ti, ti);
     __syncthreads();
 
-    // ---- G = W^T W on the MFMA (NTJ x NTJ tiles; at NTJ = 1 wave 0 alone),
-    // k assigned as in C V (lane (g, n) takes rows 16q + 4g + r); two
-    // accumulators per tile (even / odd r) so consecutive MFMAs do not wait
-    // on each other
-    if (wave < NG) {  // wave-uniform
-      const lds_f32* pa = lV + 4 * g * SP + 16 * ti0 + n;  // W[16 q + 4 g + r][16 ti + n]
-      const lds_f32* pb = lV + 4 * g * SP + 16 * tj0 + n;  // W[16 q + 4 g + r][16 tj + n]
-      f32x4 acc[TPG][2];
-#pragma unroll
-      for (int t = 0; t < TPG; ++t) acc[t][0] = acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-      for (int q = 0; q < kD / 16; ++q) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float bv = pb[(16 * q + r) * SP];
-#pragma unroll
-          for (int t = 0; t < TPG; ++t)
-            acc[t][r & 1] = mfma4(pa[(16 * q + r) * SP + 16 * RS * t], bv, acc[t][r & 1]);
-        }
-      }
-      lds_f32* pg = lG + (16 * ti0 + 4 * g) * GP + 16 * tj0 + n;
-#pragma unroll
-      for (int t = 0; t < TPG; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pg[(16 * RS * t + i) * GP] = acc[t][0][i] + acc[t][1][i];
-    }
-    __syncthreads();
-
-    if constexpr (KP <= 32) {
-    // ---- ridge, Cholesky G = L L^T and L^-1, one pass in wave 0.
-    // Lane i holds row i of G.  Step j takes the pivot from lane j, scales
-    // column j by r_j = 1/sqrt(pivot) and publishes it to LDS (column j of
-    // L, with r_j in place of L_jj); every lane reads the column back as
-    // 16-byte broadcasts and uses it twice: the right-looking update of its
-    // row of G, and step j of the forward substitution L x = e_c that lane
-    // c runs for column c of L^-1.  Rows of finished lanes (lane <= j) keep
-    // being updated in their upper triangle, which is never read.
-    if (wave == 0) {
-      // the lane index, opaque to the compiler, so that the per-column lane
-      // masks below are formed where they are used instead of being hoisted
-      // out of the iteration loop (where they would not fit in registers)
-      int ln = lane;
-      asm volatile("" : "+v"(ln));
-      const int lr = min(ln, KP - 1);  // lanes >= KP compute on a copy of row KP-1 and store nothing
-      const lds_f32* prow = lG + lr * GP;
-      const float dii = prow[lr];
-      float dg = ln < k ? dii : 0.f;
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) dg += shfl_xor(dg, off);
-      const float ridge = eps * (dg / (float)k);
-      // the padding rows and columns of G are zero (V's padding columns
-      // are): a unit diagonal there makes them the identity
-      if (ln < KP) lG[ln * GP + ln] = ln < k ? dii + ridge : 1.f;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      float row[KP], x[KP];
-#pragma unroll
-      for (int m = 0; m < KP; ++m) {
-        row[m] = prow[m];
-        x[m] = ln == m ? 1.f : 0.f;
-      }
-      // G's storage is rewritten below as L by columns (sL[j * KP + m] =
-      // L_mj), after every lane's loads above
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      lds_f32* const sL = lG;
-      // column j is written unconditionally (a guarded store per step would
-      // split the pass into blocks and let the compiler sink the
-      // substitution to the end): lanes >= KP write past column j, into
-      // columns that are rewritten before they are read, or into the tail
-      // of the array
-      lds_f32* const pl = lG + ln;
-#pragma unroll
-      for (int j = 0; j < KP; ++j) {
-        const float piv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, row[j]), j));
-        bad |= !(piv > 0.f && piv <= 3.402823466e38f);
-        const float rj = __builtin_amdgcn_rsqf(piv);
-        const float lij = ln > j ? row[j] * rj : (ln == j ? rj : 0.f);
-        pl[j * KP] = lij;
-        x[j] *= rj;
-        // the entries the next kLook pivots depend on, L_{j+1..j+kLook, j},
-        // come straight from their lanes; the rest of the column goes
-        // through LDS, whose round trip then has kLook steps to complete
-#pragma unroll
-        for (int d = 1; d <= kLook; ++d) {
-          if (j + d < KP) {  // compile-time
-            const float c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lij), j + d));
-            row[j + d] = fmaf(-lij, c, row[j + d]);
-            x[j + d] = fmaf(-c, x[j], x[j + d]);
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int m4 = (j + kLook + 1) & ~3; m4 < KP; m4 += 4) {
-          const f32x4 col = *(const lds_f32x4*)&sL[j * KP + m4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int m = m4 + q;
-            if (m > j + kLook) {  // compile-time
-              row[m] = fmaf(-lij, col[q], row[m]);
-              x[m] = fmaf(-col[q], x[j], x[m]);
-            }
-          }
-        }
-      }
-      // unconditional (rows KP..63 of the array take the idle lanes'
-      // values and are never read): a guarded store would let the compiler
-      // sink the whole substitution into it, holding every column read
-      // above in registers until the end
-      lds_f32* px = lLt + ln * LP;
-#pragma unroll
-      for (int i = 0; i < KP; ++i) px[i] = x[i];
-    }
-    __syncthreads();
-    } else {
-    // ---- ridge: G += eps * mean(diag G) * I (wave 0); the padding rows
-    // and columns of G are zero (V's padding columns are): a unit diagonal
-    // there makes them the identity
+    // ---- ridge: G += eps * mean(diag G) * I (wave 0); the padding rows and
+    // columns of G are zero (V's padding columns are): a unit diagonal there
+    // makes them the identity
     if (wave == 0) {
       const int lr = min(lane, KP - 1);
-      const float dii = lG[lr * GP + lr];
-      float dg = lane < k ? dii : 0.f;
+      const float dii = lG[lr * GS + lr];
+      const float dg = row_sum(lane < k ? dii : 0.f);
+      float tr = lane_value(dg, 0);
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) dg += shfl_xor(dg, off);
-      const float ridge = eps * (dg / (float)k);
-      if (lane < KP) lG[lane * GP + lane] = lane < k ? dii + ridge : 1.f;
+      for (int t = 1; t < NT; ++t) tr += lane_value(dg, 16 * t);
+      const float ridge = eps * (tr / (float)k);
+      if (lane < KP) lG[lane * GS + lane] = lane < k ? dii + ridge : 1.f;
+    } else {
+      int t = 0;
+#pragma unroll
+      for (int ti = 1; ti < NT; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < ti; ++tj)
+          if (t++ % 3 == wave - 1) g_tile(ti, tj);
     }
-    __syncthreads();
 
-    // ---- blocked Cholesky G = L L^T and X = L^-1, 16-column panels.
-    // Panel p: wave 0 factors columns 16p..16p+15 (lane i holds those
-    // entries of row i; the entries of column j that the panel's later
-    // columns need come lane to lane by readlane), writes them to sLc by
-    // columns (r_j = 1 / L_jj on the diagonal) and, in lanes 16p..16p+15,
-    // the diagonal block of X by forward substitution.  All waves then
-    // subtract the panel's product from the trailing lower tiles of G on
-    // the MFMA.  Afterwards X's blocks below the diagonal follow by block
-    // rows: X_qr = -X_qq (sum_{s=r}^{q-1} L_qs X_sr), two 16 x 16 MFMA
-    // products per tile.  X goes to sLt transposed (row c = column c of X,
-    // the layout the solve below reads); its upper blocks stay zero.
+    // ---- blocked Cholesky G = L L^T and X = L^-1 over 16-column panels,
+    // one barrier per panel.  Wave 0 eliminates panel p's diagonal block
+    // (X_pp = L_pp^-1) and publishes it; then it alone prepares the next
+    // diagonal block and eliminates that, while waves 1-3 update the other
+    // trailing tiles G_ij -= L_ip L_jp^T and form row p of X,
+    // X_pr = -X_pp sum_{s=r}^{p-1} L_ps X_sr.  L_qp = G_qp X_pp^T is formed
+    // by every wave that needs it, transposed (X_pp G_qp^T), so that the
+    // accumulators are the operands of the next product.
 #pragma unroll
-    for (int p = 0; p < NP16; ++p) {
-      const int P0 = 16 * p;
+    for (int p = 0; p < NT; ++p) {
       if (wave == 0) {
-        const int lr = min(lane, KP - 1);  // lanes >= KP work on a copy of row KP-1 and store nothing
-        const lds_f32* prow = lG + lr * GP + P0;
-        float a[16], xv[16], lc[16];
+        wave_lds_fence();
+        float a[16];
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-          a[c] = prow[c];
-          xv[c] = lane == P0 + c ? 1.f : 0.f;
+        for (int c4 = 0; c4 < 4; ++c4) {
+          const f32x4 v = *(const lds_f32x4*)&lG[(16 * p + n) * GS + 16 * p + 4 * c4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) a[4 * c4 + i] = v[i];
         }
-#pragma unroll
-        for (int jj = 0; jj < 16; ++jj) {
-          const int j = P0 + jj;
-          const float piv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a[jj]), j));
-          bad |= !(piv > 0.f && piv <= 3.402823466e38f);
-          const float rj = __builtin_amdgcn_rsqf(piv);
-          const float lij = lane > j ? a[jj] * rj : (lane == j ? rj : 0.f);
-          lc[jj] = lij;
-          xv[jj] *= rj;
-#pragma unroll
-          for (int mm = jj + 1; mm < 16; ++mm) {
-            const float c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lij), P0 + mm));
-            a[mm] = fmaf(-lij, c, a[mm]);
-            xv[mm] = fmaf(-c, xv[jj], xv[mm]);
-          }
-        }
-        if (lane < KP) {
-#pragma unroll
-          for (int jj = 0; jj < 16; ++jj) lLc[(P0 + jj) * KP + lane] = lc[jj];
-        }
-        if (lane >= P0 && lane < P0 + 16) {
-#pragma unroll
-          for (int mm = 0; mm < 16; ++mm) lLt[lane * LP + P0 + mm] = xv[mm];
-        }
+        *(lds_f32x4*)&lX[(16 * p + n) * GS + 16 * p + 4 * g] = invert_block(a, g, n, bad);
       }
       __syncthreads();
-      if (p + 1 < NP16) {
-        // G[16 ti + a][16 tj + b] -= sum_c L[16 ti + a][P0 + c] L[16 tj + b][P0 + c]
-        // over the lower tiles p < tj <= ti < NP16, tile t to wave t mod 4
-        int t = 0;
+      const f32x4 xp = *(const lds_f32x4*)&lX[(16 * p + n) * GS + 16 * p + 4 * g];
+      auto l_t = [&](int q) {  // L_qp[n][4 g + i]
+        const f32x4 gq = *(const lds_f32x4*)&lG[(16 * q + n) * GS + 16 * p + 4 * g];
+        f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ti = p + 1; ti < NP16; ++ti) {
+        for (int r = 0; r < 4; ++r) d = mfma4(xp[r], gq[r], d);
+        return d;
+      };
+      auto update = [&](int ti, int tj) {  // G_ij -= L_ip L_jp^T; a diagonal tile's wave keeps L_ip
+        const f32x4 li = l_t(ti);
+        const f32x4 lj = ti == tj ? li : l_t(tj);
+        f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int tj = p + 1; tj <= ti; ++tj, ++t) {
-            if (t % 4 == wave) {  // wave-uniform
-              f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int r = 0; r < 4; ++r) d = mfma4(lj[r], li[r], d);
+        lds_f32x4* pg = (lds_f32x4*)&lG[(16 * ti + n) * GS + 16 * tj + 4 * g];
+        *pg = *pg - d;
+        if (ti == tj) *(lds_f32x4*)&lL[(16 * ti + n) * GS + 16 * p + 4 * g] = li;
+      };
+      auto x_tile = [&](int r) {  // X_pr
+        f32x4 s_acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-              for (int st = 0; st < 4; ++st) {
-                const int cc = P0 + 4 * st + g;
-                acc = mfma4(lLc[cc * KP + 16 * ti + n], lLc[cc * KP + 16 * tj + n], acc);
-              }
-              lds_f32* pg = lG + (16 * ti + 4 * g) * GP + 16 * tj + n;
+        for (int s = 0; s < NT - 1; ++s) {
+          if (s >= r && s < p) {
+            const f32x4 lv = *(const lds_f32x4*)&lL[(16 * p + n) * GS + 16 * s + 4 * g];
 #pragma unroll
-              for (int i = 0; i < 4; ++i) pg[i * GP] -= acc[i];
-            }
+            for (int i = 0; i < 4; ++i)
+              s_acc = mfma4(lv[i], lX[(16 * s + 4 * g + i) * GS + 16 * r + n], s_acc);
           }
         }
+        f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d = mfma4(xp[i], s_acc[i], d);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lX[(16 * p + 4 * g + i) * GS + 16 * r + n] = -d[i];
+      };
+      if (p + 1 < NT) {
+        if (wave == 0) {
+          update(p + 1, p + 1);
+        } else {
+          int t = 0;
+#pragma unroll
+          for (int ti = p + 1; ti < NT; ++ti)
+#pragma unroll
+            for (int tj = p + 1; tj <= ti; ++tj) {
+              if (ti == p + 1 && tj == p + 1) continue;
+              if (t++ % 3 == wave - 1) update(ti, tj);
+            }
+#pragma unroll
+          for (int r = 0; r < p; ++r)
+            if (t++ % 3 == wave - 1) x_tile(r);
+        }
+      } else if (p > 0) {
+#pragma unroll
+        for (int r = 0; r < p; ++r)
+          if (r % 4 == wave) x_tile(r);
         __syncthreads();
       }
     }
-#pragma unroll
-    for (int q = 1; q < NP16; ++q) {
-      if (wave < q) {  // tile (q, r = wave)
-        const int r = wave;
-        f32x4 tacc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < NP16 - 1; ++s) {
-          if (s >= r && s < q) {  // wave-uniform
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-              const int kk = 16 * s + 4 * st + g;
-              tacc = mfma4(lLc[kk * KP + 16 * q + n], lLt[(16 * r + n) * LP + kk], tacc);
-            }
-          }
-        }
-        lds_f32* pt = lT + wave * 256;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pt[(4 * g + i) * 16 + n] = tacc[i];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        f32x4 xacc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          const int kk = 4 * st + g;
-          xacc = mfma4(lLt[(16 * q + kk) * LP + 16 * q + n], pt[kk * 16 + n], xacc);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) lLt[(16 * r + n) * LP + 16 * q + 4 * g + i] = -xacc[i];
-      }
-      __syncthreads();
-    }
-    }
 
-    // ---- V = W (L^-1)^T on the MFMA: V[r][j] = sum_m W[r][m] (L^-1)^T[m][j],
-    // k assigned as in C V, so one 16-byte read of W's row feeds four steps
-    {
-      const lds_f32* pa = lV + (16 * ti0 + n) * SP + 4 * g;  // W[16 ti + n][16 q + 4 g + r]
-      const lds_f32* pb = lLt + 4 * g * LP + 16 * tj0 + n;   // (L^-1)^T[16 q + 4 g + r][16 tj + n]
-      f32x4 acc[TPW], a[2][TPW];
-      float bv[2][4];
+    // ---- V^T = X W^T (X lower triangular): tile (tj, ti) over q <= tj, W^T
+    // from the registers it was formed in
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tj = 0; tj < NT; ++tj) {
+      vt[tj][0] = vt[tj][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) a[0][t] = *(const lds_f32x4*)&pa[16 * RS * t * SP];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) bv[0][r] = pb[r * LP];
-#pragma unroll
-      for (int q = 0; q < KP / 16; ++q) {
-        const int cur = q & 1, nxt = cur ^ 1;
-        if (q + 1 < KP / 16) {
-#pragma unroll
-          for (int t = 0; t < TPW; ++t) a[nxt][t] = *(const lds_f32x4*)&pa[16 * RS * t * SP + 16 * (q + 1)];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) bv[nxt][r] = pb[(16 * (q + 1) + r) * LP];
-        }
+      for (int q = 0; q <= tj; ++q) {
+        const f32x4 xa = *(const lds_f32x4*)&lX[(16 * tj + n) * GS + 16 * q + 4 * g];
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int t = 0; t < TPW; ++t) acc[t] = mfma4(a[cur][t][r], bv[cur][r], acc[t]);
+          for (int t = 0; t < 2; ++t) vt[tj][t] = mfma4(xa[r], wt[q][t][r], vt[tj][t]);
       }
-      __syncthreads();
-      lds_f32* pw = lV + (16 * ti0 + 4 * g) * SP + 16 * tj0 + n;
-#pragma unroll
-      for (int t = 0; t < TPW; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pw[(16 * RS * t + i) * SP] = acc[t][i];
     }
-    __syncthreads();
+    if (it + 1 < iters) {
+#pragma unroll
+      for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) lV[(16 * tj + 4 * g + i) * VS + 16 * (2 * wave + t) + n] = vt[tj][t][i];
+      __syncthreads();
+    }
   }
 
   if (info && tid == 0) info[bh] = bad ? 1 : 0;  // thread 0 is in wave 0, which ran the pivots
   float* O = out + b * o_sb + (int64_t)h * o_sh;
-  for (int e = tid; e < D * k; e += kThreads) {
-    const int r = e / k, c = e - (e / k) * k;
-    O[r * o_sr + c * o_sc] = sV[r * SP + c];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int row = 16 * (2 * wave + t) + n;
+    if (row < D) {
+#pragma unroll
+      for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (16 * tj + 4 * g + i < k) O[row * o_sr + (16 * tj + 4 * g + i) * o_sc] = vt[tj][t][i];
+    }
   }
 }
 
@@ -756,11 +710,11 @@ __global__ void __launch_bounds__(kThreads) power_iter128_kernel(
 
 template <int KP>
 hipError_t launch(const rk_tensor* cov, const rk_tensor* v0, const rk_tensor* out, int64_t BH, int H, int k,
-                  int iters, float eps, int32_t* info, int D, hipStream_t s) {
+                  int iters, float eps, int32_t* info, int cvec, int D, hipStream_t s) {
   hipLaunchKernelGGL((power_iter_kernel<KP>), dim3((unsigned)BH), dim3(kThreads), 0, s, (const float*)cov->data,
                      cov->stride[0], cov->stride[1], cov->stride[2], cov->stride[3], (const float*)v0->data,
                      v0->stride[0], v0->stride[1], v0->stride[2], v0->stride[3], (float*)out->data, out->stride[0],
-                     out->stride[1], out->stride[2], out->stride[3], H, k, iters, eps, info, D);
+                     out->stride[1], out->stride[2], out->stride[3], H, k, iters, eps, info, cvec, D);
   return hipGetLastError();
 }
 
@@ -787,15 +741,16 @@ extern "C" int rk_power_iteration(const rk_tensor* cov, const rk_tensor* v0, con
   if (!cov->data || !v0->data || !out->data) return RK_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
+  // 16-byte loads of whole rows of C
+  const int cvec = D == kD && cov->stride[3] == 1 && cov->stride[2] % 4 == 0 && cov->stride[1] % 4 == 0 &&
+                   cov->stride[0] % 4 == 0 && (((uintptr_t)cov->data) & 15) == 0;
   if (k <= 16)
-    e = launch<16>(cov, v0, out, B * H, (int)H, (int)k, num_iters, eps, info, (int)D, s);
+    e = launch<16>(cov, v0, out, B * H, (int)H, (int)k, num_iters, eps, info, cvec, (int)D, s);
   else if (k <= 32)
-    e = launch<32>(cov, v0, out, B * H, (int)H, (int)k, num_iters, eps, info, (int)D, s);
+    e = launch<32>(cov, v0, out, B * H, (int)H, (int)k, num_iters, eps, info, cvec, (int)D, s);
   else if (k <= 64)
-    e = launch<64>(cov, v0, out, B * H, (int)H, (int)k, num_iters, eps, info, (int)D, s);
+    e = launch<64>(cov, v0, out, B * H, (int)H, (int)k, num_iters, eps, info, cvec, (int)D, s);
   else {
-    const int cvec = D == kD && cov->stride[3] == 1 && cov->stride[2] % 4 == 0 && cov->stride[1] % 4 == 0 &&
-                     cov->stride[0] % 4 == 0 && (((uintptr_t)cov->data) & 15) == 0;
     hipLaunchKernelGGL(power_iter128_kernel, dim3((unsigned)(B * H)), dim3(kThreads), 0, s, (const float*)cov->data,
                        cov->stride[0], cov->stride[1], cov->stride[2], cov->stride[3], (const float*)v0->data,
                        v0->stride[0], v0->stride[1], v0->stride[2], v0->stride[3], (float*)out->data,
