@@ -105,9 +105,14 @@ __device__ __forceinline__ uint32_t order_key(float v) {
 
 // Channels c0 .. c0 + 7 of row t; channels at or past D read as zeros (no
 // load).  VEC: one 16-byte load (D % 8 == 0, so the group is all in or out).
-template <bool VEC>
+// NT: non-temporal, for rows that this launch reads once.
+template <bool VEC, bool NT = false>
 __device__ __forceinline__ uint4 ld8(const uint16_t* base, int64_t ss, int64_t sc, int64_t t, int c0, int D) {
-  if constexpr (VEC) {
+  if constexpr (VEC && NT) {
+    if (c0 >= D) return make_uint4(0u, 0u, 0u, 0u);
+    const u32x4 v = __builtin_nontemporal_load((const u32x4*)(base + t * ss + c0));
+    return make_uint4(v.x, v.y, v.z, v.w);
+  } else if constexpr (VEC) {
     return c0 < D ? *(const uint4*)(base + t * ss + c0) : make_uint4(0u, 0u, 0u, 0u);
   } else {
     uint32_t w[4] = {0, 0, 0, 0};
@@ -208,7 +213,9 @@ constexpr int kTilePad = 8;   // LDS row padding (elements): 16-byte aligned row
 // grid (splits, B*H): workgroup x sums dtype(k^2) over tokens
 // [x*chunk, (x+1)*chunk) of one head into part[bh][x][128].  Thread (row
 // group rg = t/16, channel chunk c8 = t%16) walks rows rg, rg+16, ...
-template <class TT, bool VEC>
+// NT: Keys larger than the 256 MB memory-side cache, of which the compaction
+// finds nothing there (917 MB: 171 -> 136 us, 6.7 TB/s).
+template <class TT, bool VEC, bool NT>
 __global__ void __launch_bounds__(kThreads) sqsum_kernel(View k, int64_t chunk, int splits, float* part) {
   __shared__ float s_sum[16][kD];
   const int tid = threadIdx.x, rg = tid >> 4, c8 = tid & 15;
@@ -220,7 +227,7 @@ __global__ void __launch_bounds__(kThreads) sqsum_kernel(View k, int64_t chunk, 
   for (int64_t t = t0 + rg; t < t1; t += 64) {
     uint4 v[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = ld8<VEC>(base, k.ss, k.sc, min(t + 16 * i, last), 8 * c8, k.C);
+    for (int i = 0; i < 4; ++i) v[i] = ld8<VEC, NT>(base, k.ss, k.sc, min(t + 16 * i, last), 8 * c8, k.C);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (t + 16 * i < t1) {
@@ -258,23 +265,56 @@ struct ThinkArgs {
   int D;         // head dim (channels past it take no part)
 };
 
-// grid (B*H), 128 threads (one per channel slot).
-template <class TT>
-__global__ void __launch_bounds__(kD) think_select_kernel(const ThinkArgs a) {
+constexpr int kWinThreads = 512;  // 32 window rows x 16 slots of eight channels
+constexpr int kWinRows = 32;
+
+// Eight channels c0.. of one query row (zeros past D), as fp32.
+template <class TT, bool QV>
+__device__ __forceinline__ void query_row8(const View& q, int64_t off, int c0, float (&f)[8]) {
+  const uint4 v = ld8<QV>(q.data + off, 0, q.sc, 0, c0, q.C);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] = TT::to_f32((uint16_t)(word(v, e >> 1) >> ((e & 1) * 16)));
+}
+
+// grid (B*H), 512 threads.  The window's rows are loaded 32 at a time, one
+// row and eight channels a thread, and pass through LDS to the channel's
+// thread, which sums them in row order (one thread per channel with a load per
+// row was a chain of G x 32 memory latencies: B=8, 32 heads 18.8 -> 7.0 us).
+template <class TT, bool QV>
+__global__ void __launch_bounds__(kWinThreads) think_select_kernel(const ThinkArgs a) {
   __shared__ uint32_t s_key[kD];
   __shared__ int s_kept[kD];
-  const int c = threadIdx.x, bh = blockIdx.x, b = bh / a.H, h = bh - b * a.H;
+  __shared__ __align__(16) float s_win[kWinRows][kD + 4];
+  const int tid = threadIdx.x, c = tid, bh = blockIdx.x, b = bh / a.H, h = bh - b * a.H;
+  const int row = tid >> 4, c0 = 8 * (tid & 15);
+  const int64_t W = a.q.S;
   float s = 0.f;
-  for (int x = 0; x < a.splits; ++x) s += a.part[((int64_t)bh * a.splits + x) * kD + c];
+  if (c < kD)
+    for (int x = 0; x < a.splits; ++x) s += a.part[((int64_t)bh * a.splits + x) * kD + c];
   const float kn = rnd<TT>(pin(s * a.f_keys));
   const bool real = c < a.D;
   float qacc = 0.f;
-  for (int gi = 0; gi < (real ? a.G : 0); ++gi) {
-    const uint16_t* qb = a.q.data + head_off(a.q.sb, a.q.sh, b, h * a.G + gi) + c * a.q.sc;
+  for (int gi = 0; gi < a.G; ++gi) {
+    const int64_t qh = head_off(a.q.sb, a.q.sh, b, h * a.G + gi);
     float w = 0.f;
-    for (int64_t t = 0; t < a.q.S; ++t) {
-      const float x = TT::to_f32(qb[t * a.q.ss]);
-      w += rnd<TT>(x * x);
+    for (int64_t w0 = 0; w0 < W; w0 += kWinRows) {
+      if (w0 + row < W) {
+        float f[8];
+        query_row8<TT, QV>(a.q, qh + (w0 + row) * a.q.ss, c0, f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s_win[row][c0 + e] = rnd<TT>(f[e] * f[e]);
+      }
+      __syncthreads();
+      if (c < kD) {
+        const int n = (int)min((int64_t)kWinRows, W - w0);
+        if (n == kWinRows) {
+#pragma unroll
+          for (int t = 0; t < kWinRows; ++t) w += s_win[t][c];
+        } else {
+          for (int t = 0; t < n; ++t) w += s_win[t][c];
+        }
+      }
+      __syncthreads();
     }
     qacc += rnd<TT>(pin(w * a.f_win));
   }
@@ -282,12 +322,14 @@ __global__ void __launch_bounds__(kD) think_select_kernel(const ThinkArgs a) {
   const float score = rnd<TT>(qn * kn);  // product of two 16-bit values: exact in fp32
   // (order keys are >= 0x7F, so a slot past D, key 0, is below every channel)
   const uint32_t key = real ? (order_key<TT>(score) << 7) | (uint32_t)c : 0u;
-  s_key[c] = key;
+  if (c < kD) s_key[c] = key;
   __syncthreads();
   int above = 0;
-  for (int j = 0; j < kD; ++j) above += s_key[j] > key;
+  if (c < kD)
+#pragma unroll 16
+    for (int j = 0; j < kD; ++j) above += s_key[j] > key;
   const int kept = real && above < a.keep;
-  s_kept[c] = kept;
+  if (c < kD) s_kept[c] = kept;
   if (real) a.mask.data[head_off(a.mask.sb, a.mask.sh, b, h) + c * a.mask.sc] = (uint8_t)kept;
   __syncthreads();
   if (kept) {
@@ -298,46 +340,50 @@ __global__ void __launch_bounds__(kD) think_select_kernel(const ThinkArgs a) {
 }
 
 // grid (splits, B*H): K_compact[b,h,t,j] = K[b,h,t,idx[j]].  Tiles of 64
-// tokens are staged in LDS with 16-byte loads (thread t loads channels
-// 8(t%16).. of rows t/16 + 16i); thread t then gathers output columns
-// 8(t%16)..+7 of the same rows from LDS (threads past Dk idle).  OVEC: one
-// 16-byte store per chunk (unit stride, aligned rows, Dk % 8 == 0).
+// tokens go through LDS: thread t loads channels 8(t%16).. of rows
+// t/16 + 16i with 16-byte loads (the next tile's are in flight while this
+// one is gathered), and the tile's 64 x ceil(Dk/8) output slots of eight
+// channels are shared out over all threads.  OVEC: one 16-byte store per
+// slot (unit stride, aligned rows, Dk % 8 == 0).
 template <bool VEC, bool OVEC>
 __global__ void __launch_bounds__(kThreads) compact_kernel(View k, const int32_t* idx, int Dk, int64_t chunk,
                                                            OutView o) {
   __shared__ __align__(16) uint16_t s_k[kTile * (kD + kTilePad)];
+  __shared__ int s_src[kD];
   const int tid = threadIdx.x, c8 = tid & 15, rq = tid >> 4;
   const int x = blockIdx.x, bh = blockIdx.y, b = bh / k.H, h = bh - b * k.H;
-  int src[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) src[e] = 8 * c8 + e < Dk ? idx[(int64_t)bh * kD + 8 * c8 + e] : 0;
+  if (tid < kD) s_src[tid] = tid < Dk ? idx[(int64_t)bh * kD + tid] : 0;
   const uint16_t* base = k.data + head_off(k.sb, k.sh, b, h);
   uint16_t* ob = o.data + head_off(o.sb, o.sh, b, h);
   const int64_t t0 = (int64_t)x * chunk, t1 = min(k.S, t0 + chunk);
+  const int nslot = (Dk + 7) >> 3;  // 1..16 slots per token
+  auto load = [&](uint4 (&v)[kTile / 16], int64_t tile) {  // rows past the end re-read the last one
+#pragma unroll
+    for (int i = 0; i < kTile / 16; ++i)
+      v[i] = ld8<VEC, true>(base, k.ss, k.sc, min(tile + rq + 16 * i, t1 - 1), 8 * c8, k.C);
+  };
+  uint4 cur[kTile / 16];
+  if (t0 < t1) load(cur, t0);
+  __syncthreads();
   for (int64_t tile = t0; tile < t1; tile += kTile) {
 #pragma unroll
-    for (int i = 0; i < kTile / 16; ++i) {
-      const int64_t t = tile + rq + 16 * i;
-      if (t < t1)
-        *(uint4*)(s_k + (rq + 16 * i) * (kD + kTilePad) + 8 * c8) = ld8<VEC>(base, k.ss, k.sc, t, 8 * c8, k.C);
-    }
+    for (int i = 0; i < kTile / 16; ++i) *(uint4*)(s_k + (rq + 16 * i) * (kD + kTilePad) + 8 * c8) = cur[i];
     __syncthreads();
-    if (8 * c8 < Dk) {
+    if (tile + kTile < t1) load(cur, tile + kTile);
+    const int rows = (int)min((int64_t)kTile, t1 - tile);
+    for (int it = tid; it < rows * nslot; it += kThreads) {
+      const int t = it / nslot, sl = it - t * nslot;
+      const uint16_t* row = s_k + t * (kD + kTilePad);
+      uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int i = 0; i < kTile / 16; ++i) {
-        const int64_t t = tile + rq + 16 * i;
-        if (t >= t1) continue;
-        const uint16_t* row = s_k + (rq + 16 * i) * (kD + kTilePad);
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
+      for (int e = 0; e < 8; ++e) w[e >> 1] |= (uint32_t)row[s_src[8 * sl + e]] << ((e & 1) * 16);
+      uint16_t* dst = ob + (tile + t) * o.ss;
+      if constexpr (OVEC) {
+        *(uint4*)(dst + 8 * sl) = make_uint4(w[0], w[1], w[2], w[3]);
+      } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) w[e >> 1] |= (uint32_t)row[src[e]] << ((e & 1) * 16);
-        if constexpr (OVEC) {
-          *(uint4*)(ob + t * o.ss + 8 * c8) = make_uint4(w[0], w[1], w[2], w[3]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (8 * c8 + e < Dk) ob[t * o.ss + (8 * c8 + e) * o.sc] = (uint16_t)(w[e >> 1] >> ((e & 1) * 16));
-        }
+        for (int e = 0; e < 8; ++e)
+          if (8 * sl + e < Dk) dst[(8 * sl + e) * o.sc] = (uint16_t)(w[e >> 1] >> ((e & 1) * 16));
       }
     }
     __syncthreads();
@@ -345,19 +391,47 @@ __global__ void __launch_bounds__(kThreads) compact_kernel(View k, const int32_t
 }
 
 // ------------------------------------------------------------------ SparK
-// grid (B*H), 128 threads: qn[bh][c] = dtype(sqrt(sum_t q_g[t][c]^2)) with
-// q_g[t][c] = dtype(sum over the G query heads * f_grp).
-template <class TT>
-__global__ void __launch_bounds__(kD) spark_qnorm_kernel(View q, int G, int H, float f_grp, float* qn) {
-  const int c = threadIdx.x, bh = blockIdx.x, b = bh / H, h = bh - b * H;
+// grid (B*H), 512 threads: qn[bh][c] = dtype(sqrt(sum_t q_g[t][c]^2)) with
+// q_g[t][c] = dtype(sum over the G query heads * f_grp).  A thread forms the
+// group means of one window row's eight channels, kHeads rows in flight;
+// the channel's thread sums their squares in row order (B=16, 4 KV heads
+// of 7 query heads: 101 us with one thread per channel, 7.9 now).
+template <class TT, bool QV>
+__global__ void __launch_bounds__(kWinThreads) spark_qnorm_kernel(View q, int G, int H, float f_grp, float* qn) {
+  constexpr int kHeads = 4;
+  __shared__ __align__(16) float s_win[kWinRows][kD + 4];
+  const int tid = threadIdx.x, c = tid, bh = blockIdx.x, b = bh / H, h = bh - b * H;
+  const int row = tid >> 4, c0 = 8 * (tid & 15);
+  const int64_t W = q.S;
   float acc = 0.f;
-  for (int64_t t = 0; t < (c < q.C ? q.S : 0); ++t) {
-    float s = 0.f;
-    for (int gi = 0; gi < G; ++gi) s += TT::to_f32(q.data[head_off(q.sb, q.sh, b, h * G + gi) + t * q.ss + c * q.sc]);
-    const float g = rnd<TT>(pin(s * f_grp));
-    acc = fmaf(g, g, acc);  // g * g is exact, so fused or not gives the same sum
+  for (int64_t w0 = 0; w0 < W; w0 += kWinRows) {
+    if (w0 + row < W) {
+      float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int g0 = 0; g0 < G; g0 += kHeads) {
+        float f[kHeads][8];
+#pragma unroll
+        for (int u = 0; u < kHeads; ++u)
+          query_row8<TT, QV>(q, head_off(q.sb, q.sh, b, h * G + min(g0 + u, G - 1)) + (w0 + row) * q.ss, c0, f[u]);
+#pragma unroll
+        for (int u = 0; u < kHeads; ++u)
+          if (g0 + u < G)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] += f[u][e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s_win[row][c0 + e] = rnd<TT>(pin(s[e] * f_grp));
+    }
+    __syncthreads();
+    if (c < kD) {
+      const int n = (int)min((int64_t)kWinRows, W - w0);
+      for (int t = 0; t < n; ++t) {
+        const float g = s_win[t][c];
+        acc = fmaf(g, g, acc);  // g * g is exact, so fused or not gives the same sum
+      }
+    }
+    __syncthreads();
   }
-  qn[(int64_t)bh * kD + c] = rnd<TT>(sqrtf(acc));
+  if (c < kD) qn[(int64_t)bh * kD + c] = rnd<TT>(sqrtf(acc));
 }
 
 struct SparkArgs {
@@ -741,6 +815,9 @@ size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 using rk::mean_factor;
 
+// Bytes of the memory-side cache: larger Keys are streamed.
+constexpr int64_t kMallBytes = INT64_C(256) << 20;
+
 // [B, H, S, C] descriptor of a 16-bit float tensor: a head dim 1 <= C <=
 // 128 (want_c == 0), C == want_c (> 0), or any C <= 128 (want_c < 0).
 int view_of(const rk_tensor* t, int want_c, View* v) {
@@ -864,17 +941,19 @@ int think_check(const rk_tensor* keys, const rk_tensor* queries, int64_t num_kv_
 }
 
 template <class TT>
-hipError_t launch_think(const View& kv, bool kvec, const View& qv, int G, int keep, const ThinkPlan& p, int64_t B,
-                        float f_keys, float f_win, float f_grp, const MaskView& mv, const rk_tensor* kc_out,
+hipError_t launch_think(const View& kv, bool kvec, const View& qv, bool qvec, int G, int keep, const ThinkPlan& p, int cus,
+                        int64_t B, float f_keys, float f_win, float f_grp, const MaskView& mv, const rk_tensor* kc_out,
                         void* ws, hipStream_t s) {
   const int64_t bh = B * kv.H;
   float* part = (float*)((char*)ws + p.off_part);
   int32_t* idx = (int32_t*)((char*)ws + p.off_idx);
   const dim3 grid((unsigned)p.splits, (unsigned)bh);
-  if (kvec)
-    hipLaunchKernelGGL((sqsum_kernel<TT, true>), grid, dim3(kThreads), 0, s, kv, p.chunk, p.splits, part);
+  if (kvec && bh * kv.S * kv.C * 2 > kMallBytes)
+    hipLaunchKernelGGL((sqsum_kernel<TT, true, true>), grid, dim3(kThreads), 0, s, kv, p.chunk, p.splits, part);
+  else if (kvec)
+    hipLaunchKernelGGL((sqsum_kernel<TT, true, false>), grid, dim3(kThreads), 0, s, kv, p.chunk, p.splits, part);
   else
-    hipLaunchKernelGGL((sqsum_kernel<TT, false>), grid, dim3(kThreads), 0, s, kv, p.chunk, p.splits, part);
+    hipLaunchKernelGGL((sqsum_kernel<TT, false, false>), grid, dim3(kThreads), 0, s, kv, p.chunk, p.splits, part);
   ThinkArgs a;
   a.part = part;
   a.splits = p.splits;
@@ -888,18 +967,27 @@ hipError_t launch_think(const View& kv, bool kvec, const View& qv, int G, int ke
   a.mask = mv;
   a.idx = idx;
   a.D = kv.C;
-  hipLaunchKernelGGL((think_select_kernel<TT>), dim3((unsigned)bh), dim3(kD), 0, s, a);
+  if (qvec)
+    hipLaunchKernelGGL((think_select_kernel<TT, true>), dim3((unsigned)bh), dim3(kWinThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((think_select_kernel<TT, false>), dim3((unsigned)bh), dim3(kWinThreads), 0, s, a);
   if (keep > 0 && kv.S > 0) {
+    // two rounds of eight workgroups per CU, whatever the sums were split
+    // into: 917 MB of Keys, keep 32, 326 us in the sums' one round of two per
+    // CU (with four of sixteen threads storing), 204 at eight per CU, 200 now
+    const int csplits = token_splits(bh, kv.S, cus, 16, 256);
+    const int64_t cchunk = cdiv(cdiv(kv.S, csplits), kTile) * kTile;
+    const dim3 cgrid((unsigned)cdiv(kv.S, cchunk), (unsigned)bh);
     const OutView o = out_of(kc_out);
     const bool ovec = rows16(kc_out) && keep % 8 == 0;
     if (kvec && ovec)
-      hipLaunchKernelGGL((compact_kernel<true, true>), grid, dim3(kThreads), 0, s, kv, idx, keep, p.chunk, o);
+      hipLaunchKernelGGL((compact_kernel<true, true>), cgrid, dim3(kThreads), 0, s, kv, idx, keep, cchunk, o);
     else if (kvec)
-      hipLaunchKernelGGL((compact_kernel<true, false>), grid, dim3(kThreads), 0, s, kv, idx, keep, p.chunk, o);
+      hipLaunchKernelGGL((compact_kernel<true, false>), cgrid, dim3(kThreads), 0, s, kv, idx, keep, cchunk, o);
     else if (ovec)
-      hipLaunchKernelGGL((compact_kernel<false, true>), grid, dim3(kThreads), 0, s, kv, idx, keep, p.chunk, o);
+      hipLaunchKernelGGL((compact_kernel<false, true>), cgrid, dim3(kThreads), 0, s, kv, idx, keep, cchunk, o);
     else
-      hipLaunchKernelGGL((compact_kernel<false, false>), grid, dim3(kThreads), 0, s, kv, idx, keep, p.chunk, o);
+      hipLaunchKernelGGL((compact_kernel<false, false>), cgrid, dim3(kThreads), 0, s, kv, idx, keep, cchunk, o);
   }
   return hipGetLastError();
 }
@@ -940,13 +1028,16 @@ int spark_check(const rk_tensor* keys, const rk_tensor* queries, int64_t num_kv_
 }
 
 template <class TT>
-hipError_t launch_spark(const View& kv, bool kvec, bool mvec, const View& qv, int G, int keep, const SparkPlan& p,
+hipError_t launch_spark(const View& kv, bool kvec, bool mvec, const View& qv, bool qvec, int G, int keep, const SparkPlan& p,
                         int64_t B,
                         float f_grp, float f_pruned, const MaskView& mv, const rk_tensor* kc_out,
                         const rk_tensor* pm_out, void* ws, hipStream_t s) {
   const int64_t bh = B * kv.H;
   float* qn = (float*)ws;
-  hipLaunchKernelGGL((spark_qnorm_kernel<TT>), dim3((unsigned)bh), dim3(kD), 0, s, qv, G, kv.H, f_grp, qn);
+  if (qvec)
+    hipLaunchKernelGGL((spark_qnorm_kernel<TT, true>), dim3((unsigned)bh), dim3(kWinThreads), 0, s, qv, G, kv.H, f_grp, qn);
+  else
+    hipLaunchKernelGGL((spark_qnorm_kernel<TT, false>), dim3((unsigned)bh), dim3(kWinThreads), 0, s, qv, G, kv.H, f_grp, qn);
   if (kv.S == 0) return hipGetLastError();
   SparkArgs a;
   a.k = kv;
@@ -1090,12 +1181,12 @@ extern "C" int rk_think_score_and_compact(const rk_tensor* keys_vision, const rk
   const float f_keys = mean_factor(B * H * D, B * H * kv.S * D);
   const float f_win = mean_factor(B * Hq * D, B * Hq * qv.S * D);
   const float f_grp = mean_factor(B * H * D, B * Hq * D);
-  const bool kvec = rows16(keys_vision) && D % 8 == 0;
+  const bool kvec = rows16(keys_vision) && D % 8 == 0, qvec = rows16(queries_recent) && D % 8 == 0;
   hipStream_t s = (hipStream_t)stream;
   const hipError_t e = keys_vision->dtype == RK_F16
-                           ? launch_think<rk::F16>(kv, kvec, qv, G, (int)keep, p, B, f_keys, f_win, f_grp, mv,
+                           ? launch_think<rk::F16>(kv, kvec, qv, qvec, G, (int)keep, p, cus, B, f_keys, f_win, f_grp, mv,
                                                    k_compact_out, workspace, s)
-                           : launch_think<rk::BF16>(kv, kvec, qv, G, (int)keep, p, B, f_keys, f_win, f_grp, mv,
+                           : launch_think<rk::BF16>(kv, kvec, qv, qvec, G, (int)keep, p, cus, B, f_keys, f_win, f_grp, mv,
                                                     k_compact_out, workspace, s);
   return e == hipSuccess ? RK_OK : RK_ERR_HIP;
 }
@@ -1138,16 +1229,16 @@ extern "C" int rk_spark_prune(const rk_tensor* keys_vision, const rk_tensor* que
   const int64_t W = qv.S, D = kv.C;
   const float f_grp = mean_factor(B * H * W * D, B * H * num_kv_groups * W * D);
   const float f_pruned = mean_factor(B * H * kv.S, B * H * kv.S * prune_count);
-  const bool kvec = rows16(keys_vision) && D % 8 == 0;
+  const bool kvec = rows16(keys_vision) && D % 8 == 0, qvec = rows16(queries) && D % 8 == 0;
   const bool mvec = D % 8 == 0 && keep_mask_out->stride[3] == 1 && keep_mask_out->stride[0] % 8 == 0 &&
                     keep_mask_out->stride[1] % 8 == 0 && keep_mask_out->stride[2] % 8 == 0 &&
                     (((uintptr_t)keep_mask_out->data) & 7) == 0;
   hipStream_t s = (hipStream_t)stream;
   const hipError_t e =
       keys_vision->dtype == RK_F16
-          ? launch_spark<rk::F16>(kv, kvec, mvec, qv, (int)num_kv_groups, (int)keep, p, B, f_grp, f_pruned, mv,
+          ? launch_spark<rk::F16>(kv, kvec, mvec, qv, qvec, (int)num_kv_groups, (int)keep, p, B, f_grp, f_pruned, mv,
                                   k_compact_out, pruned_mean_out, workspace, s)
-          : launch_spark<rk::BF16>(kv, kvec, mvec, qv, (int)num_kv_groups, (int)keep, p, B, f_grp, f_pruned, mv,
+          : launch_spark<rk::BF16>(kv, kvec, mvec, qv, qvec, (int)num_kv_groups, (int)keep, p, B, f_grp, f_pruned, mv,
                                    k_compact_out, pruned_mean_out, workspace, s);
   return e == hipSuccess ? RK_OK : RK_ERR_HIP;
 }
