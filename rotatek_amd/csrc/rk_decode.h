@@ -52,6 +52,14 @@ struct DecodeArgs {
   int64_t vs_sb, vs_sh;
   int64_t o_sb, o_sh, o_sd;
   int64_t S_v, S_f, chunk_vis, chunk_full;
+  // SparK-pruned visual Keys (ks holds each token's kept channels): the
+  // per-token keep mask [B, H_kv, S_v, 128] (rows of 16-byte aligned bytes)
+  // and the pruned channels' mean [B, H_kv, S_v]
+  const uint8_t* sm;
+  int64_t sm_sb, sm_sh;
+  const uint16_t* pm;
+  int64_t pm_sb, pm_sh;
+  uint32_t sm_ss, pm_ss;
   // within-head strides (elements); a head's span is < 2^31 elements
   uint32_t kf_ss, kf_sd, vf_ss, vf_sd, ks_ss, ks_sd, vs_ss, vs_sd;
   int32_t G, Dk, hpu, spk, units_per_b, wg_vis, np, rot_x;
@@ -96,6 +104,10 @@ hipError_t decode_launch_f16_hd(int dkb, int hmax, bool has_vis, const DecodeArg
 hipError_t decode_launch_bf16_hd(int dkb, int hmax, bool has_vis, const DecodeArgs& a, dim3 grid, hipStream_t s);
 // The same for fp32 q / K / V (the VALU kernel, one query head per unit).
 hipError_t decode_launch_f32(bool has_vis, bool vec, const DecodeArgs& a, dim3 grid, hipStream_t s);
+
+// SparK-pruned visual Keys at head_dim 128, 16-byte rows, at most 64 kept
+// channels (kb = ceil(Dk / 32)): both 16-bit types (rk_decode_spark.hip).
+hipError_t decode_launch_spark(int dtype, int kb, int hmax, const DecodeArgs& a, dim3 grid, hipStream_t s);
 
 // Workgroups of the merge kernel: one per unit, or one per 16 units of one
 // query head each (merge_kernel's sliced form).

@@ -525,6 +525,14 @@ int32_t decode_policy(const Checked& c, bool has_vis, int32_t policy, int cus) {
   return RK_POLICY_GQA;
 }
 
+// The plan over SparK-pruned visual Keys: their 128 mask bytes a token count
+// as 64 more channels.
+int plan_spark(const Checked& c, int32_t policy, int cus, rk_decode_plan* p) {
+  Checked w = c;
+  w.Dk += 64;
+  return plan_for(w, true, policy, cus, p);
+}
+
 int resolve_cus(int32_t num_cus, int* st) {
   *st = RK_OK;
   if (num_cus > 0) return num_cus;
@@ -567,18 +575,19 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
                const rk_tensor* ks, const rk_tensor* vs, const rk_tensor* out, int32_t policy,
                void* ws, size_t ws_bytes, void* stream, bool has_vis,
                int32_t* len_full = nullptr, int64_t v_gap_at = -1, int64_t v_gap = 0,
-               const rk_tensor* k_new = nullptr, const rk_tensor* v_new = nullptr) {
+               const rk_tensor* k_new = nullptr, const rk_tensor* v_new = nullptr,
+               const rk_tensor* sm = nullptr, const rk_tensor* pm = nullptr) {
   int st = RK_OK;
   const int cus = resolve_cus(0, &st);
   if (st) return st;
   policy = decode_policy(c, has_vis, policy, cus);
   rk_decode_plan p;
-  st = plan_for(c, has_vis, policy, cus, &p);
+  st = sm ? plan_spark(c, policy, cus, &p) : plan_for(c, has_vis, policy, cus, &p);
   if (st) return st;
   if (!ws || (((uintptr_t)ws) & 255) != 0 || ws_bytes < p.workspace_bytes) return RK_ERR_WORKSPACE;
   if (c.B == 0) return RK_OK;
   const bool vis_work = has_vis && c.S_v > 0;
-  if (!q->data || !out->data || (vis_work && ((c.Dk > 0 && (!R->data || !ks->data)) || !vs->data)) ||
+  if (!q->data || !out->data || (vis_work && ((c.Dk > 0 && ((!sm && !R->data) || !ks->data)) || !vs->data)) ||
       (c.S_f > 0 && (!kf->data || !vf->data)))
     return RK_ERR_NULL;
   const WsLayout w = ws_layout(p);
@@ -614,7 +623,18 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
   a.q_vec = q->stride[2] == 1 && q->stride[1] % 8 == 0 && q->stride[0] % 8 == 0 &&
             (((uintptr_t)q->data) & 15) == 0 && c.D % 8 == 0;
   int dkb = 1;
+  if (sm) {
+    a.sm = (const uint8_t*)sm->data;
+    a.sm_sb = sm->stride[0];
+    a.sm_sh = sm->stride[1];
+    a.sm_ss = (uint32_t)sm->stride[2];
+    a.pm = (const uint16_t*)pm->data;
+    a.pm_sb = pm->stride[0];
+    a.pm_sh = pm->stride[1];
+    a.pm_ss = (uint32_t)pm->stride[2];
+  }
   if (has_vis) {
+    if (!sm) {
     a.R = R->data;
     a.r_dtype = R->dtype;
     set4(R, a.R_sb, a.R_sh, a.R_sd, a.R_sk);
@@ -633,6 +653,7 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
     a.r_vec = rk::is_half(R->dtype) && (c.Dk <= 64 || (c.Dk <= 128 && R->dtype == c.dtype)) &&
               R->stride[3] == 1 && R->stride[2] == c.Dk && (c.D * c.Dk) % 8 == 0 &&
               R->stride[1] % 8 == 0 && R->stride[0] % 8 == 0 && (((uintptr_t)R->data) & 15) == 0;
+    }
     a.ks = (const uint16_t*)ks->data;
     a.vs = (const uint16_t*)vs->data;
     if (!set_head(vs, a.vs_sb, a.vs_sh, a.vs_ss, a.vs_sd)) return RK_ERR_STRIDE;
@@ -724,7 +745,9 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
     return rk::decode_launch_f32(has_vis, v32, a, grid, s) == hipSuccess ? RK_OK : RK_ERR_HIP;
   }
   hipError_t e;
-  if (vec && c.D < 128)  // 16-byte loads with the channels past D masked
+  if (sm)
+    e = rk::decode_launch_spark(c.dtype, dkb, hmax, a, grid, s);
+  else if (vec && c.D < 128)  // 16-byte loads with the channels past D masked
     e = c.dtype == RK_F16 ? rk::decode_launch_f16_hd(dkb, hmax, has_vis, a, grid, s)
                           : rk::decode_launch_bf16_hd(dkb, hmax, has_vis, a, grid, s);
   else
@@ -936,6 +959,106 @@ extern "C" int rk_full_channel_decode(const rk_tensor* q, const rk_tensor* k, co
   if (policy != RK_POLICY_PAPER && policy != RK_POLICY_GQA) return RK_ERR_ARG;
   return run_decode(c, q, nullptr, nullptr, k, v, nullptr, nullptr, nullptr, out, policy, workspace,
                     workspace_bytes, stream, false);
+}
+
+// ---- decode over ThinK / SparK pruned Keys, without recovering them
+
+namespace {
+
+// What the fused form takes; everything else is recovered first
+// (rk_think_recover / rk_spark_recover, then rk_full_channel_decode).
+int check_recovered(const rk_tensor* q, const rk_tensor* R, const rk_tensor* k_full, const rk_tensor* v_buf,
+                    int64_t v_gap_at, int64_t v_gap, const rk_tensor* mask, const rk_tensor* pm, const rk_tensor* ks,
+                    const rk_tensor* vs, int64_t G, const rk_tensor* out, int32_t policy, rk_tensor* v_logical,
+                    rk_tensor* r_shape, Checked* c) {
+  if (!k_full || !v_buf || !ks || !q || !out || (!R == !mask) || (!mask != !pm)) return RK_ERR_NULL;
+  int st;
+  if ((st = rk::check_desc(v_buf, 4)) || (st = rk::check_desc(k_full, 4)) || (st = rk::check_desc(ks, 4))) return st;
+  const int64_t S_f = k_full->shape[2];
+  if (v_gap < 0 || v_gap_at < 0 || v_gap_at > S_f || v_gap >= (INT64_C(1) << 31)) return RK_ERR_ARG;
+  if (v_buf->shape[2] != S_f + v_gap) return RK_ERR_SHAPE;
+  if (!head_span_ok(v_buf)) return RK_ERR_STRIDE;
+  *v_logical = *v_buf;
+  v_logical->shape[2] = S_f;
+  if (!R) {  // SparK has no rotation: stand in its shape for the checks
+    memset(r_shape, 0, sizeof(*r_shape));
+    r_shape->dtype = ks->dtype;
+    r_shape->ndim = 4;
+    r_shape->shape[0] = ks->shape[0];
+    r_shape->shape[1] = ks->shape[1];
+    r_shape->shape[2] = q->ndim == 3 ? q->shape[2] : 0;
+    r_shape->shape[3] = ks->shape[3];
+    R = r_shape;
+  }
+  if ((st = check_rotatek(q, R, nullptr, k_full, v_logical, nullptr, ks, vs, G, c))) return st;
+  if ((st = check_out(out, *c))) return st;
+  if (policy != RK_POLICY_PAPER && policy != RK_POLICY_GQA) return RK_ERR_ARG;
+  if (c->dtype == RK_F32) return RK_ERR_DTYPE;
+  if (c->B == 0 || c->S_v == 0 || c->Dk == 0) return RK_ERR_SHAPE;
+  if (!mask) return RK_OK;
+  // SparK: head_dim 128, at most 64 kept channels (a block of more does not
+  // fit the ring's registers), 16-byte rows of everything
+  if (c->D != 128) return RK_ERR_HEAD_DIM;
+  if (c->Dk > 64 || c->Dk % 8 != 0) return RK_ERR_KEEP_DIM;
+  if ((st = rk::check_desc(mask, 4)) || (st = rk::check_desc(pm, 4))) return st;
+  if (mask->dtype != RK_U8 || pm->dtype != c->dtype) return RK_ERR_DTYPE;
+  for (int i = 0; i < 3; ++i)
+    if (mask->shape[i] != ks->shape[i] || pm->shape[i] != ks->shape[i]) return RK_ERR_SHAPE;
+  if (mask->shape[3] != 128 || pm->shape[3] != 1) return RK_ERR_SHAPE;
+  if (!mask->data || !pm->data) return RK_ERR_NULL;
+  if (mask->stride[3] != 1 || mask->stride[2] >= (INT64_C(1) << 26) || pm->stride[2] >= (INT64_C(1) << 26) ||
+      (c->S_v + 32) * mask->stride[2] >= (INT64_C(1) << 31) || (c->S_v + 32) * pm->stride[2] >= (INT64_C(1) << 31))
+    return RK_ERR_STRIDE;
+  for (int i = 0; i < 3; ++i)
+    if (mask->shape[i] > 1 && mask->stride[i] % 16 != 0) return RK_ERR_STRIDE;
+  if ((((uintptr_t)mask->data) & 15) || !rk::vec_ok(k_full) || !rk::vec_ok(v_buf) || !rk::vec_ok(ks) ||
+      !rk::vec_ok(vs))
+    return RK_ERR_STRIDE;
+  return RK_OK;
+}
+
+}  // namespace
+
+extern "C" int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* R_select, const rk_tensor* zero_bias,
+                                         const rk_tensor* k_full, const rk_tensor* v_buf, int64_t v_gap_at,
+                                         int64_t v_gap, const rk_tensor* spark_mask, const rk_tensor* pruned_mean,
+                                         const rk_tensor* k_pruned, const rk_tensor* v_sparse, int64_t num_kv_groups,
+                                         const rk_tensor* out, int32_t policy, int32_t num_cus,
+                                         size_t* workspace_bytes) {
+  Checked c;
+  rk_tensor vl, rs;
+  (void)zero_bias;
+  int st = check_recovered(q, R_select, k_full, v_buf, v_gap_at, v_gap, spark_mask, pruned_mean, k_pruned, v_sparse,
+                           num_kv_groups, out, policy, &vl, &rs, &c);
+  if (st) return st;
+  const int cus = resolve_cus(num_cus, &st);
+  if (st) return st;
+  rk_decode_plan p;
+  policy = decode_policy(c, true, policy, cus);
+  if ((st = spark_mask ? plan_spark(c, policy, cus, &p) : plan_for(c, true, policy, cus, &p))) return st;
+  if (workspace_bytes) *workspace_bytes = p.workspace_bytes;
+  return RK_OK;
+}
+
+extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* R_select, const rk_tensor* zero_bias,
+                                   const rk_tensor* k_full, const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
+                                   const rk_tensor* spark_mask, const rk_tensor* pruned_mean,
+                                   const rk_tensor* k_pruned, const rk_tensor* v_sparse, int64_t num_kv_groups,
+                                   const rk_tensor* out, int32_t policy, void* workspace, size_t workspace_bytes,
+                                   void* stream) {
+  Checked c;
+  rk_tensor vl, rs;
+  int st = check_recovered(q, R_select, k_full, v_buf, v_gap_at, v_gap, spark_mask, pruned_mean, k_pruned, v_sparse,
+                           num_kv_groups, out, policy, &vl, &rs, &c);
+  if (st) return st;
+  if (zero_bias) {
+    if ((st = rk::check_desc(zero_bias, 3))) return st;
+    if (!rk::is_float_param(zero_bias->dtype)) return RK_ERR_DTYPE;
+    if (zero_bias->shape[0] != c.B || zero_bias->shape[1] != c.H_kv || zero_bias->shape[2] != c.D) return RK_ERR_SHAPE;
+  }
+  return run_decode(c, q, R_select, zero_bias, k_full, v_buf, nullptr, k_pruned, v_sparse, out, policy, workspace,
+                    workspace_bytes, stream, true, nullptr, v_gap > 0 ? v_gap_at : -1, v_gap, nullptr, nullptr,
+                    spark_mask, pruned_mean);
 }
 
 // ---- allocation-free decode (rk_rotatek_decode_noalloc)

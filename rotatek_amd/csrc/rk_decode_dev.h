@@ -228,6 +228,54 @@ struct FullBuf {
   uint4 v[8];
 };
 
+// SparK visual block: the kept values of its 32 rows (16-byte slots shared
+// out over the wave), the mask bytes and fill of the lane's two score rows,
+// and the V rows.
+template <int KB>
+struct SparkBuf {
+  uint4 c[2 * KB];
+  uint4 m[2][2];
+  uint32_t f[2];
+  uint4 v[8];
+};
+
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+
+// Bit e set when mask byte e (of 32) is not zero.
+__device__ __forceinline__ uint32_t mask_bits32(const uint4 (&m)[2]) {
+  uint32_t out = 0u;
+#pragma unroll
+  for (int d = 0; d < 8; d += 2) {
+    uint32_t byte = 0u;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t w = word(m[d >> 2], (d + j) & 3);
+      const uint32_t nz = ((((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) >> 7) & 0x01010101u;
+      byte = __builtin_amdgcn_udot4(nz, j ? 0x80402010u : 0x08040201u, byte, false);
+    }
+    out |= byte << (4 * d);
+  }
+  return out;
+}
+
+// Eight channels' worth of MFMA operand words: the next of the row's kept
+// values (at LDS address `at`, which moves on) where the mask has a bit,
+// the fill elsewhere.
+__device__ __forceinline__ uint4 expand8(uint32_t bits, int e0, const lds_u16*& at, uint32_t fill2) {
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int b0 = __builtin_amdgcn_sbfe(bits, e0 + 2 * i, 1), b1 = __builtin_amdgcn_sbfe(bits, e0 + 2 * i + 1, 1);
+    const uint32_t lo = at[0];
+    at -= b0;
+    const uint32_t hi = at[0];
+    at -= b1;
+    const uint32_t m2 = ((uint32_t)b0 & 0xffffu) | ((uint32_t)b1 & 0xffff0000u);
+    w[i] = ((lo | (hi << 16)) & m2) | (fill2 & ~m2);
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 // ---- partial records and their merge
 //   out = sum_p acc_p 2^(m_p - M) / (sum_p l_p 2^(m_p - M) + 1e-6),
 //   M = max_p m_p                                  (fused_decode.py:275-296)
@@ -516,7 +564,11 @@ __device__ __forceinline__ void merge_fused(const DecodeArgs& a, int u, int b, i
 // (a.fused set).  A separate instantiation: inlined into every
 // kernel, the merge's code raised the split pass's register pressure
 // enough to spill scalar registers in its loops.
-template <class TT, int DKB, bool VEC, int HMAX, bool HAS_VIS, bool APPEND, bool DPART = false, bool FUSED = false>
+// SPK: the visual Keys are SparK's (kept channels per token, mask, mean of
+// the others): the workgroup puts each block's rows back together in
+// registers as score operands instead of reading recovered Keys.
+template <class TT, int DKB, bool VEC, int HMAX, bool HAS_VIS, bool APPEND, bool DPART = false, bool FUSED = false,
+          bool SPK = false>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 decode_kernel(const DecodeArgs a) {
   static_assert(!DPART || VEC, "the element-wise kernels mask head_dim at run time");
@@ -543,7 +595,11 @@ decode_kernel(const DecodeArgs a) {
   // partial sums; all of it for 65-128 channels, whose q R runs on the MFMA
   // with no partial sums), else its own
   constexpr int kRawChunks = DKB == 4 ? 2048 : 1024;
-  __shared__ uint4 s_rsep[HMAX >= 16 ? 1 : kRawChunks];
+  __shared__ uint4 s_rsep[HMAX >= 16 || SPK ? 1 : kRawChunks];
+  // SPK: a block's kept values per wave, rows 16 bytes apart (a read may
+  // pass a row's last value by one)
+  constexpr int kCmpRow = 64 * DKB + 16;  // bytes, at the largest Dk
+  __shared__ __align__(16) char s_cmp[SPK ? kWaves * kBlk * kCmpRow : 16];
 
   const int tid = threadIdx.x;
   // wave index in a scalar register: the ring's block bookkeeping (block
@@ -659,7 +715,114 @@ decode_kernel(const DecodeArgs a) {
     }
   };
 
-  if (is_vis) {
+  if (SPK && is_vis) {
+    // ---- visual span, SparK: lane (g, n) brings channels 32g .. 32g + 31 of
+    // its two score rows (k-step kb of the score products takes 32g + 8kb ..
+    // + 7 from it, and from q alike).  The kept values of those channels are
+    // consecutive in the row, from the number kept in the lanes below; they
+    // are read one by one from LDS and merged with the fill by the mask.
+    // Bound by memory like the other paths: about 380 vector and 70 LDS
+    // instructions per 32 tokens and wave, under its 15 KB of loads.  B=8, 32
+    // heads, 14000 tokens, keep 32 (fp16), with 2000 prompt/text tokens:
+    // 746 us recovering the Keys and attending them, 333 here (5.7 TB/s).
+    const int64_t t_begin = x < a.nfast ? (int64_t)x * a.chunk_fast
+                                        : (int64_t)a.nfast * a.chunk_fast + (int64_t)(x - a.nfast) * a.chunk_vis;
+    const int64_t t_end = min(a.S_v, t_begin + (x < a.nfast ? a.chunk_fast : a.chunk_vis));
+    const uint32_t t_last = (uint32_t)(t_end - 1);
+    const uint16_t* ksb = a.ks + b * a.ks_sb + kv * a.ks_sh;
+    const uint16_t* vsb = a.vs + b * a.vs_sb + kv * a.vs_sh;
+    const uint8_t* smb = a.sm + b * a.sm_sb + kv * a.sm_sh;
+    const uint16_t* pmb = a.pm + b * a.pm_sb + kv * a.pm_sh;
+    const int64_t nblk = (t_end - t_begin + kBlk - 1) / kBlk;
+    const uint32_t kss2 = 2u * a.ks_ss, vss2 = 2u * a.vs_ss;
+    // this lane's slots of the block's kept values: row and byte column (a
+    // slot past the last re-reads it)
+    const int nsl = a.Dk >> 3;
+    const uint32_t crow_b = 2u * a.Dk + 16u;  // LDS bytes of a row
+    uint32_t cro[2 * DKB], cco[2 * DKB], cld[2 * DKB];
+#pragma unroll
+    for (int j = 0; j < 2 * DKB; ++j) {
+      const int item = min(lane + 64 * j, kBlk * nsl - 1), row = item / nsl, col = item - row * nsl;
+      cro[j] = (uint32_t)row * kss2;
+      cco[j] = 16u * col;
+      cld[j] = (uint32_t)row * crow_b + 16u * col;
+    }
+    const uint32_t mro0 = krow0 * a.sm_ss, mro1 = krow1 * a.sm_ss, mlast = t_last * a.sm_ss;
+    auto load = [&](SparkBuf<DKB>& B, int64_t blk) {
+      const uint32_t t0 = min((uint32_t)(t_begin + blk * kBlk), t_last);
+#pragma unroll
+      for (int j = 0; j < 2 * DKB; ++j)
+        B.c[j] = load_row8b<true, true>(ksb, min(cro[j] + t0 * kss2, t_last * kss2) + cco[j], 0u, 1u, 8);
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb) {
+        const uint8_t* mp = smb + min((sb ? mro1 : mro0) + t0 * a.sm_ss, mlast) + 32u * g;
+        B.m[sb][0] = ((const uint4*)mp)[0];
+        B.m[sb][1] = ((const uint4*)mp)[1];
+        B.f[sb] = pmb[min((sb ? krow1 : krow0) + t0, t_last) * a.pm_ss];
+      }
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        B.v[r] = load_row8b<true, true>(vsb, min((8u * g + r) * vss2 + t0 * vss2, t_last * vss2) + 16u * n, 0u, 1u, 8);
+    };
+    Ring<2, SparkBuf<DKB>> ring(nblk, wave, rot_seed);
+    ring.prime(load);
+    load_q();
+    store_q();
+    __syncthreads();
+    uint4 qf[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      uint16_t hv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) hv[e] = TT::from_f32((n < HMAX) ? s_q[nq][32 * g + 8 * kb + e] : 0.f);
+      qf[kb] = pack8(hv);
+    }
+    char* scw = s_cmp + wave * (kBlk * kCmpRow);
+    auto wave_fence = [] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto compute = [&](SparkBuf<DKB>& B, int64_t blk) {
+      const int lim = (int)min(t_end - (t_begin + blk * kBlk), (int64_t)kBlk);
+#pragma unroll
+      for (int j = 0; j < 2 * DKB; ++j) *(uint4*)(scw + cld[j]) = B.c[j];
+      uint32_t bits[2];
+      bits[0] = mask_bits32(B.m[0]);
+      bits[1] = mask_bits32(B.m[1]);
+      // kept channels in the lanes below, both rows in one word
+      const int cnt = __popc(bits[0]) | (__popc(bits[1]) << 16);
+      const int c16 = __shfl_xor(cnt, 16, 64), c32 = __shfl_xor(cnt + c16, 32, 64);
+      const int below = ((g & 1) ? c16 : 0) + ((g & 2) ? c32 : 0);
+      int first[2] = {below & 0xffff, below >> 16};
+      // a mask row with more than Dk kept channels: those past the Dk-th
+      // take the fill
+      if (__any(first[0] + __popc(bits[0]) > a.Dk || first[1] + __popc(bits[1]) > a.Dk)) {
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb) {
+          const int room = max(a.Dk - first[sb], 0);
+          first[sb] = min(first[sb], a.Dk);
+          while (__popc(bits[sb]) > room) bits[sb] &= ~(0x80000000u >> __clz(bits[sb]));
+        }
+      }
+      wave_fence();
+      float s[8];
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb) {
+        const lds_u16* at = (const lds_u16*)(const uint16_t*)(scw + (sb ? krow1 : krow0) * crow_b) + first[sb];
+        const uint32_t fill2 = B.f[sb] | (B.f[sb] << 16);
+        f32x4 cc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) cc = TT::mfma(expand8(bits[sb], 8 * kb, at, fill2), qf[kb], cc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          s[4 * sb + i] = (8 * g + 4 * sb + i < lim) ? cc[i] * a.scale_log2 : -INFINITY;
+      }
+      wave_fence();
+      softmax_pv<TT>(s, B.v, m, l, acc);
+    };
+    ring.run(load, compute);
+  } else if (is_vis) {
     // ---- visual span: rotated, truncated Keys (Dk channels)
     const int64_t t_begin = x < a.nfast ? (int64_t)x * a.chunk_fast
                                         : (int64_t)a.nfast * a.chunk_fast + (int64_t)(x - a.nfast) * a.chunk_vis;

@@ -125,6 +125,33 @@ def varlen_workspace_bytes(q_full, R_partial, delta_mu, k_full, v_buf, mask_full
     return need.value
 
 
+def recovered_decode(q, R_select, zero_bias, k_full, v_buf, v_gap_at: int, v_gap: int, spark_mask, pruned_mean,
+                     k_pruned, v_sparse, num_kv_groups: int) -> torch.Tensor | None:
+    """Decode over ThinK (``R_select``) or SparK (``spark_mask`` /
+    ``pruned_mean``) pruned Keys without recovering them
+    (rk_recovered_decode); ``None`` where that entry does not take the inputs."""
+    if q.dim() != 3 or not q.is_cuda:
+        return None
+    lib = _lib.load()
+    d = [_lib.desc(t) for t in (q, R_select, zero_bias, k_full, v_buf, spark_mask, pruned_mean, k_pruned, v_sparse)]
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    do = _lib.desc(out)
+    r = [_lib.ref(x) for x in d]
+    args = (*r[:5], int(v_gap_at), int(v_gap), *r[5:], int(num_kv_groups), ctypes.byref(do), _lib.RK_POLICY_PAPER)
+
+    def launch(ws):
+        return lib.rk_recovered_decode(*args, ws.data_ptr(), ws.numel(), _lib.stream_handle(q.device))
+
+    st = launch(_lib.workspace(q.device, 0))
+    if st == _lib.RK_ERR_WORKSPACE:
+        need = ctypes.c_size_t(0)
+        _lib.check(lib.rk_recovered_decode_check(*args, 0, ctypes.byref(need)), "recovered_decode")
+        st = launch(_lib.workspace(q.device, need.value))
+    if st in (_lib.RK_ERR_HIP, _lib.RK_ERR_NO_DEVICE):
+        _lib.check(st, "recovered_decode")
+    return out if st == _lib.RK_OK else None
+
+
 def append_kv(k_new, v_new, k_buf, v_buf, len_full: torch.Tensor) -> None:
     """Write one token's K/V [B,H,1,D] at row ``len_full[b]`` of the span
     buffers and advance ``len_full`` on the device (rk_append_kv)."""
