@@ -406,6 +406,12 @@ int rk_gather_rotation(const rk_tensor* R_full, const rk_tensor* idx,
                        const rk_tensor* mean, const rk_tensor* R_out,
                        const rk_tensor* delta_mu_out, void* stream);
 
+/* rk_gather_rotation of the first k = R_out->shape[3] columns of R_full
+ * (eigenvectors in descending order), with the keep mask [B,H,D] u8 = channel
+ * < k (kv_pruning_utils.py:146-159). */
+int rk_leading_rotation(const rk_tensor* R_full, const rk_tensor* mean, const rk_tensor* R_out,
+                        const rk_tensor* delta_mu_out, const rk_tensor* mask_out, void* stream);
+
 /* ---- ThinK / SparK baselines (the methods RotateK is compared against).
  * Rounding follows the reference's torch GPU ops: each square rounded to
  * the key dtype, a 16-bit mean = dtype(fp32 sum * float(n_out)/float(n_in)),

@@ -117,6 +117,7 @@ _SIGNATURES = {
     "rk_channel_scores": (ctypes.c_int, [_P, _P, _P, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "rk_topk_channels": (ctypes.c_int, [_P, ctypes.c_int64, _P, _P, ctypes.c_void_p]),
     "rk_gather_rotation": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_void_p]),
+    "rk_leading_rotation": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_void_p]),
     "rk_think_score_and_compact_check": (ctypes.c_int, [_P, _P, ctypes.c_int64, ctypes.c_int64, _P, _P,
                                                         ctypes.c_int32, ctypes.POINTER(ctypes.c_size_t)]),
     "rk_think_score_and_compact": (ctypes.c_int, [_P, _P, ctypes.c_int64, ctypes.c_int64, _P, _P,

@@ -127,6 +127,20 @@ def gather_rotation(R_full: torch.Tensor, idx: torch.Tensor, mean: torch.Tensor,
     return Rp, dmu
 
 
+def leading_rotation(basis: torch.Tensor, k: int, mean: torch.Tensor, dtype: torch.dtype):
+    """(R_partial [B,H,D,k], delta_mu [B,H,D], keep mask [B,H,D] bool) in
+    ``dtype`` from the first ``k`` columns of ``basis`` and the fp32 Key mean."""
+    _gpu(basis, "basis")
+    B, H, D = mean.shape
+    Rp = torch.empty(B, H, D, k, device=basis.device, dtype=dtype)
+    dmu = torch.empty(B, H, D, device=basis.device, dtype=dtype)
+    mask = torch.empty(B, H, D, device=basis.device, dtype=torch.bool)
+    d = [_lib.desc(t) for t in (basis, mean, Rp, dmu, mask)]
+    _lib.check(_lib.load().rk_leading_rotation(*[ctypes.byref(x) for x in d],
+                                               _lib.stream_handle(basis.device)), "leading_rotation")
+    return Rp, dmu, mask
+
+
 def query_weight(cov: torch.Tensor, query_states: torch.Tensor, num_key_value_groups: int,
                  out: torch.Tensor | None = None) -> torch.Tensor:
     """Query-aware weighting of the covariance (kv_pruning_utils.py:116-140)
@@ -164,5 +178,5 @@ def eigen_rotation(cov: torch.Tensor, on_host: bool | None = None) -> torch.Tens
     return vecs.flip(dims=[-1]).to(cov.device, non_blocking=True)
 
 
-__all__ = ["key_covariance", "rotate_keys", "channel_scores", "topk_channels", "gather_rotation",
+__all__ = ["key_covariance", "rotate_keys", "channel_scores", "topk_channels", "gather_rotation", "leading_rotation",
            "query_weight", "eigen_rotation", "QUERY_WINDOW"]

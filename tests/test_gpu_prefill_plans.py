@@ -86,3 +86,45 @@ def test_rotation_output_paths(S, k, dtype):
     assert torch.equal(prefill.rotate_keys(K, R.float()), want)
     assert torch.equal(wide[..., :k], want) and bool((wide[..., k:] == 9).all())
     assert torch.equal(odd[..., 1:k + 1], want) and bool((odd[..., k + 1:] == 9).all()) and bool((odd[..., 0] == 9).all())
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,k", [(128, 1), (128, 31), (128, 32), (128, 96), (128, 128), (64, 17), (33, 33), (1, 1)])
+def test_leading_rotation_is_gather_of_the_first_columns(D, k, out_dtype):
+    """The first k columns and their mask in one launch: what the gather with
+    idx = 0..k-1 gives, from a basis with more columns and from a strided one."""
+    print(f"[case] leading rotation D={D} k={k} {out_dtype}", flush=True)
+    B, H = 2, 3
+    g = torch.Generator(device="cuda").manual_seed(D * k)
+    full = torch.randn(B, H, D, D, generator=g, device="cuda")
+    mean = torch.randn(B, H, D, generator=g, device="cuda")
+    idx = torch.arange(k, device="cuda").expand(B, H, k)
+    for basis in (full, full[..., :k].contiguous(), full.transpose(-1, -2)):
+        Rp, dmu, mask = prefill.leading_rotation(basis, k, mean, out_dtype)
+        want_R, want_dmu = prefill.gather_rotation(basis, idx, mean, out_dtype)
+        assert torch.equal(Rp, want_R) and torch.equal(Rp, basis[..., :k].to(out_dtype))
+        assert torch.equal(dmu, want_dmu)
+        m = mean.double().unsqueeze(-1)
+        r = Rp.double()
+        exact = (m - r @ (r.transpose(-1, -2).contiguous() @ m)).squeeze(-1)
+        # fp32 sums of D and k products, then the output's rounding
+        scale = float(exact.abs().max()) + float((r.abs() @ (r.abs().transpose(-1, -2).contiguous() @ m.abs())).max())
+        ulp = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7, torch.float32: 0.0}[out_dtype]
+        assert float((dmu.double() - exact).abs().max()) <= scale * 1e-5 + ulp * float(exact.abs().max())
+        assert mask.dtype == torch.bool and torch.equal(mask, (torch.arange(D, device="cuda") < k).expand(B, H, D))
+
+
+def test_failed_factorisation_raises_from_update_rotatek():
+    """Keys whose fp16 covariance overflows fail the first pivot: the call
+    raises and leaves the pruner's state as it was."""
+    from rotatek_amd.pruning import ChannelPruner
+    print("[case] update_rotatek with a failed pivot", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(0)
+    K = (torch.randn(1, 2, 3000, 128, generator=g, device="cuda") * 40).half()
+    p = ChannelPruner(0.75, 10, 10, solver="power_iter")
+    for _ in range(3):
+        with pytest.raises(torch.linalg.LinAlgError):
+            p.update_rotatek(K, K, K, None, 1)
+        assert not hasattr(p, "current_rotatek_R_partial")
+    out = p.update_rotatek(K / 40, K / 40, K, None, 1)
+    assert bool(torch.isfinite(out[0]).all())
