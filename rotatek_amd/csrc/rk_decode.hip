@@ -967,11 +967,11 @@ namespace {
 
 // What the fused form takes; everything else is recovered first
 // (rk_think_recover / rk_spark_recover, then rk_full_channel_decode).
-int check_recovered(const rk_tensor* q, const rk_tensor* R, const rk_tensor* k_full, const rk_tensor* v_buf,
+int check_recovered(const rk_tensor* q, const rk_tensor* tm, const rk_tensor* k_full, const rk_tensor* v_buf,
                     int64_t v_gap_at, int64_t v_gap, const rk_tensor* mask, const rk_tensor* pm, const rk_tensor* ks,
                     const rk_tensor* vs, int64_t G, const rk_tensor* out, int32_t policy, rk_tensor* v_logical,
-                    rk_tensor* r_shape, Checked* c) {
-  if (!k_full || !v_buf || !ks || !q || !out || (!R == !mask) || (!mask != !pm)) return RK_ERR_NULL;
+                    rk_tensor* R, Checked* c) {
+  if (!k_full || !v_buf || !ks || !q || !out || (!tm == !mask) || (!mask != !pm)) return RK_ERR_NULL;
   int st;
   if ((st = rk::check_desc(v_buf, 4)) || (st = rk::check_desc(k_full, 4)) || (st = rk::check_desc(ks, 4))) return st;
   const int64_t S_f = k_full->shape[2];
@@ -980,22 +980,28 @@ int check_recovered(const rk_tensor* q, const rk_tensor* R, const rk_tensor* k_f
   if (!head_span_ok(v_buf)) return RK_ERR_STRIDE;
   *v_logical = *v_buf;
   v_logical->shape[2] = S_f;
-  if (!R) {  // SparK has no rotation: stand in its shape for the checks
-    memset(r_shape, 0, sizeof(*r_shape));
-    r_shape->dtype = ks->dtype;
-    r_shape->ndim = 4;
-    r_shape->shape[0] = ks->shape[0];
-    r_shape->shape[1] = ks->shape[1];
-    r_shape->shape[2] = q->ndim == 3 ? q->shape[2] : 0;
-    r_shape->shape[3] = ks->shape[3];
-    R = r_shape;
-  }
+  // the shape of ThinK's selection rotation (in the workspace); SparK has
+  // none, and the shape stands in for the checks
+  memset(R, 0, sizeof(*R));
+  R->dtype = ks->dtype;
+  R->ndim = 4;
+  R->shape[0] = ks->shape[0];
+  R->shape[1] = ks->shape[1];
+  R->shape[2] = q->ndim == 3 ? q->shape[2] : 0;
+  R->shape[3] = ks->shape[3];
+  for (int i = 3; i >= 0; --i) R->stride[i] = i == 3 ? 1 : R->stride[i + 1] * R->shape[i + 1];
   if ((st = check_rotatek(q, R, nullptr, k_full, v_logical, nullptr, ks, vs, G, c))) return st;
   if ((st = check_out(out, *c))) return st;
   if (policy != RK_POLICY_PAPER && policy != RK_POLICY_GQA) return RK_ERR_ARG;
   if (c->dtype == RK_F32) return RK_ERR_DTYPE;
   if (c->B == 0 || c->S_v == 0 || c->Dk == 0) return RK_ERR_SHAPE;
-  if (!mask) return RK_OK;
+  if (tm) {
+    if ((st = rk::check_desc(tm, 3))) return st;
+    if (tm->dtype != RK_U8) return RK_ERR_DTYPE;
+    if (tm->shape[0] != c->B || tm->shape[1] != c->H_kv || tm->shape[2] != c->D) return RK_ERR_SHAPE;
+    if (c->Dk > c->D) return RK_ERR_KEEP_DIM;
+    return tm->data ? RK_OK : RK_ERR_NULL;
+  }
   // SparK: head_dim 128, at most 64 kept channels (a block of more does not
   // fit the ring's registers), 16-byte rows of everything
   if (c->D != 128) return RK_ERR_HEAD_DIM;
@@ -1019,7 +1025,7 @@ int check_recovered(const rk_tensor* q, const rk_tensor* R, const rk_tensor* k_f
 
 }  // namespace
 
-extern "C" int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* R_select, const rk_tensor* zero_bias,
+extern "C" int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* zero_bias,
                                          const rk_tensor* k_full, const rk_tensor* v_buf, int64_t v_gap_at,
                                          int64_t v_gap, const rk_tensor* spark_mask, const rk_tensor* pruned_mean,
                                          const rk_tensor* k_pruned, const rk_tensor* v_sparse, int64_t num_kv_groups,
@@ -1028,7 +1034,7 @@ extern "C" int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* R_
   Checked c;
   rk_tensor vl, rs;
   (void)zero_bias;
-  int st = check_recovered(q, R_select, k_full, v_buf, v_gap_at, v_gap, spark_mask, pruned_mean, k_pruned, v_sparse,
+  int st = check_recovered(q, think_mask, k_full, v_buf, v_gap_at, v_gap, spark_mask, pruned_mean, k_pruned, v_sparse,
                            num_kv_groups, out, policy, &vl, &rs, &c);
   if (st) return st;
   const int cus = resolve_cus(num_cus, &st);
@@ -1036,11 +1042,12 @@ extern "C" int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* R_
   rk_decode_plan p;
   policy = decode_policy(c, true, policy, cus);
   if ((st = spark_mask ? plan_spark(c, policy, cus, &p) : plan_for(c, true, policy, cus, &p))) return st;
-  if (workspace_bytes) *workspace_bytes = p.workspace_bytes;
+  // ThinK's selection rotation sits behind the decode's own workspace
+  if (workspace_bytes) *workspace_bytes = p.workspace_bytes + (think_mask ? align256(2 * (size_t)rk::numel(&rs)) : 0);
   return RK_OK;
 }
 
-extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* R_select, const rk_tensor* zero_bias,
+extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* zero_bias,
                                    const rk_tensor* k_full, const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
                                    const rk_tensor* spark_mask, const rk_tensor* pruned_mean,
                                    const rk_tensor* k_pruned, const rk_tensor* v_sparse, int64_t num_kv_groups,
@@ -1048,7 +1055,7 @@ extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* R_select
                                    void* stream) {
   Checked c;
   rk_tensor vl, rs;
-  int st = check_recovered(q, R_select, k_full, v_buf, v_gap_at, v_gap, spark_mask, pruned_mean, k_pruned, v_sparse,
+  int st = check_recovered(q, think_mask, k_full, v_buf, v_gap_at, v_gap, spark_mask, pruned_mean, k_pruned, v_sparse,
                            num_kv_groups, out, policy, &vl, &rs, &c);
   if (st) return st;
   if (zero_bias) {
@@ -1056,9 +1063,21 @@ extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* R_select
     if (!rk::is_float_param(zero_bias->dtype)) return RK_ERR_DTYPE;
     if (zero_bias->shape[0] != c.B || zero_bias->shape[1] != c.H_kv || zero_bias->shape[2] != c.D) return RK_ERR_SHAPE;
   }
-  return run_decode(c, q, R_select, zero_bias, k_full, v_buf, nullptr, k_pruned, v_sparse, out, policy, workspace,
-                    workspace_bytes, stream, true, nullptr, v_gap > 0 ? v_gap_at : -1, v_gap, nullptr, nullptr,
-                    spark_mask, pruned_mean);
+  size_t dec_bytes = workspace_bytes;
+  if (think_mask) {  // a decode over one-hot R = q's kept channels
+    const size_t r_bytes = align256(2 * (size_t)rk::numel(&rs));
+    size_t need = 0;
+    if ((st = rk_recovered_decode_check(q, think_mask, zero_bias, k_full, v_buf, v_gap_at, v_gap, spark_mask,
+                                        pruned_mean, k_pruned, v_sparse, num_kv_groups, out, policy, 0, &need)))
+      return st;
+    if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < need) return RK_ERR_WORKSPACE;
+    dec_bytes = need - r_bytes;
+    rs.data = (char*)workspace + dec_bytes;
+    if ((st = rk_channel_selection(think_mask, &rs, stream))) return st;
+  }
+  return run_decode(c, q, &rs, zero_bias, k_full, v_buf, nullptr, k_pruned, v_sparse, out, policy, workspace,
+                    dec_bytes, stream, true, nullptr, v_gap > 0 ? v_gap_at : -1, v_gap, nullptr, nullptr, spark_mask,
+                    pruned_mean);
 }
 
 // ---- allocation-free decode (rk_rotatek_decode_noalloc)

@@ -125,19 +125,25 @@ def varlen_workspace_bytes(q_full, R_partial, delta_mu, k_full, v_buf, mask_full
     return need.value
 
 
-def recovered_decode(q, R_select, zero_bias, k_full, v_buf, v_gap_at: int, v_gap: int, spark_mask, pruned_mean,
-                     k_pruned, v_sparse, num_kv_groups: int) -> torch.Tensor | None:
-    """Decode over ThinK (``R_select``) or SparK (``spark_mask`` /
-    ``pruned_mean``) pruned Keys without recovering them
+def recovered_decode(q, think_mask, zero_bias, k_buf, v_buf, n_prompt: int, n_vision: int, n_text: int, spark_mask,
+                     pruned_mean, k_pruned, num_kv_groups: int) -> torch.Tensor | None:
+    """Decode over ThinK (``think_mask``) or SparK (``spark_mask`` /
+    ``pruned_mean``) pruned Keys in a span cache's buffers (prompt | text Keys;
+    prompt | visual | text Values) without recovering them
     (rk_recovered_decode); ``None`` where that entry does not take the inputs."""
     if q.dim() != 3 or not q.is_cuda:
         return None
     lib = _lib.load()
-    d = [_lib.desc(t) for t in (q, R_select, zero_bias, k_full, v_buf, spark_mask, pruned_mean, k_pruned, v_sparse)]
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    do = _lib.desc(out)
-    r = [_lib.ref(x) for x in d]
-    args = (*r[:5], int(v_gap_at), int(v_gap), *r[5:], int(num_kv_groups), ctypes.byref(do), _lib.RK_POLICY_PAPER)
+    # the spans as descriptors over the buffers (slicing costs the host more)
+    dk, dv, dvs, do = _lib.desc(k_buf), _lib.desc(v_buf), _lib.desc(v_buf), _lib.desc(out)
+    dk.shape[2], dv.shape[2], dvs.shape[2] = n_prompt + n_text, n_prompt + n_vision + n_text, n_vision
+    if dvs.data:
+        dvs.data += n_prompt * v_buf.stride(2) * v_buf.element_size()
+    dq, dt, dz, dm, dp, dkp = (_lib.desc(t) for t in (q, think_mask, zero_bias, spark_mask, pruned_mean, k_pruned))
+    ref = _lib.ref
+    args = (ref(dq), ref(dt), ref(dz), ref(dk), ref(dv), n_prompt, n_vision, ref(dm), ref(dp), ref(dkp), ref(dvs),
+            int(num_kv_groups), ref(do), _lib.RK_POLICY_PAPER)
 
     def launch(ws):
         return lib.rk_recovered_decode(*args, ws.data_ptr(), ws.numel(), _lib.stream_handle(q.device))
