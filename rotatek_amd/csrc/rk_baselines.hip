@@ -447,6 +447,7 @@ struct SparkArgs {
 
 // Packed 16-bit lanes: two channels per dword, the lower channel in the low
 // half.
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef short i16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
@@ -524,6 +525,15 @@ __device__ __forceinline__ float qsumf(float v) {
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false));
   return v;
 }
+// Least / largest over the four lanes of this lane's quad.
+__device__ __forceinline__ int qmin(int v) {
+  v = min(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false));
+  return min(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false));
+}
+__device__ __forceinline__ int qmax(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false));
+  return max(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false));
+}
 // Exclusive prefix sum over the lanes of the quad below this one.
 __device__ __forceinline__ int qprefix(int v) {
   const int q = threadIdx.x & 3;
@@ -547,7 +557,7 @@ __device__ __forceinline__ int qprefix(int v) {
 // are compacted through LDS in channel order.  MVEC: 8-byte mask stores.
 template <class TT, bool KVEC, bool MVEC, bool CVEC>
 __global__ void __launch_bounds__(kThreads) spark_kernel(const SparkArgs a) {
-  constexpr int kRow = kD + 8;  // compact row slot; element kD is the sink of pruned values
+  constexpr int kRow = kD + 40;  // compact row; the 32 elements from kD on take the pruned values
   __shared__ __align__(16) uint16_t s_row[kThreads / 4][kRow];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, qd = lane >> 2, q = lane & 3;
   const int x = blockIdx.x, bh = blockIdx.y, b = bh / a.k.H, h = bh - b * a.k.H;
@@ -590,56 +600,97 @@ __global__ void __launch_bounds__(kThreads) spark_kernel(const SparkArgs a) {
       uint32_t key[16];
       const u16x2 nan_key = {(unsigned short)SparkScore<TT>::kNaNKey, (unsigned short)SparkScore<TT>::kNaNKey};
 #pragma unroll
-      for (int i = 0; i < 16; ++i)  // |score| bits (scores are >= 0), every NaN -> one key above inf
+      for (int i = 0; i < 16; ++i)  // score bits (scores are >= 0), every NaN, of either sign -> one key above inf
         key[i] = __builtin_bit_cast(
-            uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, sc.score(kw[i], i) & 0x7FFF7FFFu), nan_key));
+            uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, sc.score(kw[i], i)), nan_key));
       uint32_t ksum = 0u;
       const u16x2 one = {1, 1};
 #pragma unroll
       for (int i = 0; i < 16; ++i) ksum = __builtin_amdgcn_udot2(__builtin_bit_cast(u16x2, key[i]), one, ksum, false);
-      uint32_t T = 0u;  // largest T with #{key >= T} >= keep in this token
+      // The threshold T: the least number of halvings of [lo, hi) with
+      // #{key >= lo} >= keep > #{key >= hi}, ended by hi = lo + 1 (then T
+      // is the keep-th largest key) or by a count of exactly keep (then any
+      // T does).  hi starts above the largest key, lo at the least of
+      // disjoint groups' largest keys, of which there are at least keep: 32
+      // groups of four for keep <= 32, 64 pairs for keep <= 64, else the
+      // least key of all.
+      u16x2 m2[8], m4[4];
 #pragma unroll
-      for (int bit = 14; bit >= 0; --bit) {
-        const uint32_t cand = T | (1u << bit);
-        T = qsum(count_ge(key, ksum, cand)) >= keep ? cand : T;
+      for (int i = 0; i < 8; ++i)
+        m2[i] = __builtin_elementwise_max(__builtin_bit_cast(u16x2, key[2 * i]), __builtin_bit_cast(u16x2, key[2 * i + 1]));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m4[i] = __builtin_elementwise_max(m2[2 * i], m2[2 * i + 1]);
+      const u16x2 mx = __builtin_elementwise_max(__builtin_elementwise_max(m4[0], m4[1]),
+                                                 __builtin_elementwise_max(m4[2], m4[3]));
+      u16x2 mn;
+      if (keep <= 32) {  // launch-uniform
+        mn = __builtin_elementwise_min(__builtin_elementwise_min(m4[0], m4[1]), __builtin_elementwise_min(m4[2], m4[3]));
+      } else if (keep <= 64) {
+        mn = m2[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) mn = __builtin_elementwise_min(mn, m2[i]);
+      } else {
+        mn = __builtin_bit_cast(u16x2, key[0]);
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mn = __builtin_elementwise_min(mn, __builtin_bit_cast(u16x2, key[i]));
       }
-      const int ge = T == 0u ? 32 : count_ge(key, ksum, T), gt = count_ge(key, ksum, T + 1u);
-      const int need = keep - qsum(gt), eq = qsum(ge - gt);
+      int lo = qmin((int)min(mn.x, mn.y)), hi = qmax((int)max(mx.x, mx.y)) + 1, at_lo = -1;
+      while (__any(hi - lo > 1)) {
+        const int mid = (lo + hi) >> 1;
+        const int c = qsum(count_ge(key, ksum, (uint32_t)max(mid, 1)));
+        const bool up = c >= keep && hi - lo > 1;
+        hi = up ? (c == keep ? mid + 1 : hi) : min(hi, max(mid, lo + 1));
+        at_lo = up ? c : at_lo;
+        lo = up ? mid : lo;
+      }
+      const uint32_t T = (uint32_t)lo;
       const unsigned short Ts = (unsigned short)T;
       const u16x2 T2 = {Ts, Ts};
 #pragma unroll
       for (int i = 0; i < 16; ++i)  // key < T: the wrapped 15-bit difference is negative
         pm[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(i16x2, __builtin_bit_cast(u16x2, key[i]) - T2) >> 15);
-      if (__any(need != eq)) {  // some token keeps only part of its ties: lowest channels first
-        int run = qprefix(ge - gt);
+      if (__any(at_lo != keep)) {
+        // in some token more than keep channels reach T: it keeps those above
+        // T and the lowest of its ties
+        const int ge = T == 0u ? 32 : count_ge(key, ksum, T), gt = count_ge(key, ksum, T + 1u);
+        const int room = max(keep - qsum(gt) - qprefix(ge - gt), 0);  // ties this lane keeps, at most
+        if (__any(ge - gt > room)) {
+          // the lane's ties, one bit per channel, without the lowest `room`
+          uint32_t nt[2] = {0u, 0u};
+          const u16x2 one1 = {1, 1};
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-#pragma unroll
-          for (int hh = 0; hh < 2; ++hh) {
-            const uint32_t k = (key[i] >> (16 * hh)) & 0xFFFFu;
-            const bool tie = k == T;
-            if (tie && run >= need) pm[i] |= 0xFFFFu << (16 * hh);
-            run += tie;
+          for (int i = 0; i < 16; ++i) {
+            const u16x2 ne = __builtin_elementwise_min(__builtin_bit_cast(u16x2, key[i] ^ __builtin_bit_cast(uint32_t, T2)), one1);
+            const u16x2 wt = {(unsigned short)(1u << (2 * (i & 7))), (unsigned short)(2u << (2 * (i & 7)))};
+            nt[i >> 3] = __builtin_amdgcn_udot2(ne, wt, nt[i >> 3], false);
           }
+          uint32_t drop = ~(nt[0] | (nt[1] << 16));
+          for (int r = min(room, ge - gt); __any(r > 0); --r) drop = r > 0 ? drop & (drop - 1u) : drop;
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            pm[i] |= ((uint32_t)__builtin_amdgcn_sbfe(drop, 2 * i, 1) & 0xFFFFu) |
+                     ((uint32_t)__builtin_amdgcn_sbfe(drop, 2 * i + 1, 1) & 0xFFFF0000u);
         }
       }
     }
-    // kept values -> LDS in channel order, the rest to the sink slot
-    int kept = 0;
+    // kept values -> LDS in channel order, the rest to a sink behind the row.
+    // Channel e of the lane goes to element pos + e - (pruned before it),
+    // so one running address serves and e is the store's offset.
+    int kept = 32;
+    const i16x2 ones = {1, 1};
 #pragma unroll
-    for (int i = 0; i < 16; ++i) kept += (int)((~pm[i]) & 1u) + (int)((~pm[i] >> 16) & 1u);
-    int pos = qprefix(kept);
+    for (int i = 0; i < 16; ++i) kept = __builtin_amdgcn_sdot2(__builtin_bit_cast(i16x2, pm[i]), ones, kept, false);
+    lds_u16* at = (lds_u16*)row + qprefix(kept);
+    lds_u16* const sink = (lds_u16*)row + kD;
     float psum = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       psum = SparkScore<TT>::add2(kw[i] & pm[i], psum);  // the pruned values (kept ones read as +0)
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const uint16_t v = (uint16_t)(kw[i] >> (16 * hh));
-        const bool k = ((pm[i] >> (16 * hh)) & 1u) == 0u;
-        row[k ? pos : kD] = v;
-        pos += k;
-      }
+      const int p0 = __builtin_amdgcn_sbfe((int)pm[i], 0, 16), p1 = (int)pm[i] >> 16;  // -1: pruned
+      (p0 ? sink : at)[2 * i] = (uint16_t)kw[i];
+      at += p0;
+      (p1 ? sink : at)[2 * i + 1] = (uint16_t)(kw[i] >> 16);
+      at += p1;
     }
     psum = qsumf(psum);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
