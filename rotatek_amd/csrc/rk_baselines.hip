@@ -634,12 +634,15 @@ __global__ void __launch_bounds__(kThreads) spark_kernel(const SparkArgs a) {
 #pragma unroll
         for (int i = 1; i < 16; ++i) mn = __builtin_elementwise_min(mn, __builtin_bit_cast(u16x2, key[i]));
       }
-      int lo = qmin((int)min(mn.x, mn.y)), hi = qmax((int)max(mx.x, mx.y)) + 1, at_lo = -1;
+      int lo = qmin((int)min(mn.x, mn.y)), hi = qmax((int)max(mx.x, mx.y)) + 1;
+      int at_lo = -1, at_hi = 0;  // #{key >= lo} (-1: not counted), #{key >= hi}
       while (__any(hi - lo > 1)) {
         const int mid = (lo + hi) >> 1;
         const int c = qsum(count_ge(key, ksum, (uint32_t)max(mid, 1)));
         const bool up = c >= keep && hi - lo > 1;
-        hi = up ? (c == keep ? mid + 1 : hi) : min(hi, max(mid, lo + 1));
+        const bool down = c < keep && hi - lo > 1;
+        hi = down ? mid : up && c == keep ? mid + 1 : hi;
+        at_hi = down ? c : at_hi;
         at_lo = up ? c : at_lo;
         lo = up ? mid : lo;
       }
@@ -650,26 +653,27 @@ __global__ void __launch_bounds__(kThreads) spark_kernel(const SparkArgs a) {
       for (int i = 0; i < 16; ++i)  // key < T: the wrapped 15-bit difference is negative
         pm[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(i16x2, __builtin_bit_cast(u16x2, key[i]) - T2) >> 15);
       if (__any(at_lo != keep)) {
-        // in some token more than keep channels reach T: it keeps those above
-        // T and the lowest of its ties
-        const int ge = T == 0u ? 32 : count_ge(key, ksum, T), gt = count_ge(key, ksum, T + 1u);
-        const int room = max(keep - qsum(gt) - qprefix(ge - gt), 0);  // ties this lane keeps, at most
-        if (__any(ge - gt > room)) {
-          // the lane's ties, one bit per channel, without the lowest `room`
-          uint32_t nt[2] = {0u, 0u};
-          const u16x2 one1 = {1, 1};
+        // in some token more than keep channels reach T, its keep-th largest
+        // key: it keeps the at_hi above T and the lowest of its ties.  The
+        // lane's ties, one bit per channel:
+        uint32_t nt[2] = {0u, 0u};
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const u16x2 ne = __builtin_elementwise_min(__builtin_bit_cast(u16x2, key[i] ^ __builtin_bit_cast(uint32_t, T2)), one1);
-            const u16x2 wt = {(unsigned short)(1u << (2 * (i & 7))), (unsigned short)(2u << (2 * (i & 7)))};
-            nt[i >> 3] = __builtin_amdgcn_udot2(ne, wt, nt[i >> 3], false);
-          }
-          uint32_t drop = ~(nt[0] | (nt[1] << 16));
-          for (int r = min(room, ge - gt); __any(r > 0); --r) drop = r > 0 ? drop & (drop - 1u) : drop;
+        for (int i = 0; i < 16; ++i) {
+          const u16x2 ne = __builtin_elementwise_min(__builtin_bit_cast(u16x2, key[i] ^ __builtin_bit_cast(uint32_t, T2)), one);
+          const u16x2 wt = {(unsigned short)(1u << (2 * (i & 7))), (unsigned short)(2u << (2 * (i & 7)))};
+          nt[i >> 3] = __builtin_amdgcn_udot2(ne, wt, nt[i >> 3], false);
+        }
+        uint32_t drop = ~(nt[0] | (nt[1] << 16));
+        const int ties = __popc(drop);
+        // (a token with an exact count keeps all it has)
+        int room = at_lo == keep ? ties : min(max(keep - at_hi - qprefix(ties), 0), ties);
+        for (; __any(room > 0); --room) drop = room > 0 ? drop & (drop - 1u) : drop;
+        if (__any(drop != 0u)) {
 #pragma unroll
           for (int i = 0; i < 16; ++i)
-            pm[i] |= ((uint32_t)__builtin_amdgcn_sbfe(drop, 2 * i, 1) & 0xFFFFu) |
-                     ((uint32_t)__builtin_amdgcn_sbfe(drop, 2 * i + 1, 1) & 0xFFFF0000u);
+            if (__any(drop & (3u << (2 * i))))  // few channels: most words have none
+              pm[i] |= ((uint32_t)__builtin_amdgcn_sbfe(drop, 2 * i, 1) & 0xFFFFu) |
+                       ((uint32_t)__builtin_amdgcn_sbfe(drop, 2 * i + 1, 1) & 0xFFFF0000u);
         }
       }
     }
@@ -680,17 +684,18 @@ __global__ void __launch_bounds__(kThreads) spark_kernel(const SparkArgs a) {
     const i16x2 ones = {1, 1};
 #pragma unroll
     for (int i = 0; i < 16; ++i) kept = __builtin_amdgcn_sdot2(__builtin_bit_cast(i16x2, pm[i]), ones, kept, false);
-    lds_u16* at = (lds_u16*)row + qprefix(kept);
-    lds_u16* const sink = (lds_u16*)row + kD;
+    uint32_t at = (uint32_t)(uintptr_t)(lds_u16*)row + 2u * qprefix(kept);
+    const uint32_t sink = (uint32_t)(uintptr_t)(lds_u16*)row + 2u * kD;
     float psum = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       psum = SparkScore<TT>::add2(kw[i] & pm[i], psum);  // the pruned values (kept ones read as +0)
-      const int p0 = __builtin_amdgcn_sbfe((int)pm[i], 0, 16), p1 = (int)pm[i] >> 16;  // -1: pruned
-      (p0 ? sink : at)[2 * i] = (uint16_t)kw[i];
-      at += p0;
-      (p1 ? sink : at)[2 * i + 1] = (uint16_t)(kw[i] >> 16);
-      at += p1;
+      // all ones: pruned
+      const uint32_t p0 = (uint32_t)__builtin_amdgcn_sbfe((int)pm[i], 0, 16), p1 = (uint32_t)((int)pm[i] >> 16);
+      ((lds_u16*)(uintptr_t)((p0 & sink) | (~p0 & at)))[2 * i] = (uint16_t)kw[i];
+      at += 2u * p0;
+      ((lds_u16*)(uintptr_t)((p1 & sink) | (~p1 & at)))[2 * i + 1] = (uint16_t)(kw[i] >> 16);
+      at += 2u * p1;
     }
     psum = qsumf(psum);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
