@@ -240,19 +240,18 @@ int rk_append_kv(const rk_tensor* k_new, const rk_tensor* v_new, const rk_tensor
  * prompt + text Keys; v_buf [B,H_kv,S_f+v_gap,D] with row t of the prompt +
  * text Values at t + v_gap from t = v_gap_at on; k_pruned [B,H_kv,S_v,Dk];
  * v_sparse [B,H_kv,S_v,D].  Either think_mask [B,H_kv,D] u8 (its
- * one-hot rotation, rk_channel_selection, is formed in the workspace;
- * zero_bias, optional, a delta_mu of zeros that carries non-finite queries
- * through) or spark_mask [B,H_kv,S_v,D] u8 with
+ * one-hot rotation, rk_channel_selection, is formed in the workspace) or
+ * spark_mask [B,H_kv,S_v,D] u8 with
  * pruned_mean [B,H_kv,S_v,1] (SparK: D = 128, Dk <= 64 and a multiple of 8,
  * 16-byte aligned rows).  Inputs outside that are refused: recover them
  * (rk_think_recover, rk_spark_recover) and run rk_full_channel_decode. */
-int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* zero_bias,
-                              const rk_tensor* k_full, const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
+int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* k_full,
+                              const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
                               const rk_tensor* spark_mask, const rk_tensor* pruned_mean, const rk_tensor* k_pruned,
                               const rk_tensor* v_sparse, int64_t num_kv_groups, const rk_tensor* out,
                               int32_t policy, int32_t num_cus, size_t* workspace_bytes);
-int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* zero_bias,
-                        const rk_tensor* k_full, const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
+int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* k_full,
+                        const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
                         const rk_tensor* spark_mask, const rk_tensor* pruned_mean, const rk_tensor* k_pruned,
                         const rk_tensor* v_sparse, int64_t num_kv_groups, const rk_tensor* out, int32_t policy,
                         void* workspace, size_t workspace_bytes, void* stream);

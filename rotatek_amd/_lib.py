@@ -92,10 +92,10 @@ _SIGNATURES = {
                                                     ctypes.c_int32, ctypes.POINTER(ctypes.c_size_t)]),
     "rk_full_channel_decode": (ctypes.c_int, [_P, _P, _P, ctypes.c_int64, _P, ctypes.c_int32,
                                               ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
-    "rk_recovered_decode_check": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_int64, _P, _P, _P, _P,
+    "rk_recovered_decode_check": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int64, _P, _P, _P, _P,
                                                  ctypes.c_int64, _P, ctypes.c_int32, ctypes.c_int32,
                                                  ctypes.POINTER(ctypes.c_size_t)]),
-    "rk_recovered_decode": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_int64, _P, _P, _P, _P,
+    "rk_recovered_decode": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int64, _P, _P, _P, _P,
                                            ctypes.c_int64, _P, ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t,
                                            ctypes.c_void_p]),
     "rk_plan_decode": (ctypes.c_int, [ctypes.c_int64] * 6 + [ctypes.c_int32] * 3

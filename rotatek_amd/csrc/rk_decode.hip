@@ -1025,15 +1025,14 @@ int check_recovered(const rk_tensor* q, const rk_tensor* tm, const rk_tensor* k_
 
 }  // namespace
 
-extern "C" int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* zero_bias,
-                                         const rk_tensor* k_full, const rk_tensor* v_buf, int64_t v_gap_at,
-                                         int64_t v_gap, const rk_tensor* spark_mask, const rk_tensor* pruned_mean,
+extern "C" int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* k_full,
+                                         const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
+                                         const rk_tensor* spark_mask, const rk_tensor* pruned_mean,
                                          const rk_tensor* k_pruned, const rk_tensor* v_sparse, int64_t num_kv_groups,
                                          const rk_tensor* out, int32_t policy, int32_t num_cus,
                                          size_t* workspace_bytes) {
   Checked c;
   rk_tensor vl, rs;
-  (void)zero_bias;
   int st = check_recovered(q, think_mask, k_full, v_buf, v_gap_at, v_gap, spark_mask, pruned_mean, k_pruned, v_sparse,
                            num_kv_groups, out, policy, &vl, &rs, &c);
   if (st) return st;
@@ -1047,8 +1046,8 @@ extern "C" int rk_recovered_decode_check(const rk_tensor* q, const rk_tensor* th
   return RK_OK;
 }
 
-extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* zero_bias,
-                                   const rk_tensor* k_full, const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
+extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_mask, const rk_tensor* k_full,
+                                   const rk_tensor* v_buf, int64_t v_gap_at, int64_t v_gap,
                                    const rk_tensor* spark_mask, const rk_tensor* pruned_mean,
                                    const rk_tensor* k_pruned, const rk_tensor* v_sparse, int64_t num_kv_groups,
                                    const rk_tensor* out, int32_t policy, void* workspace, size_t workspace_bytes,
@@ -1058,16 +1057,11 @@ extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_ma
   int st = check_recovered(q, think_mask, k_full, v_buf, v_gap_at, v_gap, spark_mask, pruned_mean, k_pruned, v_sparse,
                            num_kv_groups, out, policy, &vl, &rs, &c);
   if (st) return st;
-  if (zero_bias) {
-    if ((st = rk::check_desc(zero_bias, 3))) return st;
-    if (!rk::is_float_param(zero_bias->dtype)) return RK_ERR_DTYPE;
-    if (zero_bias->shape[0] != c.B || zero_bias->shape[1] != c.H_kv || zero_bias->shape[2] != c.D) return RK_ERR_SHAPE;
-  }
   size_t dec_bytes = workspace_bytes;
   if (think_mask) {  // a decode over one-hot R = q's kept channels
     const size_t r_bytes = align256(2 * (size_t)rk::numel(&rs));
     size_t need = 0;
-    if ((st = rk_recovered_decode_check(q, think_mask, zero_bias, k_full, v_buf, v_gap_at, v_gap, spark_mask,
+    if ((st = rk_recovered_decode_check(q, think_mask, k_full, v_buf, v_gap_at, v_gap, spark_mask,
                                         pruned_mean, k_pruned, v_sparse, num_kv_groups, out, policy, 0, &need)))
       return st;
     if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < need) return RK_ERR_WORKSPACE;
@@ -1075,7 +1069,7 @@ extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_ma
     rs.data = (char*)workspace + dec_bytes;
     if ((st = rk_channel_selection(think_mask, &rs, stream))) return st;
   }
-  return run_decode(c, q, &rs, zero_bias, k_full, v_buf, nullptr, k_pruned, v_sparse, out, policy, workspace,
+  return run_decode(c, q, &rs, nullptr, k_full, v_buf, nullptr, k_pruned, v_sparse, out, policy, workspace,
                     dec_bytes, stream, true, nullptr, v_gap > 0 ? v_gap_at : -1, v_gap, nullptr, nullptr, spark_mask,
                     pruned_mean);
 }

@@ -125,7 +125,7 @@ def varlen_workspace_bytes(q_full, R_partial, delta_mu, k_full, v_buf, mask_full
     return need.value
 
 
-def recovered_decode(q, think_mask, zero_bias, k_buf, v_buf, n_prompt: int, n_vision: int, n_text: int, spark_mask,
+def recovered_decode(q, think_mask, k_buf, v_buf, n_prompt: int, n_vision: int, n_text: int, spark_mask,
                      pruned_mean, k_pruned, num_kv_groups: int) -> torch.Tensor | None:
     """Decode over ThinK (``think_mask``) or SparK (``spark_mask`` /
     ``pruned_mean``) pruned Keys in a span cache's buffers (prompt | text Keys;
@@ -140,9 +140,9 @@ def recovered_decode(q, think_mask, zero_bias, k_buf, v_buf, n_prompt: int, n_vi
     dk.shape[2], dv.shape[2], dvs.shape[2] = n_prompt + n_text, n_prompt + n_vision + n_text, n_vision
     if dvs.data:
         dvs.data += n_prompt * v_buf.stride(2) * v_buf.element_size()
-    dq, dt, dz, dm, dp, dkp = (_lib.desc(t) for t in (q, think_mask, zero_bias, spark_mask, pruned_mean, k_pruned))
+    dq, dt, dm, dp, dkp = (_lib.desc(t) for t in (q, think_mask, spark_mask, pruned_mean, k_pruned))
     ref = _lib.ref
-    args = (ref(dq), ref(dt), ref(dz), ref(dk), ref(dv), n_prompt, n_vision, ref(dm), ref(dp), ref(dkp), ref(dvs),
+    args = (ref(dq), ref(dt), ref(dk), ref(dv), n_prompt, n_vision, ref(dm), ref(dp), ref(dkp), ref(dvs),
             int(num_kv_groups), ref(do), _lib.RK_POLICY_PAPER)
 
     def launch(ws):

@@ -139,3 +139,18 @@ def test_non_finite_queries():
         q[0, 0, int((~m).nonzero()[0])] = float("inf")
         got, want = c.decode_recovered(q, 0, 1), _staged(c, q, 1)
         assert torch.equal(got.isnan(), want.isnan())
+
+
+def test_refused_calls_stay_refused():
+    """Pruned Keys off the device and unified layers raise before any launch, as with recovered Keys."""
+    print("[case] recovered refusals", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q = torch.randn(1, 2, 128, generator=g, device="cuda").half()
+    for method in ("think", "spark"):
+        c = _cache(method, 1, 2, 60, 4, 4, 32, torch.float16, g)
+        c.key_cache_pruned[0] = c.key_cache_pruned[0].cpu()
+        with pytest.raises(RuntimeError, match="GPU tensor"):
+            c.decode_recovered(q, 0, 1)
+    c._spans[0].unified = True
+    with pytest.raises(ValueError, match="unified"):
+        c.decode_recovered(q, 0, 1)
