@@ -17,7 +17,7 @@
 //   spark_qnorm_kernel   q_g = dtype(mean over the G query heads of a KV
 //                        head), q_norm = dtype(||q_g||_2 over the window)
 //   spark_kernel         4 lanes per token: score = dtype(dtype(k^2) qn);
-//                        keep the Dk largest (bitwise search for the
+//                        keep the Dk largest (bounded search for the
 //                        threshold score over packed 15-bit keys, lowest
 //                        channels among the ties); writes K_compact, the
 //                        per-token mask and dtype(mean of the pruned values)
@@ -172,40 +172,6 @@ __device__ __forceinline__ int prefix16(int v) {
   return incl - v;
 }
 
-// Sum of v over the 16 lanes of this lane's row, in every lane of the row
-// (DPP row rotations by 8, 4, 2, 1).
-__device__ __forceinline__ int sum16(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x124, 0xF, 0xF, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x122, 0xF, 0xF, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x121, 0xF, 0xF, false);
-  return v;
-}
-
-template <int CTL>
-__device__ __forceinline__ float fdpp(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTL, 0xF, 0xF, false));
-}
-
-__device__ __forceinline__ float fsum16(float v) {
-  v += fdpp<0x128>(v);
-  v += fdpp<0x124>(v);
-  v += fdpp<0x122>(v);
-  v += fdpp<0x121>(v);
-  return v;
-}
-
-// Exclusive prefix sum of v over the 16 lanes of this lane's row (DPP row
-// shifts by 1, 2, 4, 8 with zero fill).
-__device__ __forceinline__ int scan16(int v) {
-  int x = v;
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);
-  return x - v;
-}
-
 constexpr int kTile = 64;     // token rows per workgroup tile
 constexpr int kTilePad = 8;   // LDS row padding (elements): 16-byte aligned rows
 
@@ -279,7 +245,7 @@ __device__ __forceinline__ void query_row8(const View& q, int64_t off, int c0, f
 // grid (B*H), 512 threads.  The window's rows are loaded 32 at a time, one
 // row and eight channels a thread, and pass through LDS to the channel's
 // thread, which sums them in row order (one thread per channel with a load per
-// row was a chain of G x 32 memory latencies: B=8, 32 heads 18.8 -> 7.0 us).
+// row was a chain of G x 32 memory latencies: B=8, 32 heads 18.8 -> 6.0 us).
 template <class TT, bool QV>
 __global__ void __launch_bounds__(kWinThreads) think_select_kernel(const ThinkArgs a) {
   __shared__ uint32_t s_key[kD];
@@ -395,7 +361,7 @@ __global__ void __launch_bounds__(kThreads) compact_kernel(View k, const int32_t
 // q_g[t][c] = dtype(sum over the G query heads * f_grp).  A thread forms the
 // group means of one window row's eight channels, kHeads rows in flight;
 // the channel's thread sums their squares in row order (B=16, 4 KV heads
-// of 7 query heads: 101 us with one thread per channel, 7.9 now).
+// of 7 query heads: 101 us with one thread per channel, 5.4 now).
 template <class TT, bool QV>
 __global__ void __launch_bounds__(kWinThreads) spark_qnorm_kernel(View q, int G, int H, float f_grp, float* qn) {
   constexpr int kHeads = 4;
@@ -550,11 +516,15 @@ __device__ __forceinline__ int qprefix(int v) {
 // tokens at once and a workgroup 64; the next 64 rows are loaded while the
 // current ones are selected.  Per token: 15-bit order-preserving score keys
 // (NaN highest, every NaN equal), kept two per dword; the keep-th largest
-// key T by a bitwise search whose counts take three packed 16-bit
-// operations per two keys; every channel above T is kept and, of those
-// equal to T, the lowest channels up to keep (a per-channel pass, taken by a
-// wave only where some token's ties straddle the boundary).  The kept values
-// are compacted through LDS in channel order.  MVEC: 8-byte mask stores.
+// key T by halving a range bounded by the token's group maxima, whose
+// counts take three packed 16-bit operations per two keys; every channel
+// above T is kept and, of those equal to T, the lowest channels up to keep
+// (one bit mask of the lane's ties, formed by a wave only where some token's
+// ties straddle the boundary).  The kept values are compacted through LDS in
+// channel order.  Bound by vector instructions, not by its bytes: the search
+// ends for a wave with its slowest token, so its bounds and its end at an
+// exact count matter most (B=16, 4 heads, 30720 tokens of bf16, keep 32, the
+// whole call: 328 us with a search bit by bit from the top, 274 now).  MVEC: 8-byte mask stores.
 template <class TT, bool KVEC, bool MVEC, bool CVEC>
 __global__ void __launch_bounds__(kThreads) spark_kernel(const SparkArgs a) {
   constexpr int kRow = kD + 40;  // compact row; the 32 elements from kD on take the pruned values
