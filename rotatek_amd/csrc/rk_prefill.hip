@@ -516,19 +516,20 @@ struct RotArgs {
   int64_t o_sb, o_sh, o_ss, o_sd;
   int32_t r_vec;  // R in the Keys' type, rows of whole, aligned 16-byte slots
   int32_t o_vec;  // 16-bit STORE: rows of whole, aligned 16-byte slots
+  int32_t fast;   // 16-bit STORE: rows of K and out of whole, aligned 16-byte slots, head_dim 128
   int32_t o_stream;  // more output than the memory-side cache holds: non-temporal stores
   float* spart;
   int64_t chunk;
   int32_t splits;
 };
 
-// The kept channel of accumulator row m of tile t.  With whole pairs of tiles
-// a lane (rows 4g..4g+3 of both) holds eight consecutive channels 32 p + 8g..,
-// so STORE writes 16 bytes per token and pair, a pair's four lanes one
-// 64-byte segment; a single tile keeps its natural order.
-template <int NT>
+// The kept channel of accumulator row m of tile t.  In PAIRs of tiles a lane
+// (rows 4g..4g+3 of both) holds eight consecutive channels 32 p + 8g.., so
+// the FAST form writes 16 bytes per token and pair, a pair's four lanes one
+// 64-byte segment; else the natural order.
+template <bool PAIR>
 __host__ __device__ constexpr int kept_of(int t, int m) {
-  return NT == 1 ? m : 32 * (t >> 1) + 8 * (m >> 2) + 4 * (t & 1) + (m & 3);
+  return PAIR ? 32 * (t >> 1) + 8 * (m >> 2) + 4 * (t & 1) + (m & 3) : 16 * t + m;
 }
 
 template <class TT, int NT, bool VEC, bool SCORE, bool FAST = false>
@@ -547,7 +548,7 @@ rot_kernel(const RotArgs a) {
   const int64_t rb = b * a.R_sb + (int64_t)h * a.R_sh;
   const int D = FAST ? 128 : a.k.D;
   constexpr int kPer = NT * 16 * 128 / kThreads;
-  constexpr int kBatch = kPer < 16 ? kPer : 16;
+  constexpr int kBatch = FAST && kPer > 16 ? 16 : kPer;
   if (FAST && a.r_vec) {
     // 16-byte loads of R's rows (8 kept channels of one channel c each)
     uint4 v[NT];
@@ -630,13 +631,14 @@ rot_kernel(const RotArgs a) {
         for (int ks = 0; ks < 4; ++ks)
           if (32 * ks + 8 * g >= D) bk[tb][ks] = make_uint4(0, 0, 0, 0);
     }
-    constexpr int NP = NT == 1 ? 1 : 2;  // tiles per pass
+    constexpr bool PAIR = FAST && NT > 1;
+    constexpr int NP = PAIR ? 2 : 1;  // tiles per pass
     // opaque: keeps the R^T fragments in LDS (hoisted out of the step loop
     // they take 16 registers a tile, and the occupancy with them)
-    int aoff = n * 0;
-    asm volatile("" : "+v"(aoff));
+    int aoff = 0;
+    if constexpr (FAST || SCORE) asm volatile("" : "+v"(aoff));
     const uint16_t* rt = &s_rt[0][0] + aoff;
-#pragma unroll 1
+#pragma unroll(FAST ? 1 : SCORE || NT <= 2 ? NT : 1)
     for (int t = 0; t < NT; t += NP) {
       f32x4 c[NP][TB];
 #pragma unroll
@@ -647,7 +649,7 @@ rot_kernel(const RotArgs a) {
       for (int ks = 0; ks < 4; ++ks) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-          const uint4 av = *(const uint4*)(rt + kept_of<NT>(t + p, n) * (128 + 8) + 32 * ks + 8 * g);
+          const uint4 av = *(const uint4*)(rt + kept_of<PAIR>(t + p, n) * (128 + 8) + 32 * ks + 8 * g);
 #pragma unroll
           for (int tb = 0; tb < TB; ++tb) c[p][tb] = TT::mfma(av, bk[tb][ks], c[p][tb]);
         }
@@ -660,7 +662,7 @@ rot_kernel(const RotArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) sc[t + p][r] += fabsf(c[p][tb][r]);
       } else {
-        const int k0 = kept_of<NT>(t, 4 * g);
+        const int k0 = kept_of<PAIR>(t, 4 * g);
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) {
           if (16 * tb + n < left) {
@@ -679,12 +681,12 @@ rot_kernel(const RotArgs a) {
                                                  TT::pack2(c[0][tb][2], c[0][tb][3]));
                 }
               }
+            } else if (k0 + 3 < a.Dk && a.o_sd == 1 && (((uintptr_t)(o + k0)) & 7) == 0) {
+              *(uint2*)(o + k0) = make_uint2(TT::pack2(c[0][tb][0], c[0][tb][1]), TT::pack2(c[0][tb][2], c[0][tb][3]));
             } else {
 #pragma unroll
-              for (int p = 0; p < NP; ++p)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                  if (k0 + 4 * p + r < a.Dk) o[(k0 + 4 * p + r) * a.o_sd] = TT::from_f32(c[p][tb][r]);
+              for (int r = 0; r < 4; ++r)
+                if (k0 + r < a.Dk) o[(k0 + r) * a.o_sd] = TT::from_f32(c[0][tb][r]);
             }
           }
         }
@@ -711,7 +713,7 @@ rot_kernel(const RotArgs a) {
         v += shfl_xor(v, 2);
         v += shfl_xor(v, 4);
         v += shfl_xor(v, 8);
-        if (n == 0) s_sc[wave][kept_of<NT>(t, 4 * g + r)] = v;
+        if (n == 0) s_sc[wave][16 * t + 4 * g + r] = v;
       }
     __syncthreads();
     for (int kk = tid; kk < NT * 16; kk += kThreads) {
@@ -1338,10 +1340,13 @@ struct CovPlan {
 // budget): rounds x (tokens per workgroup + 360 for the centre, the sum of
 // the waves and the partial, 8 us) + 0.66 per partial for the finalisation's
 // reads (a single workgroup per head has none).  B=10, 32 heads, 4000 tokens:
-// 2 -> 3 splits, 177 -> 161 us; B=32, 14000 tokens: one.
-int cov_splits_for(int64_t bh, int64_t S, int cus) {
+// 2 -> 3 splits, 177 -> 161 us; B=32, 14000 tokens: one.  A workgroup takes
+// at least 512 tokens of 16-bit Keys (32 heads, 4097 tokens, 256 allowed: 33.3
+// us for the whole covariance, 32.2 so), 256 of fp32, whose products take
+// eight times as long (2304 tokens: 50.6 -> 45.7 us).
+int cov_splits_for(int64_t bh, int64_t S, int cus, bool f32) {
   if (S <= 0 || bh <= 0) return 1;
-  const int64_t cap = std::min<int64_t>(cdiv(S, 256), 64);
+  const int64_t cap = std::min<int64_t>(cdiv(S, f32 ? 256 : 512), 64);
   double best = 0;
   int splits = 1;
   for (int64_t s = 1; s <= cap; ++s) {
@@ -1351,7 +1356,7 @@ int cov_splits_for(int64_t bh, int64_t S, int cus) {
   return splits;
 }
 
-CovPlan cov_plan(int64_t B, int64_t H, int64_t S, int cus) {
+CovPlan cov_plan(int64_t B, int64_t H, int64_t S, int cus, bool f32) {
   CovPlan p;
   const int64_t bh = B * H;
   // the mean pass has no epilogue to speak of: at most 512 tokens a
@@ -1359,7 +1364,7 @@ CovPlan cov_plan(int64_t B, int64_t H, int64_t S, int cus) {
   // tokens, one workgroup per head: 938 us, 3.9 TB/s; 28 per head: 560)
   p.mean_splits = (int)std::min<int64_t>(std::max<int64_t>(splits_for(bh, S, cus, 256), cdiv(S, 512)), 4096);
   p.mean_chunk = cdiv(S > 0 ? S : 1, p.mean_splits);
-  p.cov_splits = cov_splits_for(bh, S, cus);
+  p.cov_splits = cov_splits_for(bh, S, cus, f32);
   p.cov_chunk = cdiv(S > 0 ? S : 1, p.cov_splits);
   p.off_mean = 0;
   p.off_cov = align256((size_t)bh * p.mean_splits * 128 * sizeof(float));
@@ -1498,7 +1503,7 @@ extern "C" int rk_key_covariance_check(const rk_tensor* keys, const rk_tensor* m
   if (mean_out && (st = check_f32_out(mean_out, 3, B, H, k.D, RK_F32))) return st;
   const int cus = resolve_cus(num_cus, &st);
   if (st) return st;
-  if (workspace_bytes) *workspace_bytes = cov_plan(B, H, k.S, cus).total;
+  if (workspace_bytes) *workspace_bytes = cov_plan(B, H, k.S, cus, keys->dtype == RK_F32).total;
   return RK_OK;
 }
 
@@ -1514,7 +1519,7 @@ extern "C" int rk_key_covariance(const rk_tensor* keys, const rk_tensor* mean_ou
   if (mean_out && (st = check_f32_out(mean_out, 3, B, H, k.D, RK_F32))) return st;
   const int cus = resolve_cus(0, &st);
   if (st) return st;
-  const CovPlan p = cov_plan(B, H, k.S, cus);
+  const CovPlan p = cov_plan(B, H, k.S, cus, keys->dtype == RK_F32);
   if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < p.total) return RK_ERR_WORKSPACE;
   if (B * H == 0) return RK_OK;
   if ((k.S > 0 && !k.data) || !cov_out->data) return RK_ERR_NULL;
@@ -1573,7 +1578,7 @@ extern "C" int rk_key_covariance_weighted(const rk_tensor* keys, const rk_tensor
   if ((st = check_queries(keys, queries, num_kv_groups, window, &qw))) return st;
   const int cus = resolve_cus(0, &st);
   if (st) return st;
-  const CovPlan p = cov_plan(B, H, k.S, cus);
+  const CovPlan p = cov_plan(B, H, k.S, cus, keys->dtype == RK_F32);
   if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < p.total) return RK_ERR_WORKSPACE;
   if (B * H == 0) return RK_OK;
   if ((k.S > 0 && !k.data) || !cov_out->data || !queries->data) return RK_ERR_NULL;
@@ -1603,7 +1608,7 @@ hipError_t launch_rot(const RotArgs& a, bool vec, dim3 grid, hipStream_t s) {
     else
       hipLaunchKernelGGL((rot32_kernel<NT, false, SCORE>), grid, dim3(kThreads), 0, s, a);
   } else {
-    if (!SCORE && vec && a.o_vec && a.k.D == 128)
+    if (!SCORE && a.fast)
       hipLaunchKernelGGL((rot_kernel<TT, NT, true, false, true>), grid, dim3(kThreads), 0, s, a);
     else if (vec)
       hipLaunchKernelGGL((rot_kernel<TT, NT, true, SCORE>), grid, dim3(kThreads), 0, s, a);
@@ -1644,13 +1649,16 @@ void fill_rot(RotArgs& a, const KeyView& k, const rk_tensor* R, int64_t Dk) {
   a.Dk = (int32_t)Dk;
 }
 
-// One round of four workgroups per CU (the STORE kernels' occupancy), of at
+// FAST: one round of four workgroups per CU (its occupancy), of at
 // least 128 tokens (one 32-token step per wave) and at most 512: shorter
 // workgroups even out the end of grids of many rounds (B=32, 32 heads, 14000
 // tokens, keep 32: 911 us with one workgroup per head, 866 at 1536 tokens,
 // 823 at 512, 830 at 256; one image, 2304 tokens, keep 64: 9.7 -> 8.8 us
-// with 128-token workgroups allowed).
-int rot_splits(int64_t bh, int64_t S, int cus) {
+// with 128-token workgroups allowed).  The others: one round of two per CU,
+// which stage R for at least 512 tokens (scores of 32 heads, 12001 tokens:
+// 35 us against 52 with FAST's splits).
+int rot_splits(int64_t bh, int64_t S, int cus, bool fast) {
+  if (!fast) return splits_for(bh, S, cus, 512);
   if (S <= 0 || bh <= 0) return 1;
   const int64_t want = std::max(std::min(cdiv(4 * (int64_t)cus, bh), cdiv(S, 128)), cdiv(S, 512));
   return (int)std::min<int64_t>(want, 4096);
@@ -1686,7 +1694,8 @@ extern "C" int rk_rotate_keys(const rk_tensor* keys, const rk_tensor* R_partial,
   a.o_vec = rows_vec(out, Dk) ? 1 : 0;
   a.o_stream = rk::numel(out) * rk::dtype_size(out->dtype) > kMallBytes ? 1 : 0;
   a.r_vec = R_partial->dtype == keys->dtype && rows_vec(R_partial, Dk) ? 1 : 0;
-  a.splits = rot_splits(B * H, k.S, cus);
+  a.fast = keys->dtype != RK_F32 && vec && a.o_vec && k.D == 128 ? 1 : 0;
+  a.splits = rot_splits(B * H, k.S, cus, a.fast);
   a.chunk = cdiv(k.S, a.splits);
   const dim3 grid((unsigned)a.splits, (unsigned)(B * H));
   const int nt = (int)cdiv(Dk, 16);
@@ -1708,7 +1717,7 @@ extern "C" int rk_channel_scores_check(const rk_tensor* keys, const rk_tensor* R
   const int cus = resolve_cus(num_cus, &st);
   if (st) return st;
   if (workspace_bytes)
-    *workspace_bytes = align256((size_t)B * H * rot_splits(B * H, k.S, cus) * 128 * sizeof(float));
+    *workspace_bytes = align256((size_t)B * H * rot_splits(B * H, k.S, cus, false) * 128 * sizeof(float));
   return RK_OK;
 }
 
@@ -1728,7 +1737,7 @@ extern "C" int rk_channel_scores(const rk_tensor* keys, const rk_tensor* R_full,
   RotArgs a;
   memset(&a, 0, sizeof(a));
   fill_rot(a, k, R_full, Dk);
-  a.splits = rot_splits(B * H, k.S, cus);
+  a.splits = rot_splits(B * H, k.S, cus, false);
   a.chunk = cdiv(k.S > 0 ? k.S : 1, a.splits);
   const size_t need = align256((size_t)B * H * a.splits * 128 * sizeof(float));
   if (!workspace || (((uintptr_t)workspace) & 255) || workspace_bytes < need) return RK_ERR_WORKSPACE;
