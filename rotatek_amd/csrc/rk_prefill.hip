@@ -1361,8 +1361,14 @@ CovPlan cov_plan(int64_t B, int64_t H, int64_t S, int cus, bool f32) {
   const int64_t bh = B * H;
   // the mean pass has no epilogue to speak of: at most 512 tokens a
   // workgroup, so that grids of many heads end evenly (B=32, 32 heads, 14000
-  // tokens, one workgroup per head: 938 us, 3.9 TB/s; 28 per head: 560)
-  p.mean_splits = (int)std::min<int64_t>(std::max<int64_t>(splits_for(bh, S, cus, 256), cdiv(S, 512)), 4096);
+  // tokens, one workgroup per head: 938 us, 3.9 TB/s; 28 per head: 560), in
+  // at most 32 workgroups per head past two per CU where heads are few, since
+  // every workgroup of the next two launches sums a head's partials again
+  // (the whole covariance, graph-replayed, 512 tokens / 32 workgroups: 8 heads
+  // of 131072 tokens 116.3 / 102.1 us, 4 of 131072 70.1 / 62.2, 32 of 30720
+  // 98.4 / 95.0; but 64 of 30720, weighted, 177.7 / 181.0)
+  const int64_t mean_cap = std::min<int64_t>(std::max<int64_t>(32, bh), 4096);
+  p.mean_splits = (int)std::max<int64_t>(splits_for(bh, S, cus, 256), std::min(cdiv(S, 512), mean_cap));
   p.mean_chunk = cdiv(S > 0 ? S : 1, p.mean_splits);
   p.cov_splits = cov_splits_for(bh, S, cus, f32);
   p.cov_chunk = cdiv(S > 0 ? S : 1, p.cov_splits);
