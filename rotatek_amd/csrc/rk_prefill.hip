@@ -1343,10 +1343,19 @@ struct CovPlan {
 // 2 -> 3 splits, 177 -> 161 us; B=32, 14000 tokens: one.  A workgroup takes
 // at least 512 tokens of 16-bit Keys (32 heads, 4097 tokens, 256 allowed: 33.3
 // us for the whole covariance, 32.2 so), 256 of fp32, whose products take
-// eight times as long (2304 tokens: 50.6 -> 45.7 us).
+// eight times as long (2304 tokens: 50.6 -> 45.7 us).  At most 64 per head
+// (fp32: one per 384 tokens up to 128), past which the estimate misses what
+// the finalisation pays for each partial of a head, about 0.06 us; where heads
+// are too few to fill the CUs so, one per CU, of 16-bit Keys no more than
+// sqrt(S / 16), where that and the tokens' 0.006 us balance.  Graph-replayed
+// whole covariance, 64 / now: one head of 131072 tokens 68.3 / 66.2 us, of
+// 1000000 285 / 131; fp32, one head of 65536 87.4 / 58.4, two 92.8 / 71.2,
+// three of 50000 82.9 / 76.5 (four of 20000, weighted, 52.3 at 64, 53.4 at 79).
 int cov_splits_for(int64_t bh, int64_t S, int cus, bool f32) {
   if (S <= 0 || bh <= 0) return 1;
-  const int64_t cap = std::min<int64_t>(cdiv(S, f32 ? 256 : 512), 64);
+  const int64_t one = cdiv(cus, bh), few = f32 ? one : std::min(one, (int64_t)sqrt((double)S / 16));
+  const int64_t many = f32 ? std::min<int64_t>(std::max<int64_t>(64, S / 384), 128) : 64;
+  const int64_t cap = std::min(cdiv(S, f32 ? 256 : 512), std::max(many, few));
   double best = 0;
   int splits = 1;
   for (int64_t s = 1; s <= cap; ++s) {
