@@ -1467,9 +1467,13 @@ hipError_t launch_cov(const KeyView& k, bool vec, const CovPlan& p, int64_t B, f
   if constexpr (TT::kBytes == 2) {
     if (vec) {
       // Keys past the memory-side cache are streamed; one workgroup per head
-      // finishes its head
+      // finishes its head where there are many.  A few end sooner with a
+      // finalisation of 36 workgroups per head: graph-replayed us at 250
+      // tokens, finishing / separate, 8 heads 21.2 / 17.1, 32 21.5 / 20.8, 40
+      // 21.6 / 21.5, 64 21.7 / 25.0; weighted (more to do per entry) 8 heads
+      // 29.6 / 23.1, 48 30.0 / 28.9, 64 30.2 / 30.8, 128 31.4 / 38.1
       const bool nt = bh * k.S * k.D * 2 > kMallBytes;
-      finished = cs == 1;
+      finished = cs == 1 && bh >= (qw ? 64 : 40);
       nt ? mean(yes, yes) : mean(yes, no);
       if (finished)
         nt ? covk(cov_kernel<TT, true, true, true>) : covk(cov_kernel<TT, true, false, true>);

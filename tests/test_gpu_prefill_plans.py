@@ -43,6 +43,23 @@ def test_covariance_one_workgroup_per_head(B, H, S, D, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("S", [1, 33, 500])
+@pytest.mark.parametrize("H", [39, 40, 63, 64, 65])
+def test_finished_heads_equal_separate_ones(H, S, dtype):
+    """Heads finished by their covariance workgroup (many heads) hold the bits
+    of the separate finalisation (eight at a time), at a non-zero mean."""
+    print(f"[case] finished heads H={H} S={S} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(H + S)
+    K = (torch.randn(1, H, S, 128, generator=g, device="cuda") + 0.7).to(dtype)
+    Q = torch.randn(1, 2 * H, 40, 128, generator=g, device="cuda").to(dtype)
+    for q in (None, Q):
+        mean, cov = prefill.key_covariance(K, q, 2)
+        for h in range(0, H, 8):
+            few = prefill.key_covariance(K[:, h:h + 8], None if q is None else q[:, 2 * h:2 * h + 16], 2)
+            assert torch.equal(mean[:, h:h + 8], few[0]) and torch.equal(cov[:, h:h + 8], few[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("S", [1030, 1031])
 def test_streamed_keys(S, dtype):
     """Keys past the memory-side cache (32 batch rows that share one row's
