@@ -252,7 +252,8 @@ def _cfg0_leg(budget_s=3.0):
 # the shared device helpers
 DECODE_SOURCES = [os.path.join(ROOT, "rotatek_amd", "csrc", f)
                   for f in ("rk_decode.hip", "rk_decode.h", "rk_decode_dev.h", "rk_decode_f16.hip",
-                            "rk_decode_bf16.hip", "rk_decode_f32.hip", "rk_decode_spark.hip", "rk_common.h")]
+                            "rk_decode_bf16.hip", "rk_decode_f32.hip", "rk_decode_spark.hip",
+                            "rk_decode_think_f16.hip", "rk_decode_think_bf16.hip", "rk_common.h")]
 PREFILL_SOURCES = [os.path.join(ROOT, "rotatek_amd", "csrc", f) for f in ("rk_prefill.hip", "rk_rotation.hip",
                                                                           "rk_common.h")]
 # the ThinK / SparK baseline kernels (their dense decode is the decode path's)

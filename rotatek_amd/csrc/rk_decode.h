@@ -109,6 +109,10 @@ hipError_t decode_launch_f32(bool has_vis, bool vec, const DecodeArgs& a, dim3 g
 // channels (kb = ceil(Dk / 32)): both 16-bit types (rk_decode_spark.hip).
 hipError_t decode_launch_spark(int dtype, int kb, int hmax, const DecodeArgs& a, dim3 grid, hipStream_t s);
 
+// ThinK-pruned visual Keys, whose R selects channels (rk_decode_think_*.hip).
+hipError_t decode_launch_think_f16(int dkb, bool vec, int hmax, const DecodeArgs& a, dim3 grid, hipStream_t s);
+hipError_t decode_launch_think_bf16(int dkb, bool vec, int hmax, const DecodeArgs& a, dim3 grid, hipStream_t s);
+
 // Workgroups of the merge kernel: one per unit, or one per 16 units of one
 // query head each (merge_kernel's sliced form).
 inline unsigned merge_grid(const DecodeArgs& a) {

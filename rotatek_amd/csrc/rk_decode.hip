@@ -576,7 +576,7 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
                void* ws, size_t ws_bytes, void* stream, bool has_vis,
                int32_t* len_full = nullptr, int64_t v_gap_at = -1, int64_t v_gap = 0,
                const rk_tensor* k_new = nullptr, const rk_tensor* v_new = nullptr,
-               const rk_tensor* sm = nullptr, const rk_tensor* pm = nullptr) {
+               const rk_tensor* sm = nullptr, const rk_tensor* pm = nullptr, bool sel = false) {
   int st = RK_OK;
   const int cus = resolve_cus(0, &st);
   if (st) return st;
@@ -747,6 +747,9 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
   hipError_t e;
   if (sm)
     e = rk::decode_launch_spark(c.dtype, dkb, hmax, a, grid, s);
+  else if (sel)
+    e = c.dtype == RK_F16 ? rk::decode_launch_think_f16(dkb, vec, hmax, a, grid, s)
+                          : rk::decode_launch_think_bf16(dkb, vec, hmax, a, grid, s);
   else if (vec && c.D < 128)  // 16-byte loads with the channels past D masked
     e = c.dtype == RK_F16 ? rk::decode_launch_f16_hd(dkb, hmax, has_vis, a, grid, s)
                           : rk::decode_launch_bf16_hd(dkb, hmax, has_vis, a, grid, s);
@@ -1071,7 +1074,7 @@ extern "C" int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_ma
   }
   return run_decode(c, q, &rs, nullptr, k_full, v_buf, nullptr, k_pruned, v_sparse, out, policy, workspace,
                     dec_bytes, stream, true, nullptr, v_gap > 0 ? v_gap_at : -1, v_gap, nullptr, nullptr, spark_mask,
-                    pruned_mean);
+                    pruned_mean, think_mask != nullptr);
 }
 
 // ---- allocation-free decode (rk_rotatek_decode_noalloc)

@@ -567,8 +567,11 @@ __device__ __forceinline__ void merge_fused(const DecodeArgs& a, int u, int b, i
 // SPK: the visual Keys are SparK's (kept channels per token, mask, mean of
 // the others): the workgroup puts each block's rows back together in
 // registers as score operands instead of reading recovered Keys.
+// SEL: R selects channels (ThinK).  An instantiation of its own: in the RotateK
+// kernels its few lines moved the register allocator to other scalar spills
+// (B=1, 32 heads, 16k: 31.0 -> 31.4 us).
 template <class TT, int DKB, bool VEC, int HMAX, bool HAS_VIS, bool APPEND, bool DPART = false, bool FUSED = false,
-          bool SPK = false>
+          bool SPK = false, bool SEL = false>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 decode_kernel(const DecodeArgs a) {
   static_assert(!DPART || VEC, "the element-wise kernels mask head_dim at run time");
@@ -1044,7 +1047,16 @@ decode_kernel(const DecodeArgs a) {
         for (int e = 0; e < 8; ++e) {
           const float v = (n < HMAX) ? s_qt[nq][kb * 32 + 8 * g + e] : 0.f;
           qmax = fmaxf(qmax, fabsf(v));
-          TT::split(v * qscale, hv[e], lv[e]);
+          if constexpr (SEL) {
+            // q R holds entries of q, whose low part would be 0, and 0 times
+            // an infinite Key NaN where q . k is infinite: two equal halves
+            // instead (the least subnormal has none)
+            const float x = v * qscale;
+            hv[e] = TT::from_f32(0.5f * x);
+            lv[e] = TT::from_f32(x - TT::to_f32(hv[e]));
+          } else {
+            TT::split(v * qscale, hv[e], lv[e]);
+          }
         }
         qh[kb] = pack8(hv);
         ql[kb] = pack8(lv);
@@ -1789,6 +1801,41 @@ hipError_t launch_one(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   if (e != hipSuccess || a.fused) return e;
   hipLaunchKernelGGL((merge_kernel<TT>), dim3(merge_grid(a)), dim3(kThreads), 0, s, a);
   return hipGetLastError();
+}
+
+// The decode over ThinK-pruned Keys.
+template <class TT, int DKB, bool VEC, int HMAX, bool DPART>
+hipError_t launch_sel(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+  constexpr bool kCanFuse = VEC && !DPART;
+  if (a.fused && !kCanFuse) return hipErrorInvalidValue;
+  if (a.fused)
+    hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, true, false, DPART, kCanFuse, false, true>), grid,
+                       dim3(kThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, true, false, DPART, false, false, true>), grid,
+                       dim3(kThreads), 0, s, a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.fused) return e;
+  hipLaunchKernelGGL((merge_kernel<TT>), dim3(merge_grid(a)), dim3(kThreads), 0, s, a);
+  return hipGetLastError();
+}
+
+template <class TT, int DKB>
+hipError_t launch_sel_any(bool vec, int hmax, const DecodeArgs& a, dim3 grid, hipStream_t s) {
+  if (!vec)
+    return hmax > 1 ? launch_sel<TT, DKB, false, 16, false>(a, grid, s) : launch_sel<TT, DKB, false, 1, false>(a, grid, s);
+  if (a.D < 128)
+    return hmax > 1 ? launch_sel<TT, DKB, true, 16, true>(a, grid, s) : launch_sel<TT, DKB, true, 1, true>(a, grid, s);
+  return hmax > 1 ? launch_sel<TT, DKB, true, 16, false>(a, grid, s) : launch_sel<TT, DKB, true, 1, false>(a, grid, s);
+}
+
+template <class TT>
+hipError_t launch_sel_dk(int dkb, bool vec, int hmax, const DecodeArgs& a, dim3 grid, hipStream_t s) {
+  switch (dkb) {
+    case 1: return launch_sel_any<TT, 1>(vec, hmax, a, grid, s);
+    case 2: return launch_sel_any<TT, 2>(vec, hmax, a, grid, s);
+    default: return launch_sel_any<TT, 4>(vec, hmax, a, grid, s);
+  }
 }
 
 template <class TT, int DKB, bool VEC, int HMAX, bool DPART>

@@ -154,3 +154,24 @@ def test_refused_calls_stay_refused():
     c._spans[0].unified = True
     with pytest.raises(ValueError, match="unified"):
         c.decode_recovered(q, 0, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("method,keep,D", [("think", 8, 128), ("think", 32, 128), ("think", 64, 128), ("think", 96, 128),
+                                           ("think", 32, 96), ("think", 20, 50), ("spark", 32, 128)])
+def test_infinite_keys(method, keep, D, dtype):
+    """A Key that is infinite against the query's sign drops its token, one with it makes the head NaN, as recovered."""
+    print(f"[case] recovered {method} infinite Keys keep={keep} D={D} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(keep)
+    c = _cache(method, 1, 3, 100, 4, 4, keep, dtype, g, D=D)
+    q = torch.randn(1, 6, D, generator=g, device="cuda").to(dtype)
+    row = c.think_mask[0][0] if method == "think" else c.spark_mask[0][0, :, 7]
+    for h in range(3):
+        q[0, 2 * h:2 * h + 2, int(row[h].nonzero()[0])] = 1.5
+    c.key_cache_pruned[0][0, :2, 7, 0] = -float("inf")
+    c.key_cache_pruned[0][0, 2, 7, 0] = float("inf")
+    got, want = c.decode_recovered(q, 0, 2), _staged(c, q, 2)
+    assert bool(torch.isfinite(want[:, :, :4]).all()) and bool(want[:, :, 4:].isnan().all())
+    assert torch.equal(got.isnan(), want.isnan())
+    err, ref = (_np(got) - _np(want))[:, :, :4], np.abs(_np(want))[:, :, :4]
+    assert (np.abs(err) <= np.maximum(TOL[dtype], ref * 2.0 ** -8)).all()
