@@ -240,7 +240,8 @@ int rk_append_kv(const rk_tensor* k_new, const rk_tensor* v_new, const rk_tensor
  * prompt + text Keys; v_buf [B,H_kv,S_f+v_gap,D] with row t of the prompt +
  * text Values at t + v_gap from t = v_gap_at on; k_pruned [B,H_kv,S_v,Dk];
  * v_sparse [B,H_kv,S_v,D].  Either think_mask [B,H_kv,D] u8 (its
- * one-hot rotation, rk_channel_selection, is formed in the workspace) or
+ * one-hot rotation, rk_channel_selection, is formed in the workspace; k_pruned
+ * in 16-byte rows wherever the other rows are) or
  * spark_mask [B,H_kv,S_v,D] u8 with
  * pruned_mean [B,H_kv,S_v,1] (SparK: D = 128, Dk <= 64 and a multiple of 8,
  * 16-byte aligned rows).  Inputs outside that are refused: recover them
