@@ -125,6 +125,22 @@ def varlen_workspace_bytes(q_full, R_partial, delta_mu, k_full, v_buf, mask_full
     return need.value
 
 
+def recovered_decode_takes(q, spark_mask, k_pruned) -> bool:
+    """Whether ``recovered_decode`` may take a ThinK (``spark_mask`` None) or
+    SparK layer: what rk_recovered_decode refuses whatever the sizes, told
+    before anything is packed or allocated (an eager step of a small refused
+    layer spent a third of its time there: 34 us, 50 with it, 34 so)."""
+    D, keep = q.shape[-1], k_pruned.shape[-1]
+    if q.dtype not in (torch.float16, torch.bfloat16) or keep == 0:
+        return False
+    if spark_mask is None:
+        return keep % 8 == 0 or D % 8 != 0
+    if D != 128 or keep > 64 or keep % 8 != 0 or spark_mask.data_ptr() % 16 != 0:
+        return False
+    *rows, last = spark_mask.stride()
+    return last == 1 and all(s % 16 == 0 or n == 1 for s, n in zip(rows, spark_mask.shape))
+
+
 def recovered_decode(q, think_mask, k_buf, v_buf, n_prompt: int, n_vision: int, n_text: int, spark_mask,
                      pruned_mean, k_pruned, num_kv_groups: int) -> torch.Tensor | None:
     """Decode over ThinK (``think_mask``) or SparK (``spark_mask`` /

@@ -3,8 +3,11 @@ the host from the entry's check."""
 import ctypes
 
 import pytest
+import torch
 
 from rotatek_amd import _lib
+from rotatek_amd.cache import DynamicCache
+from rotatek_amd.kernels import _launch
 
 CUS = 256
 
@@ -44,3 +47,44 @@ def test_think_compact_rows(D, Dk, taken):
     wide = _desc((2, 3, 70, Dk), _lib.RK_F16, (3 * 70 * (Dk + 3), 70 * (Dk + 3), Dk + 3, 1))
     if D % 8 == 0:
         assert _check("think", D, Dk, k_pruned=wide) != 0
+
+
+def _layout(method, D, Dk, dtype, kind, B=2, H=3, S_v=70):
+    q, kp = torch.zeros(B, 2 * H, D, dtype=dtype), torch.zeros(B, H, S_v, Dk, dtype=dtype)
+    if method == "think":
+        return q, None, kp
+    wide = torch.zeros(B, H, S_v, 2 * D + 16, dtype=torch.bool)
+    return q, {"rows": torch.zeros(B, H, S_v, D, dtype=torch.bool), "offset": wide[..., 8:8 + D],
+               "strided": wide[..., 16:16 + D], "split": wide[..., :2 * D:2]}[kind], kp
+
+
+@pytest.mark.parametrize("method,kind", [("think", "rows"), ("spark", "rows"), ("spark", "offset"), ("spark", "strided"),
+                                         ("spark", "split")])
+def test_early_refusal_is_the_entry_refusal(method, kind):
+    """What the host rule turns away, the entry refuses too, and these layouts the other way round."""
+    codes = {torch.float16: _lib.RK_F16, torch.bfloat16: _lib.RK_BF16, torch.float32: _lib.RK_F32}
+    for dtype, code in codes.items():
+        for D in (1, 50, 64, 96, 100, 128):
+            for Dk in [k for k in (0, 1, 8, 13, 32, 64, 72, 128) if k <= D]:
+                q, mask, kp = _layout(method, D, Dk, dtype, kind)
+                taken = _check(method, D, Dk, code, mask=_lib.desc(mask)) == 0
+                assert _launch.recovered_decode_takes(q, mask, kp) == taken, (dtype, D, Dk)
+
+
+@pytest.mark.parametrize("method,D,Dk,kind", [("spark", 128, 96, "rows"), ("spark", 128, 13, "rows"), ("spark", 64, 32, "rows"),
+                                              ("spark", 128, 32, "offset"), ("think", 128, 13, "rows")])
+def test_refused_before_anything_is_packed(monkeypatch, method, D, Dk, kind):
+    q, mask, kp = _layout(method, D, Dk, torch.float16, kind)
+    B, H, S_v, _ = kp.shape
+    c = DynamicCache(reserve_tokens=4)
+    c.store_pruned(kp, torch.zeros(B, H, 2, D).half(), torch.zeros(B, H, 3, D).half(), None,
+                   torch.zeros(B, H, S_v + 5, D).half(), 0)
+    c.think_mask.append(torch.zeros(B, H, D, dtype=torch.bool) if method == "think" else None)
+    c.spark_mask.append(mask)
+    c.spark_pruned_mean.append(torch.zeros(B, H, S_v, 1).half())
+
+    def never(*a):
+        raise AssertionError("reached the launcher")
+
+    monkeypatch.setattr(_launch, "recovered_decode", never)
+    assert c._decode_pruned(q, 0, 2) is None
