@@ -68,7 +68,10 @@ struct DecodeArgs {
   // others chunk_vis; see rk_plan_decode)
   int32_t cmajor, nfast;
   int64_t chunk_fast;
-  int32_t units;
+  // not 0: dense, one unit per query head, several of them per KV head.  Then
+  // 1, or their number G: the units of a KV head that read the same chunk run
+  // in consecutive slots of one XCD (see decode_kernel)
+  int32_t xgroup, units;
   int32_t r_dtype, dm_dtype, has_bias, has_mask;
   // prologue layouts: q rows contiguous and 16-byte aligned (one 16-byte load
   // per thread); R a contiguous, 16-byte aligned [128][Dk] 16-bit block

@@ -564,6 +564,9 @@ __device__ __forceinline__ void merge_fused(const DecodeArgs& a, int u, int b, i
 // (a.fused set).  A separate instantiation: inlined into every
 // kernel, the merge's code raised the split pass's register pressure
 // enough to spill scalar registers in its loops.
+// SHARE (dense, one-head units with 16-byte loads): G units read each K/V row,
+// so their V loads are ordinary ones, which the caches keep (B=2, 4 KV heads
+// of 7, 600 tokens, K/V from memory: 12.4 -> 11.4 us).
 // SPK: the visual Keys are SparK's (kept channels per token, mask, mean of
 // the others): the workgroup puts each block's rows back together in
 // registers as score operands instead of reading recovered Keys.
@@ -571,7 +574,7 @@ __device__ __forceinline__ void merge_fused(const DecodeArgs& a, int u, int b, i
 // kernels its few lines moved the register allocator to other scalar spills
 // (B=1, 32 heads, 16k: 31.0 -> 31.4 us).
 template <class TT, int DKB, bool VEC, int HMAX, bool HAS_VIS, bool APPEND, bool DPART = false, bool FUSED = false,
-          bool SPK = false, bool SEL = false>
+          bool SPK = false, bool SEL = false, bool SHARE = false>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 decode_kernel(const DecodeArgs a) {
   static_assert(!DPART || VEC, "the element-wise kernels mask head_dim at run time");
@@ -616,6 +619,20 @@ decode_kernel(const DecodeArgs a) {
   int u = a.cmajor ? (int)blockIdx.x : (int)blockIdx.y;
   int x = a.cmajor ? (int)blockIdx.y : (int)blockIdx.x + (a.rot_x ? u % a.np : 0);
   x = x >= a.np ? x - a.np : x;
+  if (SHARE && a.xgroup > 1) {
+    // Workgroup id i = y * np + x runs on XCD i mod 8 as the (i / 8)-th of
+    // that XCD.  Each XCD takes a contiguous range of the work items
+    // ((b, kv) major, then chunk, then the query head j of the group), so
+    // the G units that read one K/V chunk are neighbours on one XCD and
+    // share its L2 instead of each fetching the chunk from memory.
+    const int64_t N = (int64_t)a.units * a.np, bid = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    const int64_t c = bid & 7, q8 = N >> 3, r8 = N & 7;
+    const int64_t item = c * q8 + min(c, r8) + (bid >> 3);
+    const int64_t grp = item / a.xgroup;  // (b, kv, chunk)
+    const int64_t ukv = grp / a.np;
+    x = (int)(grp - ukv * a.np);
+    u = (int)(ukv * a.xgroup + (item - grp * a.xgroup));
+  }
   const int b = u / a.units_per_b;
   const int r_in_b = u - b * a.units_per_b;
   const int kv = r_in_b / a.spk;
@@ -663,7 +680,9 @@ decode_kernel(const DecodeArgs a) {
   for (int j = 0; j < 8; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // A-operand token row of this lane inside a block, per score sub-block
   const uint32_t krow0 = 8 * (n >> 2) + (n & 3), krow1 = krow0 + 4;
-  const uint32_t rot_seed = ((uint32_t)u * 0x9E3779B1u) ^ ((uint32_t)x * 0x85EBCA77u);
+  // the units of one KV head visit a chunk's blocks in the same order
+  const uint32_t useed = (uint32_t)(SHARE && a.xgroup > 1 ? u / a.xgroup : u);
+  const uint32_t rot_seed = (useed * 0x9E3779B1u) ^ ((uint32_t)x * 0x85EBCA77u);
 
   // Prologue order: the first NBUF K/V blocks are requested, then the
   // prologue's own loads (q rows; R / delta_mu or the mask bytes), and only
@@ -1129,7 +1148,7 @@ decode_kernel(const DecodeArgs a) {
       for (int r = 0; r < 8; ++r) {
         uint32_t row = min(t0 + 8u * g + r, t_last);
         row += row >= a.vf_gap_at ? a.vf_gap : 0u;
-        B.v[r] = load_row8<VEC, true>(vfb, row * a.vf_ss, vch, a.vf_sd, vnv);
+        B.v[r] = load_row8<VEC, !SHARE>(vfb, row * a.vf_ss, vch, a.vf_sd, vnv);
       }
     };
 
@@ -1789,6 +1808,17 @@ hipError_t launch_one(const DecodeArgs& a, dim3 grid, hipStream_t s) {
       launched = true;
     }
   }
+  if constexpr (VEC && HMAX == 1 && !HAS_VIS) {
+    if (a.xgroup) {
+      if (a.fused)
+        hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, 1, false, false, DPART, kCanFuse, false, false, true>), grid,
+                           dim3(kThreads), 0, s, a);
+      else
+        hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, 1, false, false, DPART, false, false, false, true>), grid,
+                           dim3(kThreads), 0, s, a);
+      launched = true;
+    }
+  }
   if (!launched) {
     if (a.fused)
       hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, HAS_VIS, false, DPART, kCanFuse>), grid,
@@ -1823,7 +1853,8 @@ hipError_t launch_sel(const DecodeArgs& a, dim3 grid, hipStream_t s) {
 template <class TT, int DKB>
 hipError_t launch_sel_any(bool vec, int hmax, const DecodeArgs& a, dim3 grid, hipStream_t s) {
   if (!vec)
-    return hmax > 1 ? launch_sel<TT, DKB, false, 16, false>(a, grid, s) : launch_sel<TT, DKB, false, 1, false>(a, grid, s);
+    return hmax > 1 ? launch_sel<TT, DKB, false, 16, false>(a, grid, s)
+                    : launch_sel<TT, DKB, false, 1, false>(a, grid, s);
   if (a.D < 128)
     return hmax > 1 ? launch_sel<TT, DKB, true, 16, true>(a, grid, s) : launch_sel<TT, DKB, true, 1, true>(a, grid, s);
   return hmax > 1 ? launch_sel<TT, DKB, true, 16, false>(a, grid, s) : launch_sel<TT, DKB, true, 1, false>(a, grid, s);

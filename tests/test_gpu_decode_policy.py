@@ -56,6 +56,22 @@ LINE = [
 ]
 
 
+# the same past one round of one workgroup per CU, and within it
+LINE += [
+    (16, 16, 2, 300, None, _lib.RK_BF16, True), (4, 8, 2, 2400, None, _lib.RK_F16, True),
+    (1, 16, 2, 4800, None, _lib.RK_BF16, True), (4, 8, 2, 4800, None, _lib.RK_BF16, False),
+    (1, 8, 2, 9600, None, _lib.RK_BF16, False), (1, 8, 2, 4800, None, _lib.RK_BF16, False),
+    (16, 4, 3, 600, None, _lib.RK_BF16, False),
+    (1, 8, 7, 1200, None, _lib.RK_F32, True), (1, 8, 7, 2400, None, _lib.RK_F32, False),
+    (1, 16, 4, 600, None, _lib.RK_F32, True), (1, 16, 4, 1200, None, _lib.RK_F32, False),
+    (1, 1, 64, 1200, None, _lib.RK_F32, True), (1, 1, 64, 2400, None, _lib.RK_F32, False),
+    (16, 1, 20, 64, None, _lib.RK_F32, True), (32, 4, 7, 64, None, _lib.RK_F32, False),
+    (16, 2, 2, 600, None, _lib.RK_F32, False),
+    (1, 4, 2, 100, (9600, 32), _lib.RK_F32, False), (4, 4, 2, 100, (2400, 32), _lib.RK_F32, True),
+    (1, 2, 2, 100, (4800, 32), _lib.RK_F32, True), (1, 8, 2, 100, (8061, 32), _lib.RK_F32, True),
+]
+
+
 @pytest.mark.parametrize("case", LINE, ids=lambda c: "-".join(str(v) for v in c))
 def test_paper_family_decomposition(case):
     B, H, G, S, vis, dtype, per_head = case
@@ -103,3 +119,22 @@ def test_paper_family_matches_oracle(B, H, G, S, S_v, dtype):
     err = np.abs(_np(got) - want)
     ulp = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -8, torch.float32: 0.0}[dtype]
     assert got.shape == want.shape and (err <= np.maximum(tol, np.abs(want) * ulp)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 128), (torch.float16, 96)])
+@pytest.mark.parametrize("B,H,S,per_head", [(7, 11, 900, True), (3, 7, 3999, True), (32, 8, 300, True), (1, 16, 4800, True), (3, 1, 1, True),
+                                            (1, 16, 1199, True), (4, 8, 4800, False)])
+def test_two_heads_per_kv_head_match_oracle(B, H, S, per_head, dtype, D):
+    """Dense units that share K/V rows, in the launch order and in XCD order
+    (a number of workgroups that 8 does and does not divide)."""
+    from rotatek_amd.kernels.full_channel_flash_decoding import full_channel_decode
+    print(f"[case] two heads per KV head B={B} H={H} S={S} D={D} {dtype}", flush=True)
+    plan = _lib.plan_decode(B, 2 * H, H, 0, 0, S, 2, _lib.RK_POLICY_PAPER if per_head else _lib.RK_POLICY_GQA, CUS)
+    assert _ws(_lib.RK_POLICY_PAPER, B, H, 2, S, DTYPES[dtype]) == plan["workspace_bytes"]
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((B, 2 * H, D), (B, H, S, D), (B, H, S, D)))
+    got, want = full_channel_decode(q, k, v, 2), od.full_channel_decode(_np(q), _np(k), _np(v), 2)
+    # the decode bars of test_gpu_decode.py, or the output's own rounding
+    tol, ulp = {torch.float16: (2e-3, 2.0 ** -10), torch.bfloat16: (1e-2, 2.0 ** -8)}[dtype]
+    assert (np.abs(_np(got) - want) <= np.maximum(tol, np.abs(want) * ulp)).all()
