@@ -130,10 +130,10 @@ struct QNormArgs {
   float* qn;
 };
 
-template <class TT, bool QV>
+template <class TT, bool QV, bool COL>
 __device__ void window_group_sums(const uint16_t* q, int64_t q_b, int64_t q_h, int64_t q_s, int64_t q_d,
                                   int64_t S, int W, int G, int D, int b, int kv, int tid, float (&acc)[2][8]);
-template <class TT>
+template <class TT, bool COL>
 __device__ void floored_query_norms(const float (&acc)[2][8], int W, int D, float inv_g, int tid,
                                     float (*s_part)[128], float* s_qn, float* s_floor);
 
@@ -146,8 +146,8 @@ __device__ __forceinline__ void head_query_norms(const KeyView& k, const QNormAr
   __shared__ float s_floor;
   const int b = bh / k.H, kv = bh - b * k.H;
   float acc[2][8];
-  window_group_sums<TT, QV>(qa.q, qa.q_b, qa.q_h, qa.q_s, qa.q_d, qa.S, qa.W, qa.G, qa.D, b, kv, tid, acc);
-  floored_query_norms<TT>(acc, qa.W, qa.D, qa.inv_g, tid, s_part, s_qn, &s_floor);
+  window_group_sums<TT, QV, true>(qa.q, qa.q_b, qa.q_h, qa.q_s, qa.q_d, qa.S, qa.W, qa.G, qa.D, b, kv, tid, acc);
+  floored_query_norms<TT, true>(acc, qa.W, qa.D, qa.inv_g, tid, s_part, s_qn, &s_floor);
   if (tid < 128) qa.qn[(int64_t)bh * 128 + tid] = s_qn[tid];
 }
 
@@ -979,27 +979,17 @@ __global__ void __launch_bounds__(kThreads) gather_kernel(const void* R, int r_d
     ((uint16_t*)dm)[b * d_b + (int64_t)h * d_h + tid * d_c] = o;
 }
 
-// grid (B*H_kv), 256 threads: query-aware weighting of one covariance
-// (kv_pruning_utils.py:116-140).  q_norm[d] = || mean_g q[g, S-W+w, d] ||_2
-// over the last W queries, the group mean (over the G query heads of the KV
-// head) rounded to the query dtype as torch's bf16/fp16 mean is; floored at
-// 1e-3 x the lower median of the 128 norms; then
-//   out = 0.5 (C o (qn qn^T) + (C o (qn qn^T))^T) + 1e-4 max(mean|diag|, 1e-6) I
-// (the clamp binds to the mean).  Every global load (the covariance and the
-// G x W query rows) is issued before the first is used, so the kernel costs
-// one memory latency plus its LDS work.  Thread (slot rs = t/16, chunk
-// c8 = t%16) owns window rows rs and rs + 16 of channels 8 c8..8 c8+7 for all
-// G heads.  The covariance goes through LDS (rows padded to 129), so the
-// transposed read is conflict-free; out may alias cov.  CV / QV: 16-byte
-// row loads of the covariance / the queries (unit inner stride, aligned).
-constexpr int kQHeads = 4;  // query heads whose window rows are loaded together (eight at a time took 134
-                            // registers and left the mean launch, which carries this code, at three waves per SIMD)
-
+// The window's query norms are formed by the mean launch's extra column
+// (COL) and by qweight_kernel.  The column loads the window rows of four query
+// heads together and ranks eight norms at a time: with eight heads and the
+// whole rank loop unrolled, as qweight_kernel has them, it took 134 registers
+// and left the summing loop beside it at three waves per SIMD.  qweight_kernel
+// has no such neighbour (64 heads of 16 query heads 19.3 us, 20.0 in fours).
 // Thread (rs = t/16, c8 = t%16) of 256: the fp32 sums over the G query
 // heads of window rows rs and rs + 16 (of the last W rows), channels
-// 8 c8..8 c8+7, G in order, the loads of kQHeads heads (16-byte rows) or
-// two heads (element-wise) issued at a time.
-template <class TT, bool QV>
+// 8 c8..8 c8+7, G in order, the loads of four or eight heads (16-byte rows)
+// or two heads (element-wise) issued at a time.
+template <class TT, bool QV, bool COL>
 __device__ void window_group_sums(const uint16_t* q, int64_t q_b, int64_t q_h, int64_t q_s, int64_t q_d,
                                   int64_t S, int W, int G, int D, int b, int kv, int tid, float (&acc)[2][8]) {
   const int rs = tid >> 4, c8 = tid & 15;
@@ -1014,7 +1004,7 @@ __device__ void window_group_sums(const uint16_t* q, int64_t q_b, int64_t q_h, i
     for (int e = 0; e < 8; ++e) acc[j][e] = 0.f;
   // element-wise loads take 64-bit addresses each: two heads at a time
   // keep them in registers (the sums run in the same head order)
-  constexpr int kQH = QV ? kQHeads : 2;
+  constexpr int kQH = !QV ? 2 : COL ? 4 : 8;
   for (int g0 = 0; g0 < G; g0 += kQH) {
     float f[kQH][2][8];
     if constexpr (TT::kBytes == 2) {
@@ -1084,7 +1074,7 @@ __device__ void window_group_sums(const uint16_t* q, int64_t q_b, int64_t q_h, i
 // L2 norms over the window, and the floor at 1e-3 x the lower median of the
 // D norms (the norm of rank (D - 1) / 2, ties by index).  Leaves s_qn[c] =
 // the floored norms (0 past D).
-template <class TT>
+template <class TT, bool COL>
 __device__ void floored_query_norms(const float (&acc)[2][8], int W, int D, float inv_g, int tid,
                                     float (*s_part)[128], float* s_qn, float* s_floor) {
   const int rs = tid >> 4, c8 = tid & 15;
@@ -1118,7 +1108,7 @@ __device__ void floored_query_norms(const float (&acc)[2][8], int W, int D, floa
   if (tid < D) {
     v = s_qn[tid];
     int rank = 0;
-#pragma unroll 8
+#pragma unroll(COL ? 8 : 32)
     for (int j4 = 0; j4 < 32; ++j4) {
       const float4 u = *(const float4*)&s_qn[4 * j4];
       const float uu[4] = {u.x, u.y, u.z, u.w};
@@ -1189,7 +1179,7 @@ __global__ void __launch_bounds__(256) qweight_kernel(const float* cov, int64_t 
     }
   }
   float acc[2][8];
-  window_group_sums<TT, QV>(q, q_b, q_h, q_s, q_d, S, W, G, D, b, kv, tid, acc);
+  window_group_sums<TT, QV, false>(q, q_b, q_h, q_s, q_d, S, W, G, D, b, kv, tid, acc);
 
   // ---- the covariance into LDS
   if constexpr (CV) {
@@ -1206,7 +1196,7 @@ __global__ void __launch_bounds__(256) qweight_kernel(const float* cov, int64_t 
       s_C[(e >> 7) * CP + (e & 127)] = cv[i];
     }
   }
-  floored_query_norms<TT>(acc, W, D, inv_g, tid, s_part, s_qn, &s_floor);
+  floored_query_norms<TT, false>(acc, W, D, inv_g, tid, s_part, s_qn, &s_floor);
   const float ridge = weighted_ridge(tid < 128 ? s_C[tid * CP + tid] : 0.f, s_qn, tid, D, rfac, s_wsum);
   // ---- out[r][c] = 0.5 (C[r][c] w + C[c][r] w) + ridge [r == c], w = qn[r] qn[c]
   float* O = out + b * o_b + (int64_t)kv * o_h;
