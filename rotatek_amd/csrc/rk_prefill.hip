@@ -984,7 +984,7 @@ __global__ void __launch_bounds__(kThreads) gather_kernel(const void* R, int r_d
 // heads together and ranks eight norms at a time: with eight heads and the
 // whole rank loop unrolled, as qweight_kernel has them, it took 134 registers
 // and left the summing loop beside it at three waves per SIMD.  qweight_kernel
-// has no such neighbour (64 heads of 16 query heads 19.3 us, 20.0 in fours).
+// has no such neighbour (128 heads of 16 query heads 19.3 us, 20.0 in fours).
 // Thread (rs = t/16, c8 = t%16) of 256: the fp32 sums over the G query
 // heads of window rows rs and rs + 16 (of the last W rows), channels
 // 8 c8..8 c8+7, G in order, the loads of four or eight heads (16-byte rows)
@@ -1334,17 +1334,18 @@ struct CovPlan {
 // at least 512 tokens of 16-bit Keys (32 heads, 4097 tokens, 256 allowed: 33.3
 // us for the whole covariance, 32.2 so), 256 of fp32, whose products take
 // eight times as long (2304 tokens: 50.6 -> 45.7 us).  At most 64 per head
-// (fp32: one per 384 tokens up to 128), past which the estimate misses what
-// the finalisation pays for each partial of a head, about 0.06 us; where heads
-// are too few to fill the CUs so, one per CU, of 16-bit Keys no more than
-// sqrt(S / 16), where that and the tokens' 0.006 us balance.  Graph-replayed
-// whole covariance, 64 / now: one head of 131072 tokens 68.3 / 66.2 us, of
-// 1000000 285 / 131; fp32, one head of 65536 87.4 / 58.4, two 92.8 / 71.2,
-// three of 50000 82.9 / 76.5 (four of 20000, weighted, 52.3 at 64, 53.4 at 79).
+// (fp32 from 32768 tokens on 128; from 40960 where 64 fill the CUs evenly), past
+// which the estimate misses what the finalisation pays for each partial of a
+// head, about 0.06 us; where heads are too few to fill the CUs so, one per
+// CU, of 16-bit Keys no more than sqrt(S / 16), where that and the tokens'
+// 0.006 us balance.  Graph-replayed whole covariance, 64 / now: one head of
+// 131072 tokens 68.3 / 66.2 us, of 1000000 285 / 131; fp32, one head of 65536
+// 87.0 / 58.4, two 92.8 / 71.2, three of 50000 82.9 / 76.1, four of 65536 94.9
+// / 84.1 (of 32768, 128 against 64: 65.6 / 60.4).
 int cov_splits_for(int64_t bh, int64_t S, int cus, bool f32) {
   if (S <= 0 || bh <= 0) return 1;
   const int64_t one = cdiv(cus, bh), few = f32 ? one : std::min(one, (int64_t)sqrt((double)S / 16));
-  const int64_t many = f32 ? std::min<int64_t>(std::max<int64_t>(64, S / 384), 128) : 64;
+  const int64_t many = f32 && S >= (64 * bh % cus ? 32768 : 40960) ? 128 : 64;
   const int64_t cap = std::min(cdiv(S, f32 ? 256 : 512), std::max(many, few));
   double best = 0;
   int splits = 1;

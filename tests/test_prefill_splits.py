@@ -41,7 +41,8 @@ def test_mean_splits(B, H, S, mean):
 @pytest.mark.parametrize("B,H,S,dtype,splits", [
     (1, 1, 131072, _lib.RK_BF16, 90), (1, 1, 1000000, _lib.RK_F16, 250), (1, 2, 1000000, _lib.RK_BF16, 128),
     (1, 4, 131072, _lib.RK_BF16, 64), (1, 1, 65536, _lib.RK_F32, 256), (1, 2, 65536, _lib.RK_F32, 128),
-    (1, 4, 65536, _lib.RK_F32, 128), (1, 4, 20000, _lib.RK_F32, 64), (1, 8, 65536, _lib.RK_F32, 64), (8, 4, 12001, _lib.RK_BF16, 16),
+    (1, 4, 65536, _lib.RK_F32, 128), (1, 4, 32768, _lib.RK_F32, 64), (1, 3, 32768, _lib.RK_F32, 128),
+    (1, 4, 20000, _lib.RK_F32, 64), (1, 8, 65536, _lib.RK_F32, 64), (8, 4, 12001, _lib.RK_BF16, 16),
     (10, 32, 4000, _lib.RK_F16, 3), (32, 32, 14000, _lib.RK_F16, 1), (1, 8, 500, _lib.RK_BF16, 1)])
 def test_covariance_splits(B, H, S, dtype, splits):
     """Few heads with long spans fill the CUs; the others keep the split of least estimated cost."""
