@@ -4,10 +4,12 @@ than the memory-side cache (streamed loads and stores), and the 16-byte
 output path of the rotation.  Inputs are small integers with a mean of zero,
 so every sum is exact and the results are compared bit for bit.
 """
+import ctypes
+
 import pytest
 import torch
 
-from rotatek_amd import prefill
+from rotatek_amd import _lib, prefill
 
 pytestmark = pytest.mark.gpu
 
@@ -25,6 +27,16 @@ def _cov_ref(K):
     """Kc^T Kc rounded to the key dtype; exact below 2^24."""
     k = K.float()
     return torch.matmul(k.transpose(-1, -2).contiguous(), k).to(K.dtype).float()
+
+
+def _cov_splits(K):
+    """Workgroups per head of the covariance pass, from the workspace it asks for
+    (per head, in rows of 128 floats: the mean's partials, at most 72 of them
+    here, 73 for each split, one)."""
+    need = ctypes.c_size_t(0)
+    d = [_lib.desc(t) for t in (K, torch.empty(*K.shape[:2], K.shape[3], K.shape[3], device="cuda"))]
+    assert _lib.load().rk_key_covariance_check(ctypes.byref(d[0]), None, ctypes.byref(d[1]), 0, ctypes.byref(need)) == 0
+    return (need.value // (K.shape[0] * K.shape[1] * 512) - 1) // 73
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -78,6 +90,27 @@ def test_streamed_keys(S, dtype):
     assert out.numel() * 2 > 256 << 20
     want = torch.matmul(one.float(), R.float()).to(dtype)
     assert torch.equal(out, want.expand(B, -1, -1, -1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,S,splits", [(16, 4, 30722, 8), (9, 32, 4098, 3), (40, 32, 1030, 1)])
+def test_streamed_keys_weighted_and_split(B, H, S, splits, dtype):
+    """Streamed Keys of mean one, in one and in several workgroups per head,
+    plain and query-weighted (batch rows share one row's memory)."""
+    print(f"[case] streamed and split B={B} H={H} S={S} {dtype}", flush=True)
+    one = _int_keys(1, H, S, 128, dtype, S)
+    cov_one = _cov_ref(one)
+    K = (one + 1).expand(B, H, S, 128)
+    assert K.numel() * 2 > 256 << 20
+    Q = torch.randn(1, 2 * H, 40, 128, generator=torch.Generator(device="cuda").manual_seed(S), device="cuda").to(dtype)
+    Q = Q.expand(B, 2 * H, 40, 128)
+    mean, cov = prefill.key_covariance(K)
+    assert _cov_splits(K) == splits
+    # the centre is the mean in the key dtype, exactly one
+    assert float((mean - 1).abs().max()) < 1e-6
+    assert torch.equal(cov, cov_one.expand(B, -1, -1, -1))
+    mean_w, cov_w = prefill.key_covariance(K, Q, 2)
+    assert torch.equal(mean_w, mean) and torch.equal(cov_w, prefill.query_weight(cov, Q, 2))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
