@@ -510,15 +510,17 @@ def run_baselines(args):
     at a decode configuration (default config 2) on one GPU: the prefill
     selection of each over the visual Keys, the decode-time recovery (the
     recovered visual rows and the full-width span written by one launch) and
-    the decode step (recovery + dense decode), next to ThinK's attention on
-    the RotateK kernel (one-hot R, no recovery) and the RotateK step on the
-    same data.  Every stage is >= 100 us at config 2, so it is timed eagerly
+    the decode step (recovery + dense decode), next to the span cache's step
+    without recovered Keys (``DynamicCache.decode_recovered``), ThinK's
+    attention on the RotateK kernel (one-hot R, no recovery) and the RotateK
+    step on the same data.  Every stage is >= 100 us at config 2, so it is timed eagerly
     with HIP events over ``--steps`` calls; bytes are algorithmic."""
     import torch
 
     from rotatek_amd import synth
     from rotatek_amd.baselines import (recover_spark, recover_think, selection_rotation, spark_prune,
                                        think_score_and_compact)
+    from rotatek_amd.cache import DynamicCache
     from rotatek_amd.kernels.full_channel_flash_decoding import full_channel_decode
     from rotatek_amd.kernels.fused_decode import rotatek_decode_fused
     from rotatek_amd.kernels.gqa_decode import full_channel_decode_gqa, rotatek_decode_gqa
@@ -566,10 +568,21 @@ def run_baselines(args):
         recover_spark(Kc_s, sm, pm, out=stage, k_text=kf)
         return dense(q, stage, V, G)
 
+    def span_cache(Kc, think_mask, spark_mask, mean):
+        c = DynamicCache(reserve_tokens=16)
+        c.store_pruned(Kc, kf[:, :, :0], kf, None, V, 0)    # V rows: visual, then text
+        c.think_mask.append(think_mask)
+        c.spark_mask.append(spark_mask)
+        c.spark_pruned_mean.append(mean)
+        return c
+
+    think_cache, spark_cache = span_cache(Kc_t, tm, None, None), span_cache(Kc_s, None, sm, pm)
     da = synth.decode_args(inp)
     R_sel = selection_rotation(tm, keep, cfg.dtype)
     think_fused_args = dict(da, R_partial=R_sel, delta_mu=None, k_sparse=Kc_t)
     for name, fn in (("think_decode_step", think_step), ("spark_decode_step", spark_step),
+                     ("think_decode_recovered", lambda: think_cache.decode_recovered(q, 0, G)),
+                     ("spark_decode_recovered", lambda: spark_cache.decode_recovered(q, 0, G)),
                      ("think_fused_decode", lambda: rot(**think_fused_args)),
                      ("rotatek_decode", lambda: rot(**da))):
         _, t, _ = timed(fn)

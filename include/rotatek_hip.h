@@ -261,7 +261,8 @@ int rk_recovered_decode(const rk_tensor* q, const rk_tensor* think_mask, const r
  * against (full_channel_flash_decoding.py:162-229, gqa_decode.py:254-277):
  * q [B,H_q,D], k/v [B,H_kv,S,D], out [B,H_q,D].  policy as above; with
  * num_kv_groups > 1 RK_POLICY_PAPER keeps one unit per query head for calls
- * short enough for one workgroup per CU, in every dtype. */
+ * short enough for one workgroup per CU, in every dtype, and for somewhat
+ * longer ones in F32 and with num_kv_groups == 2. */
 int rk_full_channel_decode_check(const rk_tensor* q, const rk_tensor* k,
                                  const rk_tensor* v, int64_t num_kv_groups,
                                  const rk_tensor* out, int32_t policy,
@@ -295,8 +296,12 @@ void rk_decode_workspace_release(void* workspace);
  * any other device or layout every mode runs two launches. */
 void rk_set_decode_merge(int32_t mode);
 
-/* Split plan the decode entry points use for a shape (host only), exposed
- * for tests and benchmarks.  Fields are filled on RK_OK. */
+/* Split plan of a shape under exactly the policy passed (host only), exposed
+ * for tests and benchmarks.  The entry points run it, with RK_POLICY_PAPER
+ * replaced by RK_POLICY_GQA as described at rk_rotatek_decode and
+ * rk_full_channel_decode, and over SparK masks (rk_recovered_decode) with Dk +
+ * 64 for Dk: workspace sizes come from their _check functions.  Fields are
+ * filled on RK_OK. */
 typedef struct rk_decode_plan {
   int64_t units;          /* work units (B*H_kv for GQA, B*H_q for paper)    */
   int32_t heads_per_unit; /* query heads handled per unit (<= 16)            */

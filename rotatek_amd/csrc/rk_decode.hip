@@ -658,24 +658,24 @@ int run_decode(const Checked& c, const rk_tensor* q, const rk_tensor* R, const r
   }
   if (has_vis) {
     if (!sm) {
-    a.R = R->data;
-    a.r_dtype = R->dtype;
-    set4(R, a.R_sb, a.R_sh, a.R_sd, a.R_sk);
-    if (dm && dm->data) {
-      a.dm = dm->data;
-      a.dm_dtype = dm->dtype;
-      a.dm_sb = dm->stride[0];
-      a.dm_sh = dm->stride[1];
-      a.dm_sd = dm->stride[2];
-      a.has_bias = 1;
-    }
-    // R staged into LDS (16-byte DMA): up to 64 channels in either 16-bit
-    // type; 65-128 only in the compute type (their q R is an MFMA product
-    // read straight from the staged rows, and R fills the kernel's s_acc)
-    // (a head's [D][Dk] block is copied as whole 16-byte chunks)
-    a.r_vec = rk::is_half(R->dtype) && (c.Dk <= 64 || (c.Dk <= 128 && R->dtype == c.dtype)) &&
-              R->stride[3] == 1 && R->stride[2] == c.Dk && (c.D * c.Dk) % 8 == 0 &&
-              R->stride[1] % 8 == 0 && R->stride[0] % 8 == 0 && (((uintptr_t)R->data) & 15) == 0;
+      a.R = R->data;
+      a.r_dtype = R->dtype;
+      set4(R, a.R_sb, a.R_sh, a.R_sd, a.R_sk);
+      if (dm && dm->data) {
+        a.dm = dm->data;
+        a.dm_dtype = dm->dtype;
+        a.dm_sb = dm->stride[0];
+        a.dm_sh = dm->stride[1];
+        a.dm_sd = dm->stride[2];
+        a.has_bias = 1;
+      }
+      // R staged into LDS (16-byte DMA): up to 64 channels in either 16-bit
+      // type; 65-128 only in the compute type (their q R is an MFMA product
+      // read straight from the staged rows, and R fills the kernel's s_acc)
+      // (a head's [D][Dk] block is copied as whole 16-byte chunks)
+      a.r_vec = rk::is_half(R->dtype) && (c.Dk <= 64 || (c.Dk <= 128 && R->dtype == c.dtype)) &&
+                R->stride[3] == 1 && R->stride[2] == c.Dk && (c.D * c.Dk) % 8 == 0 &&
+                R->stride[1] % 8 == 0 && R->stride[0] % 8 == 0 && (((uintptr_t)R->data) & 15) == 0;
     }
     a.ks = (const uint16_t*)ks->data;
     a.vs = (const uint16_t*)vs->data;

@@ -1798,7 +1798,7 @@ hipError_t launch_one(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   if (a.fused && !kCanFuse) return hipErrorInvalidValue;
   bool launched = false;
   if constexpr (HAS_VIS) {  // the span cache's step always carries the visual span
-    if (!launched && a.k_new) {
+    if (a.k_new) {
       if (a.fused)
         hipLaunchKernelGGL((decode_kernel<TT, DKB, VEC, HMAX, true, true, DPART, kCanFuse>), grid,
                            dim3(kThreads), 0, s, a);

@@ -1136,10 +1136,10 @@ __device__ void floored_query_norms(const float (&acc)[2][8], int W, int D, floa
 // head) rounded to the query dtype as torch's bf16/fp16 mean is; floored at
 // 1e-3 x the lower median of the 128 norms; then
 //   out = 0.5 (C o (qn qn^T) + (C o (qn qn^T))^T) + 1e-4 max(mean|diag|, 1e-6) I
-// (the clamp binds to the mean).  Every global load (the covariance and the
-// G x W query rows) is issued before the first is used, so the kernel costs
-// one memory latency plus its LDS work.  The covariance goes through LDS
-// (rows padded to 129), so the transposed read is conflict-free; out may
+// (the clamp binds to the mean).  Up to eight query heads, every global load
+// (the covariance and the G x W query rows) is issued before the first is
+// used, so the kernel costs one memory latency plus its LDS work.  The
+// covariance goes through LDS (rows padded to 129), so the transposed read is conflict-free; out may
 // alias cov.  CV / QV: 16-byte row loads of the covariance / the queries
 // (unit inner stride, aligned).
 template <class TT, bool CV, bool QV>
