@@ -746,7 +746,7 @@ decode_kernel(const DecodeArgs a) {
     // Bound by memory like the other paths: about 380 vector and 70 LDS
     // instructions per 32 tokens and wave, under its 15 KB of loads.  B=8, 32
     // heads, 14000 tokens, keep 32 (fp16), with 2000 prompt/text tokens:
-    // 746 us recovering the Keys and attending them, 333 here (5.7 TB/s).
+    // 745 us recovering the Keys and attending them, 333 here (5.7 TB/s).
     const int64_t t_begin = x < a.nfast ? (int64_t)x * a.chunk_fast
                                         : (int64_t)a.nfast * a.chunk_fast + (int64_t)(x - a.nfast) * a.chunk_vis;
     const int64_t t_end = min(a.S_v, t_begin + (x < a.nfast ? a.chunk_fast : a.chunk_vis));
