@@ -512,9 +512,11 @@ int plan_for(const Checked& c, bool has_vis, int32_t policy, int cus, rk_decode_
 // prologue, softmax and merge.  Graph-replayed us per step, per head /
 // grouped.  Dense, 8 KV heads of 4, B=1: bf16 300 tokens 10.6 / 12.2, 1200
 // 11.2 / 12.7, and past the round 4800 16.5 / 13.2; fp32 2000 tokens 12.3 /
-// 19.7, 8000 (1 MB workgroups) 37.6 / 25.4.  RotateK in 16 bits stays grouped:
-// its lines cross inside the round (keep 32, 4 KV heads of 7, 1000 + 100
-// tokens 10.1 / 10.8, 2304 + 128 12.7 / 11.2).  Three lines lie elsewhere:
+// 19.7, 8000 (1 MB workgroups) 37.6 / 25.4.  RotateK, keep 32, fp32, 4 KV heads
+// of 7: 1000 + 100 tokens 11.7 / 25.1, 4097 + 60 16.9 / 26.7 (two heads per KV
+// head and 384-token workgroups 18.2 / 17.3, but one launch: eager 19.1 / 21.9).
+// RotateK in 16 bits stays grouped: its lines cross inside the round (1000 +
+// 100 tokens 10.1 / 10.8, 2304 + 128 12.7 / 11.2).  Two lines lie elsewhere:
 //  - dense in 16 bits with two heads per KV head, one round of two workgroups
 //    per CU of 257-384 tokens, at most 16 per unit: with the XCD order 17.4 /
 //    18.4 (16 KV heads, 4800 tokens), 15.7 / 18.9 (256, 300), from memory
@@ -526,11 +528,6 @@ int plan_for(const Checked& c, bool has_vis, int32_t policy, int cus, rk_decode_
 //    16.1 / 24.9, 1200 20.9 / 25.0, 2400 30.9 / 27.1; 16 of 4, 600 tokens
 //    16.7 / 19.5, 1200 21.7 / 19.5; one of 64, 1200 tokens 19.2 / 26.9, 2400
 //    27.8 / 28.1.  A round is charged its tokens and 64 more.
-//  - RotateK in fp32 with two heads per KV head: 257-384 tokens give a
-//    workgroup's waves one or two blocks, where the grouped plan has one each;
-//    that pays only if the round is full (4 KV heads, 9600 tokens, 208
-//    workgroups 19.1 / 17.6; B=4, 2400 tokens, 256 workgroups 14.2 / 17.6; of
-//    640 tokens, 8 KV heads, 8061 tokens, 22.5 / 24.2).
 int32_t decode_policy(const Checked& c, bool has_vis, int32_t policy, int cus) {
   if (policy != RK_POLICY_PAPER || c.G == 1) return policy;
   const bool f32 = c.dtype == RK_F32;
@@ -538,12 +535,10 @@ int32_t decode_policy(const Checked& c, bool has_vis, int32_t policy, int cus) {
   if ((has_vis && !f32) || plan_for(c, has_vis, policy, cus, &p) != RK_OK) return RK_POLICY_GQA;
   const int64_t bytes = std::max(p.chunk_full * 256, p.chunk_vis * (c.Dk + 128)) * rk::dtype_size(c.dtype);
   bool per_head = p.grid <= cus && bytes <= knobs().max_wg;
-  if (has_vis)
-    per_head = per_head && (c.G > 2 || p.chunk_vis <= 256 || p.chunk_vis > 384 || p.grid * 16 >= (int64_t)cus * 15);
-  else if (f32 && c.G >= 4)
+  if (!has_vis && f32 && c.G >= 4)
     per_head = per_head || cdiv(p.grid, cus) * (64 + std::max<int64_t>(128, std::min(p.chunk_full, c.S_f))) <=
                                (c.G >= 8 ? 768 : c.G > 4 ? 640 : 448);
-  else if (!f32 && c.G == 2)
+  else if (!has_vis && !f32 && c.G == 2)
     per_head = per_head || (p.grid <= 2 * (int64_t)cus && p.chunk_full > 256 && p.chunk_full <= 384 && p.wg_full <= 16);
   return per_head ? policy : RK_POLICY_GQA;
 }

@@ -67,7 +67,7 @@ LINE += [
     (1, 1, 64, 1200, None, _lib.RK_F32, True), (1, 1, 64, 2400, None, _lib.RK_F32, False),
     (16, 1, 20, 64, None, _lib.RK_F32, True), (32, 4, 7, 64, None, _lib.RK_F32, False),
     (16, 2, 2, 600, None, _lib.RK_F32, False),
-    (1, 4, 2, 100, (9600, 32), _lib.RK_F32, False), (4, 4, 2, 100, (2400, 32), _lib.RK_F32, True),
+    (1, 4, 2, 100, (9600, 32), _lib.RK_F32, True), (4, 4, 2, 100, (2400, 32), _lib.RK_F32, True),
     (1, 2, 2, 100, (4800, 32), _lib.RK_F32, True), (1, 8, 2, 100, (8061, 32), _lib.RK_F32, True),
 ]
 
