@@ -130,13 +130,15 @@ def recovered_decode_takes(q, spark_mask, k_pruned) -> bool:
     SparK layer: what rk_recovered_decode refuses whatever the sizes, told
     before anything is packed or allocated (an eager step of a small refused
     layer spent a third of its time there: 34 us, 50 with it, 34 so)."""
-    D, keep = q.shape[-1], k_pruned.shape[-1]
-    if q.dtype not in (torch.float16, torch.bfloat16) or keep == 0:
+    keep = k_pruned.size(-1)
+    if q.dtype is not torch.float16 and q.dtype is not torch.bfloat16 or keep == 0:
         return False
     if spark_mask is None:
-        return keep % 8 == 0 or D % 8 != 0
-    if D != 128 or keep > 64 or keep % 8 != 0 or spark_mask.data_ptr() % 16 != 0:
+        return keep % 8 == 0 or q.size(-1) % 8 != 0
+    if keep > 64 or keep % 8 != 0 or q.size(-1) != 128 or spark_mask.data_ptr() % 16 != 0:
         return False
+    if spark_mask.is_contiguous():      # rows of 128 bytes
+        return True
     *rows, last = spark_mask.stride()
     return last == 1 and all(s % 16 == 0 or n == 1 for s, n in zip(rows, spark_mask.shape))
 
