@@ -123,7 +123,8 @@ def test_paper_family_matches_oracle(B, H, G, S, S_v, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 128), (torch.float16, 96)])
-@pytest.mark.parametrize("B,H,S,per_head", [(7, 11, 900, True), (3, 7, 3999, True), (32, 8, 300, True), (1, 16, 4800, True), (3, 1, 1, True),
+@pytest.mark.parametrize("B,H,S,per_head", [(7, 11, 900, True), (3, 7, 3999, True), (32, 8, 300, True),
+                                            (1, 16, 4800, True), (3, 1, 1, True),
                                             (1, 16, 1199, True), (4, 8, 4800, False)])
 def test_two_heads_per_kv_head_match_oracle(B, H, S, per_head, dtype, D):
     """Dense units that share K/V rows, in the launch order and in XCD order
@@ -133,7 +134,8 @@ def test_two_heads_per_kv_head_match_oracle(B, H, S, per_head, dtype, D):
     plan = _lib.plan_decode(B, 2 * H, H, 0, 0, S, 2, _lib.RK_POLICY_PAPER if per_head else _lib.RK_POLICY_GQA, CUS)
     assert _ws(_lib.RK_POLICY_PAPER, B, H, 2, S, DTYPES[dtype]) == plan["workspace_bytes"]
     g = torch.Generator(device="cuda").manual_seed(S)
-    q, k, v = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((B, 2 * H, D), (B, H, S, D), (B, H, S, D)))
+    shapes = ((B, 2 * H, D), (B, H, S, D), (B, H, S, D))
+    q, k, v = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in shapes)
     got, want = full_channel_decode(q, k, v, 2), od.full_channel_decode(_np(q), _np(k), _np(v), 2)
     # the decode bars of test_gpu_decode.py, or the output's own rounding
     tol, ulp = {torch.float16: (2e-3, 2.0 ** -10), torch.bfloat16: (1e-2, 2.0 ** -8)}[dtype]

@@ -31,7 +31,8 @@ def _rows(B, H, S, dtype):
 
 
 @pytest.mark.parametrize("B,H,S,mean", [(1, 8, 65536, 64), (1, 8, 131072, 64), (4, 4, 65536, 32), (1, 32, 30720, 32),
-                                        (16, 4, 30720, 60), (32, 32, 30720, 60), (32, 32, 14000, 28), (8, 4, 12001, 24), (1, 32, 2304, 9),
+                                        (16, 4, 30720, 60), (32, 32, 30720, 60), (32, 32, 14000, 28),
+                                        (8, 4, 12001, 24), (1, 32, 2304, 9),
                                         (1, 8, 500, 2), (1, 1, 1, 1)])
 def test_mean_splits(B, H, S, mean):
     """Two workgroups per CU, or 512 tokens each while that is at most 32 (with few heads) per head."""

@@ -58,8 +58,8 @@ def _layout(method, D, Dk, dtype, kind, B=2, H=3, S_v=70):
                "strided": wide[..., 16:16 + D], "split": wide[..., :2 * D:2]}[kind], kp
 
 
-@pytest.mark.parametrize("method,kind", [("think", "rows"), ("spark", "rows"), ("spark", "offset"), ("spark", "strided"),
-                                         ("spark", "split")])
+@pytest.mark.parametrize("method,kind", [("think", "rows"), ("spark", "rows"), ("spark", "offset"),
+                                         ("spark", "strided"), ("spark", "split")])
 def test_early_refusal_is_the_entry_refusal(method, kind):
     """What the host rule turns away, the entry refuses too, and these layouts the other way round."""
     codes = {torch.float16: _lib.RK_F16, torch.bfloat16: _lib.RK_BF16, torch.float32: _lib.RK_F32}
@@ -71,8 +71,8 @@ def test_early_refusal_is_the_entry_refusal(method, kind):
                 assert _launch.recovered_decode_takes(q, mask, kp) == taken, (dtype, D, Dk)
 
 
-@pytest.mark.parametrize("method,D,Dk,kind", [("spark", 128, 96, "rows"), ("spark", 128, 13, "rows"), ("spark", 64, 32, "rows"),
-                                              ("spark", 128, 32, "offset"), ("think", 128, 13, "rows")])
+@pytest.mark.parametrize("method,D,Dk,kind", [("spark", 128, 96, "rows"), ("spark", 128, 13, "rows"),
+                                              ("spark", 64, 32, "rows"), ("spark", 128, 32, "offset"), ("think", 128, 13, "rows")])
 def test_refused_before_anything_is_packed(monkeypatch, method, D, Dk, kind):
     q, mask, kp = _layout(method, D, Dk, torch.float16, kind)
     B, H, S_v, _ = kp.shape
